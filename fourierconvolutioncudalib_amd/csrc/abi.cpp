@@ -83,6 +83,13 @@ ConvShape shape_from_any(const int* imDim, const int* kernelDim) {
   return s;
 }
 
+// shape_from_any as the convolution entry points run it: extended to
+// compile-time transform lengths where that is faster
+ConvShape conv_shape(const int* imDim, const int* kernelDim) {
+  const ConvShape s = shape_from_any(imDim, kernelDim);
+  return needs_long_path(s) ? s : with_extension(s);
+}
+
 // device workspace of one device-resident convolution of `s`
 size_t conv_workspace_bytes(const ConvShape& s) {
   return needs_long_path(s) ? long_workspace_bytes(s) : workspace_layout(s).total();
@@ -149,12 +156,14 @@ size_t device_budget(const DevicePool& pool) {
 // How a host-pointer convolution of `s` runs within `budget`: a z-slab plan
 // (nslabs > 0) or the single shot.
 struct HostPlan {
+  ConvShape s{};  // the shape the single shot runs
   SlabPlan sp;
   size_t device_bytes = 0;  // everything it allocates on the device
 };
 
 HostPlan host_plan(const ConvShape& s, size_t budget) {
   HostPlan h;
+  h.s = s;
   if (needs_long_path(s)) {  // long axes: one shot, no slabs
     h.device_bytes = (sizeof(float) * (size_t)s.voxels() + 255) / 256 * 256 +
                      long_workspace_bytes(s) +
@@ -170,7 +179,10 @@ HostPlan host_plan(const ConvShape& s, size_t budget) {
       return h;
     }
   }
-  h.device_bytes = single;
+  // extended where the larger spectrum fits the budget too
+  h.s = with_extension(s);
+  if (single_shot_device_bytes(h.s) > budget) h.s = s;
+  h.device_bytes = single_shot_device_bytes(h.s);
   return h;
 }
 
@@ -204,13 +216,13 @@ void host_convolution(const ConvShape& s, const float* im, const float* kernel, 
              "the convolution needs " + std::to_string(hp.device_bytes >> 20) +
                  " MiB of device memory (device budget " + std::to_string(budget >> 20) +
                  " MiB) and no z-slab plan fits the budget");
-  const size_t nws = conv_workspace_bytes(s);
+  const size_t nws = conv_workspace_bytes(hp.s);
   void* dimg = pool_reserve(reinterpret_cast<void**>(&pool.img), &pool.img_bytes, nimg);
   void* dker = pool_reserve(reinterpret_cast<void**>(&pool.ker), &pool.ker_bytes, nker);
   void* ws = pool_reserve(&pool.ws, &pool.ws_bytes, nws);
   staged_upload(dev, dimg, im, nimg, pool.stream);
   staged_upload(dev, dker, kernel, nker, pool.stream);
-  enqueue_any(s, static_cast<float*>(dimg), static_cast<float*>(dimg), static_cast<float*>(dker),
+  enqueue_any(hp.s, static_cast<float*>(dimg), static_cast<float*>(dimg), static_cast<float*>(dker),
               op, ws, pool.stream);
   staged_download(dev, out, dimg, nimg, pool.stream);
 }
@@ -225,9 +237,31 @@ long long host_device_bytes(const ConvShape& s, int dev) {
   return (long long)host_plan(s, device_budget(pool)).device_bytes;
 }
 
+// device workspace of a boundary-mode convolution: the padded transform's
+// (an extended shape needs less); the periodic mode is the plain convolution
+size_t boundary_workspace(const ConvShape& s, const PaddedProblem& p, int boundary) {
+  return workspace_layout(boundary == kMapPeriodic ? with_extension(s) : p.padded).total();
+}
+
+// boundary-mode convolution of raw shape `s` in a workspace of ws_bytes,
+// which holds the padded transform
+void enqueue_boundary(const ConvShape& s, const PaddedProblem& p, int boundary, float* d_out,
+                      const float* d_image, const float* d_kernel, Op op, void* ws,
+                      size_t ws_bytes, hipStream_t st) {
+  ConvShape e;
+  if (boundary == kMapPeriodic) {
+    e = with_extension(s);
+    enqueue_convolution(ws_bytes < workspace_layout(e).total() ? s : e, d_out, d_image, d_kernel,
+                        op, ws, st);
+  } else if (boundary_extension(s, p, boundary, &e))
+    run_convolution(e, d_out, d_image, d_kernel, op, ws, st);
+  else
+    enqueue_convolution_padded(p, d_out, d_image, d_kernel, op, ws, st);
+}
+
 // host-pointer boundary-mode convolution through the device pool
-void host_convolution_padded(const PaddedProblem& p, const float* im, const float* kernel,
-                             float* out, Op op, int dev) {
+void host_convolution_padded(const ConvShape& raw, const PaddedProblem& p, int boundary,
+                             const float* im, const float* kernel, float* out, Op op, int dev) {
   FC_REQUIRE(im != nullptr && kernel != nullptr && out != nullptr, kInvalidArgument,
              "null data pointer");
   DeviceGuard guard(dev);
@@ -237,14 +271,14 @@ void host_convolution_padded(const PaddedProblem& p, const float* im, const floa
   const ConvShape& s = p.padded;
   const size_t nimg = sizeof(float) * (size_t)p.vp.n[0] * p.vp.n[1] * p.vp.n[2];
   const size_t nker = sizeof(float) * (size_t)s.kx * s.ky * s.kz;
-  const size_t nws = workspace_layout(s).total();
+  const size_t nws = boundary_workspace(raw, p, boundary);
   void* dimg = pool_reserve(reinterpret_cast<void**>(&pool.img), &pool.img_bytes, nimg);
   void* dker = pool_reserve(reinterpret_cast<void**>(&pool.ker), &pool.ker_bytes, nker);
   void* ws = pool_reserve(&pool.ws, &pool.ws_bytes, nws);
   staged_upload(dev, dimg, im, nimg, pool.stream);
   staged_upload(dev, dker, kernel, nker, pool.stream);
-  enqueue_convolution_padded(p, static_cast<float*>(dimg), static_cast<float*>(dimg),
-                             static_cast<float*>(dker), op, ws, pool.stream);
+  enqueue_boundary(raw, p, boundary, static_cast<float*>(dimg), static_cast<float*>(dimg),
+                   static_cast<float*>(dker), op, ws, nws, pool.stream);
   staged_download(dev, out, dimg, nimg, pool.stream);
 }
 
@@ -422,7 +456,7 @@ long long fcamd_host_device_bytes(const int* imDim, const int* kernelDim, int de
 
 long long fcamd_workspace_bytes(const int* imDim, const int* kernelDim) {
   long long r = -1;
-  (void)guarded([&] { r = (long long)conv_workspace_bytes(shape_from_any(imDim, kernelDim)); });
+  (void)guarded([&] { r = (long long)conv_workspace_bytes(conv_shape(imDim, kernelDim)); });
   return r;
 }
 
@@ -431,9 +465,12 @@ int fcamd_convolve3d_device(float* d_out, const float* d_image, const int* imDim
                             long long workspace_bytes, void* stream) {
   return guarded([&] {
     FC_REQUIRE(d_out && d_image && d_kernel, kInvalidArgument, "null device pointer");
-    ConvShape s = shape_from_any(imDim, kernelDim);
+    ConvShape s = conv_shape(imDim, kernelDim);
     const Op o = op_from(op);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    // a workspace that holds the unextended transform is enough for it
+    if (d_workspace && s.extended() && workspace_bytes < (long long)conv_workspace_bytes(s))
+      s = direct_shape(s);
     const size_t need = conv_workspace_bytes(s);
     if (d_workspace) {
       FC_REQUIRE(workspace_bytes >= (long long)need, kInvalidArgument, "workspace too small");
@@ -454,8 +491,8 @@ int fcamd_convolve3d_device(float* d_out, const float* d_image, const int* imDim
 long long fcamd_boundary_workspace_bytes(const int* imDim, const int* kernelDim, int boundary) {
   long long r = -1;
   (void)guarded([&] {
-    r = (long long)workspace_layout(padded_problem(raw_shape(imDim, kernelDim), boundary).padded)
-            .total();
+    const ConvShape raw = raw_shape(imDim, kernelDim);
+    r = (long long)boundary_workspace(raw, padded_problem(raw, boundary), boundary);
   });
   return r;
 }
@@ -476,20 +513,23 @@ int fcamd_convolve3d_boundary_device(float* d_out, const float* d_image, const i
                                      void* stream) {
   return guarded([&] {
     FC_REQUIRE(d_out && d_image && d_kernel, kInvalidArgument, "null device pointer");
-    const PaddedProblem p = padded_problem(raw_shape(imDim, kernelDim), boundary);
+    const ConvShape raw = raw_shape(imDim, kernelDim);
+    const PaddedProblem p = padded_problem(raw, boundary);
     const Op o = op_from(op);
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const size_t need = workspace_layout(p.padded).total();
     if (d_workspace) {
-      FC_REQUIRE(workspace_bytes >= (long long)need, kInvalidArgument, "workspace too small");
-      enqueue_convolution_padded(p, d_out, d_image, d_kernel, o, d_workspace, st);
+      FC_REQUIRE(workspace_bytes >= (long long)workspace_layout(p.padded).total(),
+                 kInvalidArgument, "workspace too small");
+      enqueue_boundary(raw, p, boundary, d_out, d_image, d_kernel, o, d_workspace,
+                       (size_t)workspace_bytes, st);
     } else {
       int dev = 0;
       FC_HIP_CHECK(hipGetDevice(&dev));
       DevicePool& pool = device_pool(dev);
       std::lock_guard<std::mutex> lk(pool.mu);
+      const size_t need = boundary_workspace(raw, p, boundary);
       void* ws = pool_reserve(&pool.ws, &pool.ws_bytes, need);
-      enqueue_convolution_padded(p, d_out, d_image, d_kernel, o, ws, st);
+      enqueue_boundary(raw, p, boundary, d_out, d_image, d_kernel, o, ws, need, st);
       // the pooled workspace is reused by the next call: finish before unlocking
       FC_HIP_CHECK(hipStreamSynchronize(st));
     }
@@ -499,8 +539,9 @@ int fcamd_convolve3d_boundary_device(float* d_out, const float* d_image, const i
 int fcamd_convolve3d_boundary_host(float* im, const int* imDim, const float* kernel,
                                    const int* kernelDim, int op, int boundary, int devCUDA) {
   return guarded([&] {
-    const PaddedProblem p = padded_problem(raw_shape(imDim, kernelDim), boundary);
-    host_convolution_padded(p, im, kernel, im, op_from(op), devCUDA);
+    const ConvShape raw = raw_shape(imDim, kernelDim);
+    const PaddedProblem p = padded_problem(raw, boundary);
+    host_convolution_padded(raw, p, boundary, im, kernel, im, op_from(op), devCUDA);
   });
 }
 

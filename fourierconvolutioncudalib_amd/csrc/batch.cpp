@@ -183,7 +183,9 @@ std::vector<std::vector<int>> lane_plan(const std::vector<ConvShape>& shapes, in
   return lanes;
 }
 
-ConvShape block_shape(const int* imDims, const int* kernelDims, int b) {
+// (lane schedule: extended where the drop-in call extends it; the length
+// groups' task tables hold plain passes)
+ConvShape block_shape(const int* imDims, const int* kernelDims, int b, int nlanes) {
   ConvShape s{};
   s.nx = imDims[3 * b];
   s.ny = imDims[3 * b + 1];
@@ -194,7 +196,8 @@ ConvShape block_shape(const int* imDims, const int* kernelDims, int b) {
   s.cx = s.kx / 2;
   s.cy = s.ky / 2;
   s.cz = s.kz / 2;
-  return s;
+  validate_block(s, nlanes);
+  return nlanes > 0 && !needs_long_path(s) ? with_extension(s) : s;
 }
 
 class BatchPlan {
@@ -252,8 +255,7 @@ BatchPlan::BatchPlan(int n, const int* imDims, const int* kernelDims, float* con
   std::vector<size_t> sizes;
   for (int b = 0; b < n; ++b) {
     Block bl{};
-    bl.s = block_shape(imDims, kernelDims, b);
-    validate_block(bl.s, nlanes);
+    bl.s = block_shape(imDims, kernelDims, b, nlanes);
     FC_REQUIRE(outs[b] && imgs[b] && kers[b], kInvalidArgument, "null block pointer");
     bl.out = outs[b];
     bl.img = imgs[b];
@@ -263,14 +265,22 @@ BatchPlan::BatchPlan(int n, const int* imDims, const int* kernelDims, float* con
   }
   std::vector<int> starts;
   if (nlanes > 0) {
-    std::vector<ConvShape> shapes;
-    for (const Block& bl : blocks_) shapes.push_back(bl.s);
-    std::vector<size_t> slot;
-    lanes_ = lane_plan(shapes, nlanes, &slot);
-    ws_need_ = 0;
-    for (size_t l = 0; l < lanes_.size(); ++l) {
-      lane_off_.push_back(ws_need_);
-      ws_need_ += slot[l];
+    auto plan_lanes = [&] {
+      std::vector<ConvShape> shapes;
+      for (const Block& bl : blocks_) shapes.push_back(bl.s);
+      std::vector<size_t> slot;
+      lanes_ = lane_plan(shapes, nlanes, &slot);
+      ws_need_ = 0;
+      lane_off_.clear();
+      for (size_t l = 0; l < lanes_.size(); ++l) {
+        lane_off_.push_back(ws_need_);
+        ws_need_ += slot[l];
+      }
+    };
+    plan_lanes();
+    if (ws && ws_bytes < ws_need_) {  // room for the unextended blocks only
+      for (Block& bl : blocks_) bl.s = direct_shape(bl.s);
+      plan_lanes();
     }
   } else {
     starts = wave_starts(sizes, wave_budget, &ws_need_);
@@ -728,13 +738,13 @@ long long fcamd_batch_workspace_bytes(int nblocks, const int* imDims, const int*
     FC_REQUIRE(nblocks >= 1 && imDims && kernelDims, kInvalidArgument, "bad batch description");
     std::vector<size_t> sizes;
     std::vector<ConvShape> shapes;
-    for (int b = 0; b < nblocks; ++b) {
-      shapes.push_back(block_shape(imDims, kernelDims, b));
-    }
     const int nlanes = default_lanes();
-    for (const ConvShape& s : shapes) {
-      validate_block(s, nlanes);
-      sizes.push_back(block_workspace(s));
+    for (int b = 0; b < nblocks; ++b) {
+      shapes.push_back(block_shape(imDims, kernelDims, b, nlanes));
+      // (the length groups need less than this where a block would be
+      // extended; one size for both schedules)
+      const ConvShape& s = shapes.back();
+      sizes.push_back(block_workspace(needs_long_path(s) ? s : with_extension(s)));
     }
     size_t need = 0;
     if (nlanes > 0) {

@@ -29,6 +29,7 @@
 #include "fft_static.hpp"
 #include "kernels_long.hpp"
 #include "static_kernels.hpp"
+#include "static_registry.hpp"
 
 namespace fcamd {
 
@@ -414,12 +415,101 @@ void validate_shape(const ConvShape& s) {
 static size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 WorkspaceLayout workspace_layout(const ConvShape& s) {
-  const size_t nxp = (size_t)padded_bins(s.nx);
+  const size_t nxp = (size_t)padded_bins(s.tx());
   WorkspaceLayout w;
-  w.spectrum = align256(sizeof(float2) * nxp * s.ny * s.nz);
+  w.spectrum = align256(sizeof(float2) * nxp * s.ty() * s.nz);
   w.krows = align256(sizeof(float2) * nxp * s.ky * s.kz);
-  w.kplanes = align256(sizeof(float2) * nxp * s.ny * s.kz);
+  w.kplanes = align256(sizeof(float2) * nxp * s.ty() * s.kz);
   return w;
+}
+
+// ---------------------------------------------------------------------------
+// extended axes
+// ---------------------------------------------------------------------------
+ConvShape direct_shape(const ConvShape& s) {
+  ConvShape d = s;
+  d.px = d.py = d.pz = 0;
+  for (int& m : d.mode) m = kMapPeriodic;
+  return d;
+}
+
+ConvShape with_extension(const ConvShape& s) {
+  const int n[3] = {s.nx, s.ny, s.nz}, k[3] = {s.kx, s.ky, s.kz};
+  int P[3];
+  bool any = false, smooth = true;
+  for (int d = 0; d < 3; ++d) {
+    P[d] = n[d];
+    if (static_lookup(n[d])) continue;
+    // axes past the reach of the in-tile chirp-z keep the plain layout, whose
+    // workspace is published per extent
+    if (n[d] > kBluesteinMaxM / 2) return s;
+    P[d] = static_length_at_least(n[d] + k[d] - 1);
+    if (P[d] == 0 || !static_lookup(P[d])) return s;
+    any = true;
+    smooth = smooth && smooth_at_least(n[d]) == n[d];
+  }
+  if (!any) return s;
+  // The extension pays until it multiplies a plane's area about fourfold and
+  // the runtime-length kernels have only small radices to run: 252 x 252 x
+  // 128 takes 86 us extended against 188 us with a 15^3 kernel (area x 1.3),
+  // 160 against 220 us with 101 x 101 x 128 (x 2.0), but 278 against 241 us
+  // with a kernel of the whole image (x 4.1).  Lengths with larger prime
+  // factors gain there too: 158 x 158 x 218 with an image-sized kernel 257
+  // against 819 us, 444 x 333 x 200 1245 against 3107 us.
+  if (smooth && (double)P[0] * P[1] > 3.0 * s.nx * s.ny) return s;
+  ConvShape e = s;
+  e.px = P[0];
+  e.py = P[1];
+  e.pz = P[2];
+  return e;
+}
+
+bool boundary_extension(const ConvShape& s, const PaddedProblem& p, int boundary, ConvShape* e) {
+  *e = s;
+  e->px = p.padded.nx;
+  e->py = p.padded.ny;
+  e->pz = p.padded.nz;
+  const int n[3] = {s.nx, s.ny, s.nz}, k[3] = {s.kx, s.ky, s.kz}, c[3] = {s.cx, s.cy, s.cz};
+  const int P[3] = {e->px, e->py, e->pz};
+  for (int d = 0; d < 3; ++d) {
+    if (!static_lookup(P[d])) return false;
+    e->mode[d] = boundary;
+    const int far = std::max(c[d], k[d] - 1 - c[d]);  // elements past either end
+    const int reach = boundary == kMapMirror ? n[d] - 1 : n[d];
+    if (P[d] != n[d] && boundary != kMapZero && boundary != kMapNearest && far > reach) return false;
+  }
+  return true;
+}
+
+AxisExt axis_ext(const ConvShape& s, int d, Op op) {
+  const int n[3] = {s.nx, s.ny, s.nz}, k[3] = {s.kx, s.ky, s.kz}, c[3] = {s.cx, s.cy, s.cz};
+  const int L = d == 0 ? s.tx() : d == 1 ? s.ty() : s.tz();
+  AxisExt e{};
+  e.n = n[d];
+  if (L == n[d] || s.mode[d] == kMapZero) return e;
+  // out[i] reads elements i - (k - 1 - c) .. i + c; a correlation the mirror
+  e.right = op == Op::kCorrelate ? k[d] - 1 - c[d] : c[d];
+  e.left = k[d] - 1 - e.right;
+  FC_REQUIRE(L >= n[d] + k[d] - 1, kInternal, "extended length too short");
+  // position p >= n is element p, position p >= L - left element p - L; one
+  // fold of the rule brings either into [0, n)
+  switch (s.mode[d]) {
+    case kMapNearest:
+      e.ra = n[d] - 1;
+      break;
+    case kMapReflect:
+      e.ra = 2 * n[d] - 1, e.rs = -1;
+      e.la = L - 1, e.ls = -1;
+      break;
+    case kMapMirror:
+      e.ra = 2 * n[d] - 2, e.rs = -1;
+      e.la = L, e.ls = -1;
+      break;
+    default:
+      e.ra = -n[d], e.rs = 1;
+      e.la = n[d] - L, e.ls = 1;
+  }
+  return e;
 }
 
 // ---------------------------------------------------------------------------
@@ -527,8 +617,13 @@ ColArgs spectrum_column_args(const ConvShape& s, const FftDesc& fy, float2* S) {
 }  // namespace
 
 void pass_x_forward(const ConvShape& s, const float* src, float2* S, const float* kernel,
-                    float2* Kx, hipStream_t st, const VPad* vp) {
+                    float2* Kx, hipStream_t st, const VPad* vp, Op op) {
   ensure_kernel_attributes();
+  if (s.extended()) {
+    PassScope ps(kPassXForward, st);
+    static_xfwd_ext(s, fft_desc(s.px, st), src, S, kernel, Kx, op, st);
+    return;
+  }
   const int nb = half_bins(s.nx);
   const long nxp = padded_bins(s.nx);
   const FftDesc fx = fft_desc(s.nx, st);
@@ -566,8 +661,14 @@ void pass_x_forward(const ConvShape& s, const float* src, float2* S, const float
   }
 }
 
-void pass_y_forward(const ConvShape& s, float2* S, const float2* Kx, float2* Kxy, hipStream_t st) {
+void pass_y_forward(const ConvShape& s, float2* S, const float2* Kx, float2* Kxy, hipStream_t st,
+                    Op op) {
   ensure_kernel_attributes();
+  if (s.extended()) {
+    PassScope ps(kPassYForward, st);
+    static_ycol_ext(s, fft_desc(s.py, st), S, -1, Kx, Kxy, op, st);
+    return;
+  }
   const int nb = half_bins(s.nx);
   const long nxp = padded_bins(s.nx);
   const FftDesc fy = fft_desc(s.ny, st);
@@ -598,30 +699,35 @@ void pass_y_forward(const ConvShape& s, float2* S, const float2* Kx, float2* Kxy
 }
 
 void forward_xy(const ConvShape& s, const float* src, float2* S, const float* kernel, float2* Kx,
-                float2* Kxy, hipStream_t st, const VPad* vp) {
-  pass_x_forward(s, src, S, kernel, Kx, st, vp);
-  pass_y_forward(s, S, kernel ? Kx : nullptr, Kxy, st);
+                float2* Kxy, hipStream_t st, const VPad* vp, Op op) {
+  pass_x_forward(s, src, S, kernel, Kx, st, vp, op);
+  pass_y_forward(s, src ? S : nullptr, kernel ? Kx : nullptr, Kxy, st, op);
 }
 
 void z_pass(const ConvShape& s, float2* S, const float2* operand, bool dense, bool conj,
             hipStream_t st, int out_planes, int out_shift) {
   ensure_kernel_attributes();
-  const long nxp = padded_bins(s.nx);
+  const long nxp = padded_bins(s.tx());
   PassScope ps(kPassZFused, st);
   ZArgs a{};
-  a.fft = fft_desc(s.nz, st);
+  a.fft = fft_desc(s.tz(), st);
   a.tx = col_tile(a.fft.buf(), 3);
-  a.nbins = half_bins(s.nx);
+  a.nbins = half_bins(s.tx());
   a.s = S;
   a.s_row = nxp;
-  a.s_plane = (long)s.ny * nxp;
+  a.s_plane = (long)s.ty() * nxp;
   a.k = operand;
   a.k_row = nxp;
-  a.k_plane = (long)s.ny * nxp;
+  a.k_plane = (long)s.ty() * nxp;
   a.nvalid = dense ? s.nz : s.kz;
   a.center = dense ? 0 : s.cz;
   a.conj = conj ? 1 : 0;
-  a.scale = (float)(1.0 / (double)s.voxels());
+  a.scale = (float)(1.0 / ((double)s.tx() * s.ty() * s.tz()));
+  if (s.extended()) {
+    FC_REQUIRE(!dense && out_planes >= s.nz && out_shift == 0, kInternal, "extended z pass form");
+    static_zfused_ext(s, a, axis_ext(s, 2, conj ? Op::kCorrelate : Op::kConvolve), st);
+    return;
+  }
   // 0 keeps the plain in-place store; a shift always takes the rotated one
   a.out_planes = (out_planes < s.nz || out_shift != 0) ? std::min(out_planes, s.nz) : 0;
   a.out_shift = out_shift;
@@ -631,6 +737,11 @@ void z_pass(const ConvShape& s, float2* S, const float2* operand, bool dense, bo
 
 void pass_y_inverse(const ConvShape& s, float2* S, hipStream_t st) {
   ensure_kernel_attributes();
+  if (s.extended()) {
+    PassScope ps(kPassYInverse, st);
+    static_ycol_ext(s, fft_desc(s.py, st), S, +1, nullptr, nullptr, Op::kConvolve, st);
+    return;
+  }
   const FftDesc fy = fft_desc(s.ny, st);
   if (s.ny > 1) {
     PassScope ps(kPassYInverse, st);
@@ -647,6 +758,11 @@ void inverse_yx(const ConvShape& s, float2* S, float* dst, hipStream_t st, const
 void pass_x_inverse(const ConvShape& s, const float2* S, float* dst, hipStream_t st,
                     const VPad* vp) {
   ensure_kernel_attributes();
+  if (s.extended()) {
+    PassScope ps(kPassXInverse, st);
+    static_xinv_ext(s, fft_desc(s.px, st), S, dst, st);
+    return;
+  }
   const FftDesc fx = fft_desc(s.nx, st);
   PassScope ps(kPassXInverse, st);
   if (!static_xinv(s, fx, S, dst, st, vp)) {
@@ -688,11 +804,11 @@ int table_lengths(const ConvShape& s, int* L) {
       if (L[i] == len) return;
     L[n++] = len;
   };
-  add(s.nx);
-  add(s.ny);
-  add(s.nz);
+  add(s.tx());
+  add(s.ty());
+  add(s.tz());
   for (int dir : {-1, +1})
-    if (plane_split(s, dir)) add(plane_half_length(s, dir));
+    if (plane_path(s, dir) && plane_split(s, dir)) add(plane_half_length(s, dir));
   return n;
 }
 
@@ -796,22 +912,66 @@ void enqueue_convolution_padded(const PaddedProblem& p, float* d_out, const floa
   FC_HIP_CHECK(hipGetLastError());
 }
 
-void enqueue_convolution(const ConvShape& s, float* d_out, const float* d_image,
+void enqueue_forward(const ConvShape& s, const float* d_image, float2* S, const float* d_kernel,
+                     float2* Kx, float2* Kxy, Op op, hipStream_t st) {
+  if (plane_path(s, -1))
+    plane_forward(s, d_image, S, d_kernel, Kxy, st);
+  else
+    forward_xy(s, d_image, S, d_kernel, Kx, Kxy, st, nullptr, op);
+}
+
+void enqueue_inverse(const ConvShape& s, float2* S, float* d_out, hipStream_t st) {
+  if (plane_path(s, +1))
+    plane_inverse(s, S, d_out, st);
+  else
+    inverse_yx(s, S, d_out, st);
+}
+
+namespace {
+// Whether the tables of an extended shape exist or may be made now.  A
+// stream that is capturing records neither the allocation nor the copy: such
+// a call runs the shape unextended, whose tables depend on the image's
+// extents only (any kernel size used before has made them, below).
+bool extension_tables(const ConvShape& s, hipStream_t st) {
+  int lens[5];
+  const int n = table_lengths(s, lens);
+  bool have = true;
+  {
+    const int dev = current_device();
+    std::lock_guard<std::mutex> lk(g_tw_mu);
+    for (int i = 0; i < n; ++i) have = have && g_desc.count(std::make_pair(dev, lens[i])) != 0;
+  }
+  if (have) return true;
+  if (st != nullptr) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    FC_HIP_CHECK(hipStreamIsCapturing(st, &cs));
+    if (cs != hipStreamCaptureStatusNone) return false;
+  }
+  const ConvShape d = direct_shape(s);
+  const int m = table_lengths(d, lens);
+  for (int i = 0; i < m; ++i) (void)fft_desc(lens[i]);
+  return true;
+}
+}  // namespace
+
+void enqueue_convolution(const ConvShape& shape, float* d_out, const float* d_image,
                          const float* d_kernel, Op op, void* ws, hipStream_t st) {
+  if (shape.extended() && !extension_tables(shape, st))
+    run_convolution(direct_shape(shape), d_out, d_image, d_kernel, op, ws, st);
+  else
+    run_convolution(shape, d_out, d_image, d_kernel, op, ws, st);
+}
+
+void run_convolution(const ConvShape& s, float* d_out, const float* d_image,
+                     const float* d_kernel, Op op, void* ws, hipStream_t st) {
   const WorkspaceLayout wl = workspace_layout(s);
   char* base = static_cast<char*>(ws);
   float2* S = reinterpret_cast<float2*>(base);
   float2* Kx = reinterpret_cast<float2*>(base + wl.spectrum);
   float2* Kxy = reinterpret_cast<float2*>(base + wl.spectrum + wl.krows);
-  if (plane_path(s, -1))
-    plane_forward(s, d_image, S, d_kernel, Kxy, st);
-  else
-    forward_xy(s, d_image, S, d_kernel, Kx, Kxy, st);
+  enqueue_forward(s, d_image, S, d_kernel, Kx, Kxy, op, st);
   z_pass(s, S, Kxy, false, op == Op::kCorrelate, st);
-  if (plane_path(s, +1))
-    plane_inverse(s, S, d_out, st);
-  else
-    inverse_yx(s, S, d_out, st);
+  enqueue_inverse(s, S, d_out, st);
   FC_HIP_CHECK(hipGetLastError());
 }
 

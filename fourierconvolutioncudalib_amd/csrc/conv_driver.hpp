@@ -18,8 +18,25 @@ struct ConvShape {
   int nx, ny, nz;
   int kx, ky, kz;
   int cx, cy, cz;
+  // Transform lengths of an extended problem (with_extension; 0: the image
+  // extents, no extension) and the rule its axes are extended by
+  int px = 0, py = 0, pz = 0;
+  int mode[3] = {kMapPeriodic, kMapPeriodic, kMapPeriodic};
+  bool extended() const { return px > 0; }
+  int tx() const { return px > 0 ? px : nx; }
+  int ty() const { return py > 0 ? py : ny; }
+  int tz() const { return pz > 0 ? pz : nz; }
   long long voxels() const { return (long long)nx * ny * nz; }
 };
+
+// `s` with the axes that have no compile-time kernels extended to the next
+// length that has (AxisExt in kernels.hpp): a circular convolution by a
+// compact kernel only needs its k - 1 neighbours past the ends, so any
+// length >= n + k - 1 gives the same result.  Returned unchanged where no
+// such length is worth it (the runtime-length kernels then run).
+ConvShape with_extension(const ConvShape& s);
+// the same problem without the extension
+ConvShape direct_shape(const ConvShape& s);
 
 // Workspace carve-up (bytes, each region 256-byte aligned).
 struct WorkspaceLayout {
@@ -70,6 +87,9 @@ void set_fft_desc_override(const FftDescSet* set);
 
 enum class Op : int { kConvolve = 0, kCorrelate = 1 };
 
+// extension of axis d (0 x, 1 y, 2 z) of an extended shape
+AxisExt axis_ext(const ConvShape& s, int d, Op op);
+
 // Passes of one convolution, in launch order (for per-pass event timing).
 enum Pass : int {
   kPassKernelRows = 0,
@@ -95,6 +115,16 @@ void pass_timing_collect(double* ms, int* count);
 void enqueue_convolution(const ConvShape& s, float* d_out, const float* d_image,
                          const float* d_kernel, Op op, void* ws, hipStream_t stream);
 
+// the same for a shape that is known to have (or may make) its tables
+void run_convolution(const ConvShape& s, float* d_out, const float* d_image,
+                     const float* d_kernel, Op op, void* ws, hipStream_t stream);
+// its three parts: image (and kernel) to S (and Kxy), the product with the
+// kernel's spectrum, back to the real image; S, Kx and Kxy are the regions of
+// workspace_layout(s).  Either of d_image and d_kernel may be null.
+void enqueue_forward(const ConvShape& s, const float* d_image, float2* S, const float* d_kernel,
+                     float2* Kx, float2* Kxy, Op op, hipStream_t stream);
+void enqueue_inverse(const ConvShape& s, float2* S, float* d_out, hipStream_t stream);
+
 // Building blocks (all asynchronous on `stream`):
 //   forward_xy  real volume -> half spectrum S (x-R2C, y-FFT); with `kernel`
 //               also the compact kernel's rows Kx and planes Kxy
@@ -102,13 +132,15 @@ void enqueue_convolution(const ConvShape& s, float* d_out, const float* d_image,
 //               compact kernel planes (dense = false) or a second spectrum
 //   inverse_yx  S -> real volume (inverse y-FFT, x-C2R), unnormalised
 void forward_xy(const ConvShape& s, const float* src, float2* S, const float* kernel, float2* Kx,
-                float2* Kxy, hipStream_t stream, const VPad* vp = nullptr);
+                float2* Kxy, hipStream_t stream, const VPad* vp = nullptr, Op op = Op::kConvolve);
 // the single passes forward_xy / inverse_yx are made of; with `vp` the x
 // passes read a virtually padded image and write its cropped interior
+// (`op` decides which neighbours an extended axis needs)
 void pass_x_forward(const ConvShape& s, const float* src, float2* S, const float* kernel,
-                    float2* Kx, hipStream_t stream, const VPad* vp = nullptr);
+                    float2* Kx, hipStream_t stream, const VPad* vp = nullptr,
+                    Op op = Op::kConvolve);
 void pass_y_forward(const ConvShape& s, float2* S, const float2* Kx, float2* Kxy,
-                    hipStream_t stream);
+                    hipStream_t stream, Op op = Op::kConvolve);
 void pass_y_inverse(const ConvShape& s, float2* S, hipStream_t stream);
 void pass_x_inverse(const ConvShape& s, const float2* S, float* dst, hipStream_t stream,
                     const VPad* vp = nullptr);
@@ -155,6 +187,10 @@ PaddedProblem padded_problem(const ConvShape& s, int boundary);
 // smallest fast transform length >= n (a 7-smooth compile-time length when
 // one is within 25 %, else the smallest 7-smooth length)
 int fast_length(int n);
+// The boundary-mode problem of image shape s as an extended shape, when every
+// padded length has compile-time kernels and one fold of the rule reaches all
+// the neighbours the kernel needs; false otherwise.
+bool boundary_extension(const ConvShape& s, const PaddedProblem& p, int boundary, ConvShape* e);
 void enqueue_convolution_padded(const PaddedProblem& p, float* d_out, const float* d_image,
                                 const float* d_kernel, Op op, void* ws, hipStream_t stream);
 

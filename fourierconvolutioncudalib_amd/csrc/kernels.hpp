@@ -86,6 +86,29 @@ __host__ __device__ inline bool vpad_out_row(const VPad& v, long r, long* out_ro
   return yo >= 0 && yo < v.m[1] && zo >= 0 && zo < v.m[2];
 }
 
+// Extension of one axis to a longer transform.  n image elements sit at
+// positions [0, n) of a transform of length L >= n + right + left; positions
+// [n, n + right) hold the elements past the end and [L - left, L) those
+// before the start (the transform is circular), each an affine map of the
+// position (one fold of the boundary rule), and the gap reads zero.  An
+// output at a position below n then depends on the extended image only, so
+// the passes write just those: every pass moves the image's own rows and
+// planes, whatever L is.
+struct AxisExt {
+  int n;
+  int right, left;
+  int ra, rs;  // position p past the end reads element ra + rs * p
+  int la, ls;  // position p before the start reads element la + ls * p
+};
+
+// element that position p >= n of a length-L transform reads, -1: zero
+__host__ __device__ inline int axis_ext_src(const AxisExt& e, int L, int p) {
+  int q = -1;
+  if (p < e.n + e.right) q = e.ra + e.rs * p;
+  if (p >= L - e.left) q = e.la + e.ls * p;
+  return q;
+}
+
 struct XPassArgs {
   FftDesc fft;          // length nx
   long nrows;           // rows to transform
@@ -216,6 +239,27 @@ struct Col2 {
   int ntx;          // bin tiles per row
   long m_tiles;     // tiles of the image part (after the kernel's)
   long ntiles;      // total tiles
+};
+
+// Passes over an extended image (AxisExt): the image's ny rows of its
+// nplanes planes sit in spectrum planes of ty >= ny rows.
+struct XExtArgs {
+  XPassArgs m;  // image rows (src_row / dst_row of the real side unused)
+  XPassArgs k;  // forward: kernel rows (kshift)
+  AxisExt ext;
+  int ny;        // image rows per plane
+  int groups;    // workgroups per plane (filled by the launcher)
+  long nplanes;  // image planes
+  long spec_plane;  // spectrum elements between planes (ty rows)
+  long k_blocks;    // workgroups of the kernel rows (filled by the launcher)
+};
+struct ColExtArgs {
+  Col2 c;
+  AxisExt ext;  // forward: rows read; inverse: rows [0, n) written
+};
+struct ZExtArgs {
+  ZArgs z;
+  AxisExt ext;
 };
 
 // fused multiview Richardson-Lucy passes (rl_kernels.hpp)

@@ -34,12 +34,7 @@ void plan_kernel(ConvPlan& p, const float* d_kernel, hipStream_t st) {
   // the kernel's rows and planes only (no image in these launches), by the
   // same kernels a plain call of this shape uses, so that executing the
   // plan reproduces the plain call bit for bit
-  if (plane_path(p.s, -1)) {
-    plane_forward(p.s, nullptr, nullptr, d_kernel, p.Kxy, st);
-  } else {
-    pass_x_forward(p.s, nullptr, nullptr, d_kernel, p.Kx, st);
-    pass_y_forward(p.s, nullptr, p.Kx, p.Kxy, st);
-  }
+  enqueue_forward(p.s, nullptr, nullptr, d_kernel, p.Kx, p.Kxy, p.op, st);
   FC_HIP_CHECK(hipGetLastError());
 }
 
@@ -78,6 +73,11 @@ void* fcamd_conv_plan_create(const int* imDim, const int* kernelDim, const float
       validate_long_shape(s);
     else
       validate_shape(s);
+    if (!lng) {
+      // a caller's workspace sized for the unextended transform stays enough
+      const ConvShape e = with_extension(s);
+      if (!d_workspace || workspace_bytes >= (long long)workspace_layout(e).total()) s = e;
+    }
     driver_init();
     auto* p = new ConvPlan();
     p->s = s;
@@ -132,15 +132,9 @@ int fcamd_conv_plan_execute(void* plan, float* d_out, const float* d_image, void
       long_apply_spectrum(p.s, d_out, d_image, p.op, p.ws, st);
       return;
     }
-    if (plane_path(p.s, -1))
-      plane_forward(p.s, d_image, p.S, nullptr, nullptr, st);
-    else
-      forward_xy(p.s, d_image, p.S, nullptr, nullptr, nullptr, st);
+    enqueue_forward(p.s, d_image, p.S, nullptr, nullptr, nullptr, p.op, st);
     z_pass(p.s, p.S, p.Kxy, false, p.op == Op::kCorrelate, st);
-    if (plane_path(p.s, +1))
-      plane_inverse(p.s, p.S, d_out, st);
-    else
-      inverse_yx(p.s, p.S, d_out, st);
+    enqueue_inverse(p.s, p.S, d_out, st);
     FC_HIP_CHECK(hipGetLastError());
   });
 }

@@ -63,7 +63,9 @@ RLProblem make_problem(int nviews, const int* imDim, const int* kernelDims) {
       validate_long_shape(s);
     else
       validate_shape(s);
-    p.views.push_back(s);
+    // (compile-time extents are returned unchanged, so only the unfused form
+    // sees extended views)
+    p.views.push_back(needs_long_path(s) ? s : with_extension(s));
   }
   return p;
 }

@@ -72,10 +72,26 @@ StaticEntry* static_lookup(int L) {
     return v != nullptr && v[0] == '1';
   }();
   if (env_disabled || g_disabled) return nullptr;
+  return static_entry(L);
+}
+
+StaticEntry* static_entry(int L) {
   ensure_registered();
   std::lock_guard<std::mutex> lk(registry_mu());
   auto it = registry().find(L);
   return it == registry().end() ? nullptr : it->second.get();
+}
+
+int static_length_at_least(int n) {
+  ensure_registered();
+  std::lock_guard<std::mutex> lk(registry_mu());
+  for (auto it = registry().lower_bound(n); it != registry().end(); ++it) {
+    int r = it->first;
+    for (int f : {2, 3, 5, 7})
+      while (r % f == 0) r /= f;
+    if (r == 1) return it->first;
+  }
+  return 0;
 }
 
 int persistent_blocks(const void* kernel, int threads) {
@@ -227,6 +243,99 @@ bool static_zfused(const ConvShape& s, const ZArgs& a, hipStream_t st) {
   if (!e) return false;
   run_selected(e->zfused, e->selected[kSZ], a, (long)s.ny, st);
   return true;
+}
+
+namespace {
+StaticEntry* entry_of(int L) {
+  StaticEntry* e = static_entry(L);
+  FC_REQUIRE(e != nullptr, kInternal, "extended shape without compile-time kernels");
+  return e;
+}
+}  // namespace
+
+void static_xfwd_ext(const ConvShape& s, const FftDesc& fx, const float* src, float2* S,
+                     const float* kernel, float2* krows, Op op, hipStream_t st) {
+  const long nxp = padded_bins(s.px);
+  XExtArgs a{};
+  a.m.fft = fx;
+  a.m.nbins = half_bins(s.px);
+  a.m.src = src;
+  a.m.dst = S;
+  a.m.dst_row = nxp;
+  a.ext = axis_ext(s, 0, op);
+  a.ny = s.ny;
+  a.nplanes = src ? s.nz : 0;
+  a.spec_plane = (long)s.py * nxp;
+  a.k = a.m;
+  a.k.nrows = kernel ? (long)s.ky * s.kz : 0;
+  a.k.src = kernel;
+  a.k.dst = krows;
+  a.k.src_row = s.kx;
+  a.k.klen = s.kx;
+  a.k.kcenter = s.cx;
+  a.k.kshift = 1;
+  entry_of(s.px)->ext.xfwd(a, st);
+}
+
+void static_xinv_ext(const ConvShape& s, const FftDesc& fx, const float2* S, float* dst,
+                     hipStream_t st) {
+  const long nxp = padded_bins(s.px);
+  XExtArgs a{};
+  a.m.fft = fx;
+  a.m.nbins = half_bins(s.px);
+  a.m.csrc = S;
+  a.m.src_row = nxp;
+  a.m.rdst = dst;
+  a.ext.n = s.nx;
+  a.ny = s.ny;
+  a.nplanes = s.nz;
+  a.spec_plane = (long)s.py * nxp;
+  entry_of(s.px)->ext.xinv(a, st);
+}
+
+void static_ycol_ext(const ConvShape& s, const FftDesc& fy, float2* S, int dir,
+                     const float2* krows, float2* kplanes, Op op, hipStream_t st) {
+  StaticEntry* e = entry_of(s.py);
+  const long nxp = padded_bins(s.px);
+  ColExtArgs b{};
+  Col2& a = b.c;
+  a.m.fft = fy;
+  a.m.nbins = half_bins(s.px);
+  a.m.src = S;
+  a.m.dst = S;
+  a.m.src_outer = a.m.dst_outer = (long)s.py * nxp;
+  a.m.src_elem = a.m.dst_elem = nxp;
+  a.m.nvalid = s.py;
+  a.m.center = 0;
+  a.m_outer = S ? s.nz : 0;
+  a.k = a.m;
+  a.k_outer = 0;
+  if (krows) {
+    a.k.src = krows;
+    a.k.dst = kplanes;
+    a.k.src_outer = (long)s.ky * nxp;
+    a.k.nvalid = s.ky;
+    a.k.center = s.cy;
+    a.k_outer = s.kz;
+  }
+  if (s.py == s.ny) {
+    run_selected(e->col, e->selected[dir < 0 ? kSCol : kSColInv], a, dir, st);
+    return;
+  }
+  b.ext = axis_ext(s, 1, op);
+  e->ext.col(b, dir, st);
+}
+
+void static_zfused_ext(const ConvShape& s, const ZArgs& a, const AxisExt& ext, hipStream_t st) {
+  StaticEntry* e = entry_of(s.pz);
+  if (s.pz == s.nz) {
+    run_selected(e->zfused, e->selected[kSZ], a, (long)s.py, st);
+    return;
+  }
+  ZExtArgs b{};
+  b.z = a;
+  b.ext = ext;
+  e->ext.zfused(b, (long)s.py, st);
 }
 
 void static_kernels_allow_large_lds() {}

@@ -27,6 +27,16 @@ bool static_ycol(const ConvShape& s, const FftDesc& fy, float2* S, int dir, cons
 bool static_ycol_fill(const ConvShape& s, const FftDesc& fy, float2* S, int dir, int cus,
                       hipStream_t st);
 bool static_zfused(const ConvShape& s, const ZArgs& a, hipStream_t st);
+// The passes of an extended shape (ConvShape::px; every axis of it has
+// compile-time kernels).  An axis whose length is the image's runs the plain
+// variants where the layout allows.  src / S and kernel / krows may be null.
+void static_xfwd_ext(const ConvShape& s, const FftDesc& fx, const float* src, float2* S,
+                     const float* kernel, float2* krows, Op op, hipStream_t st);
+void static_xinv_ext(const ConvShape& s, const FftDesc& fx, const float2* S, float* dst,
+                     hipStream_t st);
+void static_ycol_ext(const ConvShape& s, const FftDesc& fy, float2* S, int dir,
+                     const float2* krows, float2* kplanes, Op op, hipStream_t st);
+void static_zfused_ext(const ConvShape& s, const ZArgs& a, const AxisExt& ext, hipStream_t st);
 void static_kernels_allow_large_lds();
 
 }  // namespace fcamd

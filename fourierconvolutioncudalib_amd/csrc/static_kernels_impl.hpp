@@ -579,6 +579,163 @@ sk_xinv_crop_flat(XPassArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// x passes over an extended image (AxisExt in kernels.hpp).  The workgroup's
+// rows lie in one plane, so they are one run of nr * n floats in the image;
+// it moves between HBM and the staging rows with consecutive lanes on
+// consecutive floats (rows of any length start at any alignment), as
+// 16-byte pieces where the rows are not extended.  The extension is applied
+// on the way from the staging rows to the transform's registers, so a row is
+// read from HBM once.
+// ---------------------------------------------------------------------------
+// row of element i of a run of rows of n < 4096 elements: (i + 1/2) / n is at
+// least 1 / (2n) > 1.2e-4 from an integer, and its single-precision error
+// stays below 2^-22 times the row count (< 2^7)
+__device__ __forceinline__ int run_row(int i, float inv_n) { return (int)(((float)i + 0.5f) * inv_n); }
+
+template <int L, int PAIRS>
+__device__ __forceinline__ void xfwd_ext_body(const XExtArgs& a, long blk, float2* lds) {
+  using P = PlanOf<L, false>;
+  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL, NB = XStage<L>::NB;
+  constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
+  const unsigned z = (unsigned)blk / (unsigned)a.groups;
+  const int r0 = 2 * PAIRS * (int)((unsigned)blk - z * (unsigned)a.groups);
+  const int nr = a.ny - r0 < MAXR ? a.ny - r0 : MAXR;
+  const AxisExt e = a.ext;
+  const int n = e.n;
+  float* st = reinterpret_cast<float*>(lds);
+  const float* src = a.m.src + ((long)z * a.ny + r0) * n;
+  if (n == L) {
+    xflat_load_rows<L, NT, MAXR>(src, st, nr);
+  } else {
+    constexpr int IT = (MAXR * L + NT - 1) / NT;
+    const int tot = nr * n;
+    const float inv = 1.f / (float)n;
+    float r[IT];
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+      const int i = threadIdx.x + j * NT;
+      r[j] = 0.f;
+      if (i < tot) r[j] = src[i];
+    }
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+      const int i = threadIdx.x + j * NT;
+      if (i < tot) {
+        const int row = run_row(i, inv);
+        st[row * SL + (i - row * n)] = r[j];
+      }
+    }
+  }
+  __syncthreads();
+  const int t = threadIdx.x % T, c = threadIdx.x / T;
+  const bool oka = 2 * c < nr, okb = 2 * c + 1 < nr;
+  float2 v[P::MAXE()];
+  sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
+    const int q = pos < n ? pos : axis_ext_src(e, L, pos);
+    const bool in = q >= 0;
+    v[slot] = make_float2(in && oka ? st[2 * c * SL + q] : 0.f,
+                          in && okb ? st[(2 * c + 1) * SL + q] : 0.f);
+  });
+  __syncthreads();
+  float2* row = lds + c * LP;
+  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  sfft_run<L, false, -1, 9>(v, t, row, addr, a.m.fft.stw);
+  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(pos)] = v[slot]; });
+  __syncthreads();
+  float2* dst = a.m.dst + (long)z * a.spec_plane + (long)r0 * a.m.dst_row;
+  constexpr int IT = (MAXR * NB + NT - 1) / NT;
+  const int nbins = nr * NB;
+#pragma unroll
+  for (int j = 0; j < IT; ++j) {
+    const int i = threadIdx.x + j * NT;
+    if (i < nbins) {
+      const int r = i / NB, kb = i - r * NB;
+      const float2* pr = lds + (r >> 1) * LP;
+      const float2 Z = pr[addr(kb)];
+      const float2 Zm = pr[addr(kb == 0 ? 0 : L - kb)];
+      dst[r * a.m.dst_row + kb] = (r & 1) ? make_float2(0.5f * (Z.y + Zm.y), 0.5f * (Zm.x - Z.x))
+                                          : make_float2(0.5f * (Z.x + Zm.x), 0.5f * (Z.y - Zm.y));
+    }
+  }
+}
+
+template <int L, int PAIRS>
+__global__ void __launch_bounds__(PAIRS * threads_per_transform<L>())
+sk_xfwd_ext(XExtArgs a) {
+  static_assert(xflat_lds_floats<L>(PAIRS) * 4 <= 65536, "flat x pass LDS");
+  __shared__ float2 lds[xflat_lds_floats<L>(PAIRS) / 2];
+  if ((long)blockIdx.x >= a.k_blocks)
+    xfwd_ext_body<L, PAIRS>(a, (long)blockIdx.x - a.k_blocks, lds);
+  else
+    xfwd_body<L, PAIRS>(a.k, blockIdx.x, lds);
+}
+
+template <int L, int PAIRS>
+__global__ void __launch_bounds__(PAIRS * threads_per_transform<L>())
+sk_xinv_ext(XExtArgs a) {
+  using P = PlanOf<L, false>;
+  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL, NB = XStage<L>::NB;
+  constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
+  static_assert(xflat_lds_floats<L>(PAIRS) * 4 <= 65536, "flat x pass LDS");
+  __shared__ float2 lds[xflat_lds_floats<L>(PAIRS) / 2];
+  const unsigned z = blockIdx.x / (unsigned)a.groups;
+  const int r0 = 2 * PAIRS * (int)(blockIdx.x - z * (unsigned)a.groups);
+  const int nr = a.ny - r0 < MAXR ? a.ny - r0 : MAXR;
+  xflat_load_bins<L, NT, MAXR>(a.m.csrc + (long)z * a.spec_plane + (long)r0 * a.m.src_row,
+                               a.m.src_row, lds, nr);
+  __syncthreads();
+  const int t = threadIdx.x % T, c = threadIdx.x / T;
+  const bool oka = 2 * c < nr, okb = 2 * c + 1 < nr;
+  const float2* sa = lds + 2 * c * NB;
+  const float2* sb = sa + NB;
+  float2 v[P::MAXE()];
+  // Z = A' + iB' over all L positions; position L - kb takes the conjugates
+  sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
+    const bool mirror = pos >= NB;
+    const int kb = mirror ? L - pos : pos;
+    float2 A = oka ? sa[kb] : make_float2(0.f, 0.f);
+    float2 B = okb ? sb[kb] : make_float2(0.f, 0.f);
+    if (kb == 0 || 2 * kb == L) {
+      A.y = 0.f;
+      B.y = 0.f;
+    }
+    if (mirror) {
+      A.y = -A.y;
+      B.y = -B.y;
+    }
+    v[slot] = make_float2(A.x - B.y, A.y + B.x);
+  });
+  __syncthreads();
+  float2* row = lds + c * LP;
+  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  sfft_run<L, false, +1>(v, t, row, addr, a.m.fft.stw);
+  // sfft_run ends on a barrier after its last LDS read
+  float* st = reinterpret_cast<float*>(lds);
+  const int n = a.ext.n;
+  sfft_for_outputs<L, false>(t, [&](int slot, int pos) {
+    st[2 * c * SL + pos] = v[slot].x;
+    st[(2 * c + 1) * SL + pos] = v[slot].y;
+  });
+  __syncthreads();
+  float* dst = a.m.rdst + ((long)z * a.ny + r0) * n;
+  if (n == L) {
+    xflat_store_rows<L, NT, MAXR>(dst, st, nr);
+    return;
+  }
+  constexpr int IT = (MAXR * L + NT - 1) / NT;
+  const int tot = nr * n;
+  const float inv = 1.f / (float)n;
+#pragma unroll
+  for (int j = 0; j < IT; ++j) {
+    const int i = threadIdx.x + j * NT;
+    if (i < tot) {
+      const int r = run_row(i, inv);
+      dst[i] = st[r * SL + (i - r * n)];
+    }
+  }
+}
+
 // batched x passes: workgroup i serves tasks[i] = {argument record, row-pair
 // group}.  Image rows (dense, unshifted) take the flat bodies; the compact
 // kernel's rows the per-pair body.
@@ -658,6 +815,35 @@ struct ColTile {
     float2* dt = a->dst + base_dst + (long)t * es;
     sfft_for_outputs<L, REV>(t, [&](int slot, int pos) { dt[(long)(pos - t) * es] = v[slot]; });
   }
+  // extended columns (AxisExt): the rows at positions below n are read and
+  // written through the base and uniform offset; only the waves that hold
+  // positions of the extension compute the mapped row
+  __device__ void load_ext(const AxisExt& e, int t, float2 (&v)[MAXE]) const {
+    const float2* src = a->src + base_src;
+    const long es = a->src_elem;
+    const float2* st = src + (long)t * es;
+    const bool okk = ok;
+    sfft_for_inputs<L, REV>(t, [&](int slot, int pos) {
+      float2 val = make_float2(0.f, 0.f);
+      if (okk) {
+        if (pos < e.n) {
+          val = st[(long)(pos - t) * es];
+        } else {
+          const int q = axis_ext_src(e, L, pos);
+          if (q >= 0) val = src[(long)q * es];
+        }
+      }
+      v[slot] = val;
+    });
+  }
+  __device__ void store_below(int n, int t, const float2 (&v)[MAXE]) const {
+    if (!ok) return;
+    const long es = a->dst_elem;
+    float2* dt = a->dst + base_dst + (long)t * es;
+    sfft_for_outputs<L, REV>(t, [&](int slot, int pos) {
+      if (pos < n) dt[(long)(pos - t) * es] = v[slot];
+    });
+  }
 };
 
 // kernel-plane tiles first, then the image's
@@ -688,6 +874,35 @@ sk_col(Col2 a2) {
   long local;
   const ColArgs& a = col2_args(a2, blockIdx.x, &local);
   col_body<L, TX, DIR, REV>(a, local, lds);
+}
+
+// y pass of an extended image: the forward reads the image's rows (mapped
+// past their ends) and writes all L, the inverse reads all L and writes the
+// image's
+template <int L, int TX, int DIR>
+__global__ void __launch_bounds__(TX * threads_per_transform<L>())
+sk_col_ext(ColExtArgs b) {
+  using CT = ColTile<L, TX>;
+  __shared__ float2 lds[L * TX];
+  long local;
+  const ColArgs& a = col2_args(b.c, blockIdx.x, &local);
+  if (DIR < 0 && (long)blockIdx.x < b.c.ntiles - b.c.m_tiles) {  // kernel planes
+    col_body<L, TX, DIR, false>(a, local, lds);
+    return;
+  }
+  const int c = threadIdx.x % TX, t = threadIdx.x / TX;
+  const CT tile(a, local, c);
+  float2 v[CT::MAXE];
+  if (DIR < 0)
+    tile.load_ext(b.ext, t, v);
+  else
+    tile.load(t, v);
+  auto addr = [&](int pos) { return pos * TX + c; };
+  sfft_run<L, false, DIR>(v, t, lds, addr, a.fft.stw);
+  if (DIR < 0)
+    tile.store(t, v);
+  else
+    tile.store_below(b.ext.n, t, v);
 }
 
 template <int L, int TX, int DIR>
@@ -828,6 +1043,34 @@ struct ZTile {
     float2* ct = col + (long)t * sp;
     sfft_for_outputs<L, true>(t, [&](int slot, int pos) { ct[(long)(pos - t) * sp] = v[slot]; });
   }
+  // extended columns (AxisExt): planes mapped past the image's ends on the
+  // way in, only the image's own planes written
+  __device__ void load_ext(const ZArgs& a, const AxisExt& e, int t, float2 (&v)[MAXE]) const {
+    const long sp = a.s_plane;
+    const float2* ct = col + (long)t * sp;
+    const float2* c0 = col;
+    const bool okk = ok;
+    sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
+      float2 val = make_float2(0.f, 0.f);
+      if (okk) {
+        if (pos < e.n) {
+          val = ct[(long)(pos - t) * sp];
+        } else {
+          const int q = axis_ext_src(e, L, pos);
+          if (q >= 0) val = c0[(long)q * sp];
+        }
+      }
+      v[slot] = val;
+    });
+  }
+  __device__ void store_below(const ZArgs& a, int n, int t, const float2 (&v)[MAXE]) const {
+    if (!ok) return;
+    const long sp = a.s_plane;
+    float2* ct = col + (long)t * sp;
+    sfft_for_outputs<L, true>(t, [&](int slot, int pos) {
+      if (pos < n) ct[(long)(pos - t) * sp] = v[slot];
+    });
+  }
   // kernel column: taps j < nvalid placed circularly at (j - center) mod L
   __device__ void load_kernel(const ZArgs& a, int t, float2 (&w)[MAXE]) const {
     const long kp = a.k_plane;
@@ -885,10 +1128,11 @@ constexpr int ktap_slots() {
 // inputs are read back by broadcast.  Compared with transforming the
 // kernel column like the image's, this drops its stage-0 butterflies, its
 // per-slot predicated loads and one LDS exchange (two per tile remain).
-template <int L, int TX>
+// (`keep`: positions written, L or the planes of an extended image)
+template <int L, int TX, bool EXT = false>
 __device__ __forceinline__ void zfused_sparse_body(const ZArgs& a, const ZTile<L, TX>& tile, int t,
                                                    int c, float2 (&v)[ZTile<L, TX>::MAXE],
-                                                   float2* lds, float2* ktaps) {
+                                                   float2* lds, float2* ktaps, int keep = L) {
   using P = PlanOf<L, false>;
   constexpr int R1 = P::R(1), M1 = P::M(1), NB1 = P::NB(1), T = P::T;
   constexpr int MAXE = ZTile<L, TX>::MAXE;
@@ -935,7 +1179,10 @@ __device__ __forceinline__ void zfused_sparse_body(const ZArgs& a, const ZTile<L
   sfft_butterflies<L, false, -1, 1>(w, t);
   zproduct_prescaled<L>(v, w, t, a.conj != 0);
   sfft_run<L, true, +1>(v, t, lds, addr, a.fft.stw);
-  tile.template store<false>(a, t, v);
+  if constexpr (EXT)
+    tile.store_below(a, keep, t, v);
+  else
+    tile.template store<false>(a, t, v);
 }
 
 // whether the two-stage tap path applies to this launch
@@ -991,6 +1238,33 @@ sb_zfused(const ZArgs* __restrict__ args, const int2* __restrict__ tasks) {
   __shared__ float2 ktaps[TX * (PATH == 0 ? 1 : ktap_slots<L>())];
   const int2 tk = tasks[blockIdx.x];
   zfused_fft_body<L, TX, PATH>(args[tk.x], tk.y, lds, ktaps);
+}
+
+// the fused z pass of an extended image; PATH 0 and 1 as above
+template <int L, int TX, int PATH>
+__global__ void __launch_bounds__(TX * threads_per_transform<L>())
+sk_zfused_ext(ZExtArgs b) {
+  using ZT = ZTile<L, TX>;
+  __shared__ float2 lds[L * TX];
+  __shared__ float2 ktaps[TX * (PATH == 0 ? 1 : ktap_slots<L>())];
+  const ZArgs& a = b.z;
+  const int c = threadIdx.x % TX, t = threadIdx.x / TX;
+  const ZT tile(a, blockIdx.x, c);
+  float2 v[ZT::MAXE];
+  tile.load_ext(a, b.ext, t, v);
+  if constexpr (PATH == 1) {
+    zfused_sparse_body<L, TX, true>(a, tile, t, c, v, lds, ktaps, b.ext.n);
+  } else {
+    (void)ktaps;
+    auto addr = [&](int pos) { return pos * TX + c; };
+    float2 w[ZT::MAXE];
+    tile.load_kernel(a, t, w);
+    sfft_run<L, false, -1>(v, t, lds, addr, a.fft.stw);
+    sfft_run<L, false, -1>(w, t, lds, addr, a.fft.stw);
+    zproduct<L>(v, w, t, a.conj != 0, a.scale);
+    sfft_run<L, true, +1>(v, t, lds, addr, a.fft.stw);
+    tile.store_below(a, b.ext.n, t, v);
+  }
 }
 
 template <int L, int TX>
@@ -1143,6 +1417,50 @@ bool sk_launch_zfused_fft(const ZArgs& a, long ny, hipStream_t st) {
   return true;
 }
 
+// launchers over an extended image
+template <int L>
+void sk_launch_xfwd_ext(const XExtArgs& a, hipStream_t st) {
+  constexpr int P = flat_pairs<L, 256>();
+  XExtArgs b = a;
+  b.groups = (a.ny + 2 * P - 1) / (2 * P);
+  b.k_blocks = ((a.k.nrows + 1) / 2 + P - 1) / P;
+  hipLaunchKernelGGL((sk_xfwd_ext<L, P>), dim3((unsigned)(b.groups * a.nplanes + b.k_blocks)),
+                     dim3(P * threads_per_transform<L>()), 0, st, b);
+}
+template <int L>
+void sk_launch_xinv_ext(const XExtArgs& a, hipStream_t st) {
+  constexpr int P = flat_pairs<L, 256>();
+  XExtArgs b = a;
+  b.groups = (a.ny + 2 * P - 1) / (2 * P);
+  hipLaunchKernelGGL((sk_xinv_ext<L, P>), dim3((unsigned)(b.groups * a.nplanes)),
+                     dim3(P * threads_per_transform<L>()), 0, st, b);
+}
+template <int L>
+void sk_launch_col_ext(const ColExtArgs& a, int dir, hipStream_t st) {
+  constexpr int TX = fit_tile<L, 16>();
+  ColExtArgs b = a;
+  b.c = col2_tiles<L, TX>(a.c);
+  const dim3 grid((unsigned)b.c.ntiles), block(TX * threads_per_transform<L>());
+  if (dir < 0)
+    hipLaunchKernelGGL((sk_col_ext<L, TX, -1>), grid, block, 0, st, b);
+  else
+    hipLaunchKernelGGL((sk_col_ext<L, TX, +1>), grid, block, 0, st, b);
+}
+template <int L>
+void sk_launch_zfused_ext(const ZExtArgs& a, long ny, hipStream_t st) {
+  constexpr int TX = fit_tile<L, 16>();
+  ZExtArgs b = a;
+  b.z.ny = ny;
+  const dim3 grid((unsigned)column_tiles(a.z.nbins, TX, ny)), block(TX * threads_per_transform<L>());
+  if constexpr (PlanOf<L, false>::S == 2) {
+    if (zfused_sparse_ok<L>(a.z.nvalid)) {
+      hipLaunchKernelGGL((sk_zfused_ext<L, TX, 1>), grid, block, 0, st, b);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0>), grid, block, 0, st, b);
+}
+
 // direct kernel DFT costs kz complex MACs per output; use it while that is
 // cheaper than a transform of the mostly-zero kernel column
 template <int L>
@@ -1235,6 +1553,10 @@ StaticEntry make_static_entry() {
   if (L < 128 || L % 4 != 0) e.selected[kSxFwd] = index_of(e.xfwd, "w256-flat");
   e.xfwd_vpad = &sk_launch_xfwd_vpad<L, 64>;
   e.xinv_crop = &sk_launch_xinv_crop_flat<L, 256>;  // 171 vs 193 us at 600 x 600 x 288
+  e.ext.xfwd = &sk_launch_xfwd_ext<L>;
+  e.ext.xinv = &sk_launch_xinv_ext<L>;
+  e.ext.col = &sk_launch_col_ext<L>;
+  e.ext.zfused = &sk_launch_zfused_ext<L>;
   e.batch.pairs = batch_pairs<L>();
   e.batch.tx = fit_tile<L, 16>();
   e.batch.xfwd = &sb_launch_xfwd<L>;

@@ -20,6 +20,14 @@ using XFwdFn = bool (*)(const XPass2&, hipStream_t);
 using XInvFn = bool (*)(const XPassArgs&, hipStream_t);
 using ColFn = bool (*)(const Col2&, int dir, hipStream_t);
 using ZFn = bool (*)(const ZArgs&, long ny, hipStream_t);
+// passes over an extended image (AxisExt in kernels.hpp); `L` is the length
+// the entry serves
+struct StaticExt {
+  void (*xfwd)(const XExtArgs&, hipStream_t) = nullptr;
+  void (*xinv)(const XExtArgs&, hipStream_t) = nullptr;
+  void (*col)(const ColExtArgs&, int dir, hipStream_t) = nullptr;
+  void (*zfused)(const ZExtArgs&, long ny, hipStream_t) = nullptr;
+};
 
 template <class F>
 struct Variant {
@@ -57,6 +65,7 @@ struct StaticEntry {
   XFwdFn xfwd_vpad = nullptr;  // x forward over a virtually padded image
   XInvFn xinv_crop = nullptr;  // x inverse writing the cropped interior
   int selected[kSNumPasses] = {0, 0, 0, 0, 0};
+  StaticExt ext;
   StaticBatch batch;
   StaticRL rl;
   int count(int pass) const {
@@ -85,6 +94,11 @@ void static_register(int L, const StaticEntry& e);
 // Entry for length L (nullptr when none or when compile-time kernels are
 // switched off).  The pointer stays valid for the life of the process.
 StaticEntry* static_lookup(int L);
+// The same whether or not they are switched off: a shape that was given
+// extended transform lengths (ConvShape::px) has no other kernels.
+StaticEntry* static_entry(int L);
+// smallest registered length >= n that has no prime factor above 7 (0: none)
+int static_length_at_least(int n);
 
 // Persistent-grid size for a kernel: resident workgroups per CU x CUs.
 int persistent_blocks(const void* kernel, int threads);
