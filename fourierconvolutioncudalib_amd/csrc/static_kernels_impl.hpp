@@ -30,14 +30,29 @@ constexpr int threads_per_transform() {
   return PlanOf<L, false>::T;
 }
 
-// largest tile <= want that keeps a workgroup within 1024 threads and
-// 64 KiB of LDS
-template <int L, int WANT>
+// Largest tile <= want that keeps a workgroup within 1024 threads and its LDS
+// (L rows of the tile).  A 16-bin tile is a 128-byte line per row and takes
+// up to CAP bytes; 8-bin tiles move half lines and reach 3.0-4.1 TB/s in a
+// bare copy where 16-bin tiles reach 5.1-6.4 (384 x 384 x 192 to 512 x 512 x
+// 256).  Two workgroups per CU (80 KiB each) always pay: y passes over L x 512
+// x 64 volumes 42.8 -> 33.9 us at L = 540, 46.3 -> 43.6 at 600, the z pass at
+// 640 180 -> 126 us.  One workgroup per CU still pays in the y passes up to
+// 768 (60.6 -> 57.9 and 56.9 -> 50.2 us), not beyond (1024: 85 -> 90 us
+// forward), and never in the z pass (720: 132 -> 138 us, 960: 180 -> 201 us).
+constexpr int kTileLds = 65536, kTileLdsZ = 81920, kTileLdsCol = 98304;
+template <int L, int WANT, int CAP = kTileLds>
 constexpr int fit_tile() {
   int tx = WANT;
-  while (tx > 1 && (tx * threads_per_transform<L>() > 1024 || (long)tx * L * 8 > 65536)) tx /= 2;
+  while (tx > 1 && (tx * threads_per_transform<L>() > 1024 ||
+                    (long)tx * L * 8 > (tx == 16 ? CAP : kTileLds)))
+    tx /= 2;
   return tx;
 }
+// tiles of the column (y) and z passes
+template <int L, int WANT>
+constexpr int col_fit() { return fit_tile<L, WANT, WANT == 16 ? kTileLdsCol : kTileLds>(); }
+template <int L, int WANT>
+constexpr int z_fit() { return fit_tile<L, WANT, WANT == 16 ? kTileLdsZ : kTileLds>(); }
 
 // row pairs per x-pass workgroup for about TGT threads (T threads per row
 // pair), within the LDS and thread limits of fit_pairs
@@ -1375,7 +1390,7 @@ Col2 col2_tiles(const Col2& a) {
 template <int L, int WANT, bool REV = false>
 bool sk_launch_col(const Col2& a, int dir, hipStream_t st) {
   if (REV && PlanOf<L, false>::S < 2) return false;  // one stage: same as forward order
-  constexpr int TX = fit_tile<L, WANT>();
+  constexpr int TX = col_fit<L, WANT>();
   const Col2 b = col2_tiles<L, TX>(a);
   const dim3 block(TX * threads_per_transform<L>());
   if (dir < 0)
@@ -1387,7 +1402,7 @@ bool sk_launch_col(const Col2& a, int dir, hipStream_t st) {
 
 template <int L, int WANT>
 bool sk_launch_col_pipe(const Col2& a, int dir, hipStream_t st) {
-  constexpr int TX = fit_tile<L, WANT>();
+  constexpr int TX = col_fit<L, WANT>();
   constexpr int threads = TX * threads_per_transform<L>();
   const Col2 b = col2_tiles<L, TX>(a);
   const void* fn = dir < 0 ? (const void*)sk_col_pipe<L, TX, -1> : (const void*)sk_col_pipe<L, TX, +1>;
@@ -1403,7 +1418,7 @@ bool sk_launch_col_pipe(const Col2& a, int dir, hipStream_t st) {
 
 template <int L, int WANT>
 bool sk_launch_zfused_fft(const ZArgs& a, long ny, hipStream_t st) {
-  constexpr int TX = fit_tile<L, WANT>();
+  constexpr int TX = z_fit<L, WANT>();
   ZArgs b = a;
   b.ny = ny;
   const dim3 grid((unsigned)column_tiles(a.nbins, TX, ny)), block(TX * threads_per_transform<L>());
@@ -1437,7 +1452,7 @@ void sk_launch_xinv_ext(const XExtArgs& a, hipStream_t st) {
 }
 template <int L>
 void sk_launch_col_ext(const ColExtArgs& a, int dir, hipStream_t st) {
-  constexpr int TX = fit_tile<L, 16>();
+  constexpr int TX = col_fit<L, 16>();
   ColExtArgs b = a;
   b.c = col2_tiles<L, TX>(a.c);
   const dim3 grid((unsigned)b.c.ntiles), block(TX * threads_per_transform<L>());
@@ -1448,7 +1463,7 @@ void sk_launch_col_ext(const ColExtArgs& a, int dir, hipStream_t st) {
 }
 template <int L>
 void sk_launch_zfused_ext(const ZExtArgs& a, long ny, hipStream_t st) {
-  constexpr int TX = fit_tile<L, 16>();
+  constexpr int TX = z_fit<L, 16>();
   ZExtArgs b = a;
   b.z.ny = ny;
   const dim3 grid((unsigned)column_tiles(a.z.nbins, TX, ny)), block(TX * threads_per_transform<L>());
@@ -1471,7 +1486,7 @@ constexpr int dft_kz_limit() {
 template <int L, int WANT>
 bool sk_launch_zfused_dft(const ZArgs& a, long ny, hipStream_t st) {
   if (a.nvalid > dft_kz_limit<L>()) return false;
-  constexpr int TX = fit_tile<L, WANT>();
+  constexpr int TX = z_fit<L, WANT>();
   ZArgs b = a;
   b.ny = ny;
   hipLaunchKernelGGL((sk_zfused_dft<L, TX>), dim3((unsigned)column_tiles(a.nbins, TX, ny)),
@@ -1529,13 +1544,13 @@ StaticEntry make_static_entry() {
             {"w256-ldsmirror", &sk_launch_xinv_lds<L, 256>},
             {"w256-flat", &sk_launch_xinv_flat<L, 256>},
             {"w128-flat", &sk_launch_xinv_flat<L, 128>}};
-  e.col = {{"t16", &sk_launch_col<L, 16>, fit_tile<L, 16>()},
+  e.col = {{"t16", &sk_launch_col<L, 16>, col_fit<L, 16>()},
            {"t16-pipe", &sk_launch_col_pipe<L, 16>},
            {"t8-pipe", &sk_launch_col_pipe<L, 8>},
            {"t16-revradix", &sk_launch_col<L, 16, true>},
-           {"t8", &sk_launch_col<L, 8>, fit_tile<L, 8>()},
-           {"t32", &sk_launch_col<L, 32>, fit_tile<L, 32>()},
-           {"t64", &sk_launch_col<L, 64>, fit_tile<L, 64>()}};
+           {"t8", &sk_launch_col<L, 8>, col_fit<L, 8>()},
+           {"t32", &sk_launch_col<L, 32>, col_fit<L, 32>()},
+           {"t64", &sk_launch_col<L, 64>, col_fit<L, 64>()}};
   e.zfused = {{"t16-fft", &sk_launch_zfused_fft<L, 16>},
               {"t16-dft", &sk_launch_zfused_dft<L, 16>},
               {"t8-fft", &sk_launch_zfused_fft<L, 8>},
