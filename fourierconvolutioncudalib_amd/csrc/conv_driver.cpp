@@ -60,20 +60,21 @@ std::vector<int> radix_plan(int L) {
 }
 
 int stage_table_segments(int L, TwSegment* seg, int* total) {
-  const StaticPlanData p = static_plan(L);
   *total = 0;
-  if (p.n <= 0) return 0;
   int n = 0;
-  for (int rev = 0; rev < 2; ++rev) {
-    int ns = 1;
-    for (int i = 0; i < p.n; ++i) {
-      const int r = rev ? p.r[p.n - 1 - i] : p.r[i];
-      if (n < kMaxTwSegments) seg[n] = TwSegment{*total, ns, r, even_up(r)};
-      ++n;
-      *total += ns * even_up(r);
-      ns *= r;
+  const StaticPlanData plans[2] = {static_plan(L), z_plan(L)};
+  if (plans[0].n <= 0) return 0;
+  for (const StaticPlanData& p : plans)
+    for (int rev = 0; rev < 2; ++rev) {
+      int ns = 1;
+      for (int i = 0; i < p.n; ++i) {
+        const int r = rev ? p.r[p.n - 1 - i] : p.r[i];
+        if (n < kMaxTwSegments) seg[n] = TwSegment{*total, ns, r, even_up(r)};
+        ++n;
+        *total += ns * even_up(r);
+        ns *= r;
+      }
     }
-  }
   return n;
 }
 

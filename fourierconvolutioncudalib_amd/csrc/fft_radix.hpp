@@ -34,6 +34,17 @@ __device__ __forceinline__ float2 twiddle(const float2* tw, int e) {
   return DIR < 0 ? w : cconj(w);
 }
 
+// a * exp(DIR * 2 pi i m / R) for the root (c, s) of a compile-time m: a
+// quarter turn is a swap (a product with its exact zeros would not fold)
+template <int R, int DIR>
+__device__ __forceinline__ float2 cmul_root(float2 a, int m, float c, float s) {
+  if (m == 0) return a;
+  if (4 * m == R) return rot90<DIR>(a);
+  if (2 * m == R) return make_float2(-a.x, -a.y);
+  if (4 * m == 3 * R) return rot90<-DIR>(a);
+  return cmul(a, make_float2(c, DIR * s));
+}
+
 namespace k {
 constexpr float kS3 = 0.86602540378443864676f;   // sin(2pi/3)
 constexpr float kC51 = 0.30901699437494742410f;  // cos(2pi/5)
@@ -137,12 +148,7 @@ struct Dft {
 #pragma unroll
       for (int k1 = 0; k1 < R1; ++k1) {
         const int m = (n2 * k1) % R;
-        if (m == 0) {
-          t[k1 * R2 + n2] = a[k1];
-        } else {
-          const float2 w = make_float2(W.c[m], DIR * W.s[m]);
-          t[k1 * R2 + n2] = cmul(a[k1], w);
-        }
+        t[k1 * R2 + n2] = cmul_root<R, DIR>(a[k1], m, W.c[m], W.s[m]);
       }
     }
 #pragma unroll
@@ -286,8 +292,7 @@ struct Dft<16, DIR> {
     const float sn[8] = {0.f, s1, k::kR2, c1, 1.f, c1, k::kR2, s1};
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      float2 w = make_float2(cs[j], DIR * sn[j]);
-      float2 t = cmul(o[j], w);
+      const float2 t = cmul_root<16, DIR>(o[j], j, cs[j], sn[j]);
       v[j] = cadd(e[j], t);
       v[j + 8] = csub(e[j], t);
     }

@@ -157,8 +157,52 @@ constexpr StaticPlanData static_plan(int L) {
   return uses_composite_plan(L) ? composite_plan(L) : classic_plan(L);
 }
 
+// Plan of the fused z pass where it differs: two stages of radices up to 25
+// (18 * 16 for 288, 24 * 16 for 384) where the plan above needs three.  The z
+// pass runs up to three transforms per tile and each of their exchanges holds
+// two barriers, so two stages instead of three halve them; the x and y passes
+// keep the plan above (radices above 16 measured 10-27 % slower there).  The
+// z pass over 512 x 128 x L volumes, 9 and 41 taps: L = 216 51 -> 33 and 51
+// -> 34 us, 300 65 -> 48 and 68 -> 51, 336 111 -> 50 and 112 -> 51, 384 72 ->
+// 52 and 73 -> 55, 400 112 -> 60 and 114 -> 64.  Beyond 432 (91 -> 86) the
+// radices leave too few waves: 480 75 -> 85, 576 95 -> 93 and 96 -> 98.
+// n = 0: the plan above.
+constexpr StaticPlanData z_plan(int L) {
+  StaticPlanData p{};
+  if (static_plan(L).n < 3 || L > 432) return p;
+  for (int r0 = 8; r0 <= 25; ++r0) {
+    const int r1 = L / r0;
+    if (r1 * r0 != L || r1 > r0 || r1 < 8) continue;
+    // radices whose butterflies exist: products of 2, 3, 5 and 7
+    int m = L;
+    for (int f : {2, 3, 5, 7})
+      while (m % f == 0) m /= f;
+    if (m != 1) continue;
+    p.n = 2;
+    p.r[0] = r0;
+    p.r[1] = r1;
+    p.t = r0;  // one butterfly per thread in either stage
+    return p;
+  }
+  return p;
+}
+// Plan identifiers of PlanOf and the sfft_* functions: a length L, or
+// L | kZPlan for its z plan.
+constexpr int kZPlan = 1 << 20;
+template <int L>
+constexpr int z_id() { return z_plan(L).n > 0 ? (L | kZPlan) : L; }
+// The same for the z kernels that transform the kernel's column like the
+// image's: 18 * 15 (270), whose 15-point butterflies cost as much as the 18
+// ones, pays with the tap path's two transforms (44 -> 39 us) and not with
+// three (44 -> 48).
+template <int L>
+constexpr int z_full_id() {
+  constexpr StaticPlanData p = z_plan(L);
+  return p.n > 0 && !(p.r[0] == 18 && p.r[1] == 15) ? (L | kZPlan) : L;
+}
+
 // Per-stage twiddle tables of a static plan, stored for the forward stage
-// order and then for the reversed order: stage s holds Ns(s) rows of
+// order and then for the reversed order (then the same for the z plan): stage s holds Ns(s) rows of
 // even(R) float2, row k = exp(-2 pi i r k / (Ns R)) for r = 0..R-1, so a
 // thread fetches its butterfly's twiddles with R/2 aligned 16-byte loads.
 constexpr int even_up(int r) { return (r + 1) / 2 * 2; }
@@ -179,9 +223,11 @@ constexpr int plan_rmax(const StaticPlanData& p) {
   return m;
 }
 
-template <int L, bool REV>
+template <int ID, bool REV>
 struct PlanOf {
-  static constexpr StaticPlanData data = static_plan(L);
+  static constexpr int L = ID & (kZPlan - 1);
+  static constexpr bool Z = (ID & kZPlan) != 0;
+  static constexpr StaticPlanData data = Z ? z_plan(L) : static_plan(L);
   static_assert(data.n > 0, "length without a static plan");
   static constexpr int S = data.n;
   static constexpr int RMAX = plan_rmax(data);
@@ -200,9 +246,13 @@ struct PlanOf {
     for (int s = 0; s < S; ++s) m = E(s) > m ? E(s) : m;
     return m;
   }
-  // offset (float2 units) of stage s's table in the combined table
+  // offset (float2 units) of stage s's table in the combined table (a constant
+  // of its own: the plan search must not be left to run time)
+  static constexpr int TWBASE =
+      (Z ? static_tw_size(static_plan(L), false) + static_tw_size(static_plan(L), true) : 0) +
+      (REV ? static_tw_size(data, false) : 0);
   static constexpr int TWOFF(int s) {
-    int off = REV ? static_tw_size(data, false) : 0;
+    int off = TWBASE;
     for (int i = 0; i < s; ++i) off += Ns(i) * even_up(R(i));
     return off;
   }
@@ -306,8 +356,8 @@ __device__ __forceinline__ void sfft_for_outputs(int t, F f) {
 // Stage s twiddle rows of the thread's butterflies, loaded ahead of use.
 // Stages of radix 8 and above keep bases instead of the row's R - 1
 // entries: W^k, W^2k, W^3k (q[0].xy, q[0].zw, q[1].xy), W^4k (q[1].zw) and,
-// from radix 9, W^8k and W^12k (q[2]); entry r = r1 + 4*r2 is
-// W^(r1 k) * W^(4 r2 k).  That is one product more for the entries with
+// from radix 9, W^8k, W^12k (q[2]), from radix 17 W^16k, W^20k (q[3]) and
+// from radix 25 W^24k (q[4]); entry r = r1 + 4*r2 is W^(r1 k) * W^(4 r2 k).  That is one product more for the entries with
 // r1, r2 > 0, but fewer loads and registers (12 instead of 32 at radix 16):
 // one stage's twiddles are live beside the image's and the kernel column's
 // values at the fused z pass's register peak, and their loads sit between
@@ -317,7 +367,7 @@ template <int L, bool REV, int s, int CM = FC_TW_COMPACT_MIN>
 struct StageTw {
   using P = PlanOf<L, REV>;
   static constexpr int R = P::R(s), Ns = P::Ns(s), NB = P::NB(s), RP = even_up(R);
-  static constexpr int CB = R >= 9 && R >= CM ? 3 : (R >= CM ? 2 : 0);
+  static constexpr int CB = R < CM ? 0 : 2 + (R + 7) / 8 - 1;
   static constexpr bool COMPACT = FC_TW_COMPACT && CB > 0;
   // odd radices below that keep entries 1..R-1 only (the row's entry 0 is
   // 1 and its last is padding): radix 3 in one float4 instead of two
@@ -334,9 +384,9 @@ struct StageTw {
                         : r1 == 2 ? make_float2(b[0].z, b[0].w)
                                   : make_float2(b[1].x, b[1].y);
       float2 hi = make_float2(b[1].z, b[1].w);  // r2 == 1
-      if constexpr (CB == 3) {
-        if (r2 == 2) hi = make_float2(b[2].x, b[2].y);
-        if (r2 == 3) hi = make_float2(b[2].z, b[2].w);
+      if (r2 >= 2) {
+        const float4 h = b[r2 / 2 + 1];
+        hi = r2 % 2 ? make_float2(h.z, h.w) : make_float2(h.x, h.y);
       }
       if (r2 == 0) return lo;
       if (r1 == 0) return hi;
@@ -370,10 +420,11 @@ __device__ __forceinline__ void sfft_load_tw(StageTw<L, REV, s, CM>& tw, int t,
         const float4 e23 = *reinterpret_cast<const float4*>(row + 2);
         tw.q[i * W::QB + 0] = make_float4(e1.x, e1.y, e23.x, e23.y);
         tw.q[i * W::QB + 1] = make_float4(e23.z, e23.w, e4.x, e4.y);
-        if constexpr (W::CB == 3) {
-          const float2 e8 = row[8];
-          const float2 e12 = W::R > 12 ? row[12] : make_float2(1.f, 0.f);
-          tw.q[i * W::QB + 2] = make_float4(e8.x, e8.y, e12.x, e12.y);
+#pragma unroll
+        for (int m = 2; m < W::CB; ++m) {
+          const float2 ea = row[8 * m - 8];
+          const float2 eb = W::R > 8 * m - 4 ? row[8 * m - 4] : make_float2(1.f, 0.f);
+          tw.q[i * W::QB + m] = make_float4(ea.x, ea.y, eb.x, eb.y);
         }
       } else if constexpr (W::SHIFT) {
 #pragma unroll

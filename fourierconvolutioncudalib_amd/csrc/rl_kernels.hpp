@@ -382,7 +382,7 @@ sk_xupdate_flat(RLXArgs a) {
 
 template <int L>
 void rl_launch_zfan(const RLZArgs& a, long ny, hipStream_t st) {
-  constexpr int TX = z_fit<L, 16>();
+  constexpr int TX = fit_tile<L, 16, kTileLdsZ>();
   RLZArgs b = a;
   b.ny = ny;
   hipLaunchKernelGGL((sk_zfan<L, TX>), dim3((unsigned)column_tiles(a.nbins, TX, ny)),
@@ -391,7 +391,7 @@ void rl_launch_zfan(const RLZArgs& a, long ny, hipStream_t st) {
 
 template <int L>
 void rl_launch_zsum(const RLZArgs& a, long ny, hipStream_t st) {
-  constexpr int TX = z_fit<L, 16>();
+  constexpr int TX = fit_tile<L, 16, kTileLdsZ>();
   RLZArgs b = a;
   b.ny = ny;
   hipLaunchKernelGGL((sk_zsum<L, TX>), dim3((unsigned)column_tiles(a.nbins, TX, ny)),

@@ -30,6 +30,17 @@ constexpr int threads_per_transform() {
   return PlanOf<L, false>::T;
 }
 
+// plan identifier and threads per column of the fused z kernels (PATH 1: the
+// tap path)
+template <int L, int PATH>
+constexpr int zk_id() {
+  return PATH == 1 ? z_id<L>() : z_full_id<L>();
+}
+template <int L, int PATH>
+constexpr int z_threads() {
+  return PlanOf<zk_id<L, PATH>(), false>::T;
+}
+
 // Largest tile <= want that keeps a workgroup within 1024 threads and its LDS
 // (L rows of the tile).  A 16-bin tile is a 128-byte line per row and takes
 // up to CAP bytes; 8-bin tiles move half lines and reach 3.0-4.1 TB/s in a
@@ -40,10 +51,10 @@ constexpr int threads_per_transform() {
 // 768 (60.6 -> 57.9 and 56.9 -> 50.2 us), not beyond (1024: 85 -> 90 us
 // forward), and never in the z pass (720: 132 -> 138 us, 960: 180 -> 201 us).
 constexpr int kTileLds = 65536, kTileLdsZ = 81920, kTileLdsCol = 98304;
-template <int L, int WANT, int CAP = kTileLds>
+template <int L, int WANT, int CAP = kTileLds, int T = threads_per_transform<L>()>
 constexpr int fit_tile() {
   int tx = WANT;
-  while (tx > 1 && (tx * threads_per_transform<L>() > 1024 ||
+  while (tx > 1 && (tx * T > 1024 ||
                     (long)tx * L * 8 > (tx == 16 ? CAP : kTileLds)))
     tx /= 2;
   return tx;
@@ -52,7 +63,9 @@ constexpr int fit_tile() {
 template <int L, int WANT>
 constexpr int col_fit() { return fit_tile<L, WANT, WANT == 16 ? kTileLdsCol : kTileLds>(); }
 template <int L, int WANT>
-constexpr int z_fit() { return fit_tile<L, WANT, WANT == 16 ? kTileLdsZ : kTileLds>(); }
+constexpr int z_fit() {
+  return fit_tile<L, WANT, WANT == 16 ? kTileLdsZ : kTileLds, z_threads<L, 0>()>();
+}
 
 // row pairs per x-pass workgroup for about TGT threads (T threads per row
 // pair), within the LDS and thread limits of fit_pairs
@@ -971,7 +984,7 @@ __device__ __forceinline__ void kernel_spectrum_direct(float2 (&w)[MAXE], int t,
                                                        const float2* __restrict__ kcol, long kplane,
                                                        int kz, int cz,
                                                        const float2* __restrict__ tw) {
-  using P = PlanOf<L, false>;
+  using P = PlanOf<z_full_id<L>(), false>;
   constexpr int s = P::S - 1;
   constexpr int R = P::R(s), M = P::M(s), NB = P::NB(s);
 #pragma unroll
@@ -1011,9 +1024,60 @@ __device__ __forceinline__ void kernel_spectrum_direct(float2 (&w)[MAXE], int t,
   }
 }
 
-template <int L, int TX>
+// Stage-0 input slots of a kernel column, from either end, that a pruned
+// z kernel keeps: a quarter of the column (n = 1) or half of it (n = 2).
+template <int ID>
+constexpr int kernel_slots(int n) {
+  return n == 1 ? (PlanOf<ID, false>::R(0) + 7) / 8 : (PlanOf<ID, false>::R(0) + 3) / 4;
+}
+// which of the two holds nvalid taps centred at `center` (0: neither)
+template <int ID>
+inline int kernel_prune(int nvalid, int center) {
+  constexpr int M = PlanOf<ID, false>::M(0);
+  const int far = nvalid - center > center ? nvalid - center : center;
+  const int need = (far + M - 1) / M;
+  return need <= kernel_slots<ID>(1) ? 1 : need <= kernel_slots<ID>(2) ? 2 : 0;
+}
+
+// w <- the kernel column's taps at the thread's stage-0 positions (ID: plan
+// identifier of length L); H as in ZTile::load_kernel
+template <int ID, int H, int MAXE>
+__device__ __forceinline__ void load_kernel_taps(float2 (&w)[MAXE], int t, bool ok,
+                                                 const float2* kcol, long kp, int nvalid,
+                                                 int center) {
+  using P = PlanOf<ID, false>;
+  constexpr int L = P::L, R = P::R(0), M = P::M(0);
+  // tap j = pos + center (- L when it wraps): base at tap t + center
+  const float2* kt = kcol + (long)(t + center) * kp;
+  const float2* kw = kt - (long)L * kp;
+  if constexpr (H == 0) {
+    sfft_for_inputs<ID, false>(t, [&](int slot, int pos) {
+      const bool wrap = pos + center >= L;
+      const int j = wrap ? pos + center - L : pos + center;
+      float2 val = make_float2(0.f, 0.f);
+      if (ok && j < nvalid) val = (wrap ? kw : kt)[(long)(pos - t) * kp];
+      w[slot] = val;
+    });
+  } else {
+    static_assert(2 * H <= R, "pruned slots overlap");
+    const int jt = ok ? t + center : -(1 << 30);  // tap of position t, or none
+    sfft_for_inputs<ID, false>(t, [&](int slot, int pos) {
+      const int r = slot % R, d = slot / R * P::T + r * M;  // pos = t + d
+      float2 val = make_float2(0.f, 0.f);
+      if (r < H) {
+        const int j = jt + d;
+        if (j >= 0 && j < nvalid) val = kt[(long)d * kp];
+      } else if (r >= R - H) {
+        if (jt + d - L >= 0) val = kw[(long)d * kp];
+      }
+      w[slot] = val;
+    });
+  }
+}
+
+template <int L, int TX, int ID>
 struct ZTile {
-  using P = PlanOf<L, false>;
+  using P = PlanOf<ID, false>;
   static constexpr int MAXE = P::MAXE();
   float2* col;
   const float2* kcol;
@@ -1034,7 +1098,7 @@ struct ZTile {
     const long sp = a.s_plane;
     const bool okk = ok;
     const float2* ct = col + (long)t * sp;
-    sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
+    sfft_for_inputs<ID, false>(t, [&](int slot, int pos) {
       float2 val = make_float2(0.f, 0.f);
       if (okk) val = ct[(long)(pos - t) * sp];
       v[slot] = val;
@@ -1048,7 +1112,7 @@ struct ZTile {
     const long sp = a.s_plane;
     if (SUBSET && a.out_planes > 0) {  // rotated subset (see ZArgs)
       const int sh = a.out_shift, np = a.out_planes;
-      sfft_for_outputs<L, true>(t, [&](int slot, int pos) {
+      sfft_for_outputs<ID, true>(t, [&](int slot, int pos) {
         int q = pos + sh;
         if (q >= L) q -= L;
         if (q < np) col[(long)q * sp] = v[slot];
@@ -1056,7 +1120,7 @@ struct ZTile {
       return;
     }
     float2* ct = col + (long)t * sp;
-    sfft_for_outputs<L, true>(t, [&](int slot, int pos) { ct[(long)(pos - t) * sp] = v[slot]; });
+    sfft_for_outputs<ID, true>(t, [&](int slot, int pos) { ct[(long)(pos - t) * sp] = v[slot]; });
   }
   // extended columns (AxisExt): planes mapped past the image's ends on the
   // way in, only the image's own planes written
@@ -1065,7 +1129,7 @@ struct ZTile {
     const float2* ct = col + (long)t * sp;
     const float2* c0 = col;
     const bool okk = ok;
-    sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
+    sfft_for_inputs<ID, false>(t, [&](int slot, int pos) {
       float2 val = make_float2(0.f, 0.f);
       if (okk) {
         if (pos < e.n) {
@@ -1082,46 +1146,39 @@ struct ZTile {
     if (!ok) return;
     const long sp = a.s_plane;
     float2* ct = col + (long)t * sp;
-    sfft_for_outputs<L, true>(t, [&](int slot, int pos) {
+    sfft_for_outputs<ID, true>(t, [&](int slot, int pos) {
       if (pos < n) ct[(long)(pos - t) * sp] = v[slot];
     });
   }
-  // kernel column: taps j < nvalid placed circularly at (j - center) mod L
+  // Kernel column: taps j < nvalid placed circularly at (j - center) mod L.
+  // H > 0: the taps lie within the first and the last H stage-0 input slots
+  // of every thread (kernel_slots), and the other slots are the constant zero
+  // that the stage-0 butterfly folds away.
+  template <int H>
   __device__ void load_kernel(const ZArgs& a, int t, float2 (&w)[MAXE]) const {
-    const long kp = a.k_plane;
-    const int center = a.center, nvalid = a.nvalid;
-    const bool okk = ok;
-    // tap j = pos + center (- L when it wraps): base at tap t + center
-    const float2* kt = kcol + (long)(t + center) * kp;
-    const float2* kw = kt - (long)L * kp;
-    sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
-      const bool wrap = pos + center >= L;
-      const int j = wrap ? pos + center - L : pos + center;
-      float2 val = make_float2(0.f, 0.f);
-      if (okk && j < nvalid) val = (wrap ? kw : kt)[(long)(pos - t) * kp];
-      w[slot] = val;
-    });
+    load_kernel_taps<ID, H>(w, t, ok, kcol, a.k_plane, a.nvalid, a.center);
   }
 };
 
 // product of the forward image spectrum (v) with the kernel spectrum (w),
 // conjugated for correlation, times the scale: v * (sc*w.x, +-sc*w.y)
-template <int L, int MAXE>
+// (ID: the plan identifier of both, see PlanOf)
+template <int ID, int MAXE>
 __device__ __forceinline__ void zproduct(float2 (&v)[MAXE], const float2 (&w)[MAXE], int t,
                                          bool cj, float sc) {
   const float si = cj ? -sc : sc;
-  sfft_for_outputs<L, false>(t, [&](int slot, int) {
+  sfft_for_outputs<ID, false>(t, [&](int slot, int) {
     v[slot] = cmul(v[slot], make_float2(sc * w[slot].x, si * w[slot].y));
   });
 }
 
 // the same product with the scale already in w (the tap path scales its
 // taps once as it loads them): v * (w.x, +-w.y)
-template <int L, int MAXE>
+template <int ID, int MAXE>
 __device__ __forceinline__ void zproduct_prescaled(float2 (&v)[MAXE], const float2 (&w)[MAXE], int t,
                                                    bool cj) {
   const float si = cj ? -1.f : 1.f;
-  sfft_for_outputs<L, false>(t, [&](int slot, int) {
+  sfft_for_outputs<ID, false>(t, [&](int slot, int) {
     v[slot] = cmul(v[slot], make_float2(w[slot].x, si * w[slot].y));
   });
 }
@@ -1129,7 +1186,7 @@ __device__ __forceinline__ void zproduct_prescaled(float2 (&v)[MAXE], const floa
 // taps per column the two-stage fast path can hold (its stage-1 radix)
 template <int L>
 constexpr int ktap_slots() {
-  return PlanOf<L, false>::S == 2 ? PlanOf<L, false>::R(1) : 1;
+  return PlanOf<z_id<L>(), false>::S == 2 ? PlanOf<z_id<L>(), false>::R(1) : 1;
 }
 
 // Two-stage plan (L = R0*R1) with the kz taps within one stage-0 stride
@@ -1145,12 +1202,12 @@ constexpr int ktap_slots() {
 // per-slot predicated loads and one LDS exchange (two per tile remain).
 // (`keep`: positions written, L or the planes of an extended image)
 template <int L, int TX, bool EXT = false>
-__device__ __forceinline__ void zfused_sparse_body(const ZArgs& a, const ZTile<L, TX>& tile, int t,
-                                                   int c, float2 (&v)[ZTile<L, TX>::MAXE],
+__device__ __forceinline__ void zfused_sparse_body(const ZArgs& a, const ZTile<L, TX, z_id<L>()>& tile, int t,
+                                                   int c, float2 (&v)[ZTile<L, TX, z_id<L>()>::MAXE],
                                                    float2* lds, float2* ktaps, int keep = L) {
-  using P = PlanOf<L, false>;
+  using P = PlanOf<z_id<L>(), false>;
   constexpr int R1 = P::R(1), M1 = P::M(1), NB1 = P::NB(1), T = P::T;
-  constexpr int MAXE = ZTile<L, TX>::MAXE;
+  constexpr int MAXE = ZTile<L, TX, z_id<L>()>::MAXE;
   auto addr = [&](int pos) { return pos * TX + c; };
   const int center = a.center, nvalid = a.nvalid;
   for (int j = t; j < nvalid; j += T)
@@ -1163,17 +1220,17 @@ __device__ __forceinline__ void zfused_sparse_body(const ZArgs& a, const ZTile<L
     e[i] = (M1 % T) != 0 && b >= M1 ? make_float2(1.f, 0.f) : cconj(a.fft.tw[b * R1]);
   }
   // image: stage 0 and its exchange; the barrier also publishes the taps
-  sfft_compute<L, false, -1, 0>(v, t, a.fft.stw);
-  sfft_store_lds<L, false, 0>(v, t, lds, addr);
-  StageTw<L, false, 1> tw1;
-  sfft_load_tw<L, false, 1>(tw1, t, a.fft.stw);
+  sfft_compute<z_id<L>(), false, -1, 0>(v, t, a.fft.stw);
+  sfft_store_lds<z_id<L>(), false, 0>(v, t, lds, addr);
+  StageTw<z_id<L>(), false, 1> tw1;
+  sfft_load_tw<z_id<L>(), false, 1>(tw1, t, a.fft.stw);
   __syncthreads();
-  sfft_load_lds<L, false, 1>(v, t, lds, addr);
+  sfft_load_lds<z_id<L>(), false, 1>(v, t, lds, addr);
   // every thread is done with the exchange tile before the inverse reuses it
   // (the taps live in their own array)
   __syncthreads();
-  sfft_twiddle<L, false, -1, 1>(v, t, tw1);
-  sfft_butterflies<L, false, -1, 1>(v, t);
+  sfft_twiddle<z_id<L>(), false, -1, 1>(v, t, tw1);
+  sfft_butterflies<z_id<L>(), false, -1, 1>(v, t);
   // the kernel column's stage-1 inputs, built only now to keep them out of
   // the image transform's register peak; same butterflies, same twiddles
   float2 w[MAXE];
@@ -1190,10 +1247,10 @@ __device__ __forceinline__ void zfused_sparse_body(const ZArgs& a, const ZTile<L
       w[i * R1 + r] = val;
     }
   }
-  sfft_twiddle<L, false, -1, 1>(w, t, tw1);
-  sfft_butterflies<L, false, -1, 1>(w, t);
-  zproduct_prescaled<L>(v, w, t, a.conj != 0);
-  sfft_run<L, true, +1>(v, t, lds, addr, a.fft.stw);
+  sfft_twiddle<z_id<L>(), false, -1, 1>(w, t, tw1);
+  sfft_butterflies<z_id<L>(), false, -1, 1>(w, t);
+  zproduct_prescaled<z_id<L>()>(v, w, t, a.conj != 0);
+  sfft_run<z_id<L>(), true, +1>(v, t, lds, addr, a.fft.stw);
   if constexpr (EXT)
     tile.store_below(a, keep, t, v);
   else
@@ -1203,100 +1260,91 @@ __device__ __forceinline__ void zfused_sparse_body(const ZArgs& a, const ZTile<L
 // whether the two-stage tap path applies to this launch
 template <int L>
 __host__ __device__ constexpr bool zfused_sparse_ok(int nvalid) {
-  return PlanOf<L, false>::S == 2 && nvalid <= PlanOf<L, false>::R(1);
+  return PlanOf<z_id<L>(), false>::S == 2 && nvalid <= PlanOf<z_id<L>(), false>::R(1);
 }
 
 // Fused z pass of one tile.  PATH 0: kernel column transformed like the
-// image's; 1: the two-stage tap path (caller guarantees zfused_sparse_ok);
-// 2: chosen per tile at run time (batched task lists mix kernels).  Paths 0
-// and 1 are separate instantiations: compiled into one kernel their register
-// peaks add up (~144 against ~105 VGPRs each).
-template <int L, int TX, int PATH>
-__device__ __forceinline__ void zfused_fft_body(const ZArgs& a, long tile_index, float2* lds,
-                                                float2* ktaps) {
-  using ZT = ZTile<L, TX>;
+// image's, its taps in the first and last H stage-0 slots (H = 0: anywhere);
+// 1: the two-stage tap path (caller guarantees zfused_sparse_ok).  Separate
+// instantiations: compiled into one kernel their register peaks add up (~144
+// against ~105 VGPRs each).  EXT: columns of an extended image.
+template <int L, int TX, int PATH, int H = 0, bool EXT = false>
+__device__ __forceinline__ void zfused_body(const ZArgs& a, const AxisExt* ext, long tile_index,
+                                            float2* lds, float2* ktaps) {
+  constexpr int ID = zk_id<L, PATH>();
+  using ZT = ZTile<L, TX, ID>;
   const int c = threadIdx.x % TX, t = threadIdx.x / TX;
   const ZT tile(a, tile_index, c);
   auto addr = [&](int pos) { return pos * TX + c; };
   float2 v[ZT::MAXE];
-  tile.load(a, t, v);
-  if constexpr (PlanOf<L, false>::S == 2 && PATH != 0) {
-    if (PATH == 1 || a.nvalid <= PlanOf<L, false>::R(1)) {
-      zfused_sparse_body<L, TX>(a, tile, t, c, v, lds, ktaps);
-      return;
-    }
+  if constexpr (EXT)
+    tile.load_ext(a, *ext, t, v);
+  else
+    tile.load(a, t, v);
+  if constexpr (PATH == 1) {
+    zfused_sparse_body<L, TX, EXT>(a, tile, t, c, v, lds, ktaps, EXT ? ext->n : L);
+  } else {
+    (void)ktaps;
+    float2 w[ZT::MAXE];
+    // a whole kernel column of a z plan is loaded after the image's transform
+    // to stay out of its registers
+    constexpr bool kLate = PlanOf<ID, false>::Z && H == 0;
+    if (!kLate) tile.template load_kernel<H>(a, t, w);
+    // every sfft_run ends with a barrier after its last LDS read, so the
+    // next transform may reuse the tile
+    sfft_run<ID, false, -1>(v, t, lds, addr, a.fft.stw);
+    if (kLate) tile.template load_kernel<H>(a, t, w);
+    sfft_run<ID, false, -1>(w, t, lds, addr, a.fft.stw);
+    zproduct<ID>(v, w, t, a.conj != 0, a.scale);
+    sfft_run<ID, true, +1>(v, t, lds, addr, a.fft.stw);
+    if constexpr (EXT)
+      tile.store_below(a, ext->n, t, v);
+    else
+      tile.template store<H == 0>(a, t, v);
   }
-  (void)ktaps;
-  float2 w[ZT::MAXE];
-  tile.load_kernel(a, t, w);
-  // every sfft_run ends with a barrier after its last LDS read, so the
-  // next transform may reuse the tile
-  sfft_run<L, false, -1>(v, t, lds, addr, a.fft.stw);
-  sfft_run<L, false, -1>(w, t, lds, addr, a.fft.stw);
-  zproduct<L>(v, w, t, a.conj != 0, a.scale);
-  sfft_run<L, true, +1>(v, t, lds, addr, a.fft.stw);
-  tile.template store<PATH == 0>(a, t, v);
 }
 
-template <int L, int TX, int PATH>
-__global__ void __launch_bounds__(TX * threads_per_transform<L>())
+template <int L, int TX, int PATH, int H = 0>
+__global__ void __launch_bounds__((TX * z_threads<L, PATH>()))
 sk_zfused_fft(ZArgs a) {
   __shared__ float2 lds[L * TX];
   __shared__ float2 ktaps[TX * (PATH == 0 ? 1 : ktap_slots<L>())];
-  zfused_fft_body<L, TX, PATH>(a, blockIdx.x, lds, ktaps);
+  zfused_body<L, TX, PATH, H>(a, nullptr, blockIdx.x, lds, ktaps);
 }
 
 template <int L, int TX, int PATH>
-__global__ void __launch_bounds__(TX * threads_per_transform<L>())
+__global__ void __launch_bounds__((TX * z_threads<L, PATH>()))
 sb_zfused(const ZArgs* __restrict__ args, const int2* __restrict__ tasks) {
   __shared__ float2 lds[L * TX];
   __shared__ float2 ktaps[TX * (PATH == 0 ? 1 : ktap_slots<L>())];
   const int2 tk = tasks[blockIdx.x];
-  zfused_fft_body<L, TX, PATH>(args[tk.x], tk.y, lds, ktaps);
+  zfused_body<L, TX, PATH>(args[tk.x], nullptr, tk.y, lds, ktaps);
 }
 
 // the fused z pass of an extended image; PATH 0 and 1 as above
-template <int L, int TX, int PATH>
-__global__ void __launch_bounds__(TX * threads_per_transform<L>())
+template <int L, int TX, int PATH, int H = 0>
+__global__ void __launch_bounds__((TX * z_threads<L, PATH>()))
 sk_zfused_ext(ZExtArgs b) {
-  using ZT = ZTile<L, TX>;
   __shared__ float2 lds[L * TX];
   __shared__ float2 ktaps[TX * (PATH == 0 ? 1 : ktap_slots<L>())];
-  const ZArgs& a = b.z;
-  const int c = threadIdx.x % TX, t = threadIdx.x / TX;
-  const ZT tile(a, blockIdx.x, c);
-  float2 v[ZT::MAXE];
-  tile.load_ext(a, b.ext, t, v);
-  if constexpr (PATH == 1) {
-    zfused_sparse_body<L, TX, true>(a, tile, t, c, v, lds, ktaps, b.ext.n);
-  } else {
-    (void)ktaps;
-    auto addr = [&](int pos) { return pos * TX + c; };
-    float2 w[ZT::MAXE];
-    tile.load_kernel(a, t, w);
-    sfft_run<L, false, -1>(v, t, lds, addr, a.fft.stw);
-    sfft_run<L, false, -1>(w, t, lds, addr, a.fft.stw);
-    zproduct<L>(v, w, t, a.conj != 0, a.scale);
-    sfft_run<L, true, +1>(v, t, lds, addr, a.fft.stw);
-    tile.store_below(a, b.ext.n, t, v);
-  }
+  zfused_body<L, TX, PATH, H, true>(b.z, &b.ext, blockIdx.x, lds, ktaps);
 }
 
 template <int L, int TX>
-__global__ void __launch_bounds__(TX * threads_per_transform<L>())
+__global__ void __launch_bounds__((TX * z_threads<L, 0>()))
 sk_zfused_dft(ZArgs a) {
-  using ZT = ZTile<L, TX>;
+  using ZT = ZTile<L, TX, z_full_id<L>()>;
   __shared__ float2 lds[L * TX];
   const int c = threadIdx.x % TX, t = threadIdx.x / TX;
   const ZT tile(a, blockIdx.x, c);
   auto addr = [&](int pos) { return pos * TX + c; };
   float2 v[ZT::MAXE];
   tile.load(a, t, v);
-  sfft_run<L, false, -1>(v, t, lds, addr, a.fft.stw);
+  sfft_run<z_full_id<L>(), false, -1>(v, t, lds, addr, a.fft.stw);
   float2 w[ZT::MAXE];
   kernel_spectrum_direct<L>(w, t, tile.ok, tile.kcol, a.k_plane, a.nvalid, a.center, a.fft.tw);
-  zproduct<L>(v, w, t, a.conj != 0, a.scale);
-  sfft_run<L, true, +1>(v, t, lds, addr, a.fft.stw);
+  zproduct<z_full_id<L>()>(v, w, t, a.conj != 0, a.scale);
+  sfft_run<z_full_id<L>(), true, +1>(v, t, lds, addr, a.fft.stw);
   tile.template store<false>(a, t, v);
 }
 
@@ -1421,10 +1469,22 @@ bool sk_launch_zfused_fft(const ZArgs& a, long ny, hipStream_t st) {
   constexpr int TX = z_fit<L, WANT>();
   ZArgs b = a;
   b.ny = ny;
-  const dim3 grid((unsigned)column_tiles(a.nbins, TX, ny)), block(TX * threads_per_transform<L>());
-  if constexpr (PlanOf<L, false>::S == 2) {
+  const dim3 grid((unsigned)column_tiles(a.nbins, TX, ny)), block(TX * z_threads<L, 0>());
+  if constexpr (PlanOf<z_id<L>(), false>::S == 2) {
     if (zfused_sparse_ok<L>(a.nvalid)) {
-      hipLaunchKernelGGL((sk_zfused_fft<L, TX, 1>), grid, block, 0, st, b);
+      hipLaunchKernelGGL((sk_zfused_fft<L, TX, 1>), grid, dim3(TX * z_threads<L, 1>()), 0, st, b);
+      return true;
+    }
+  }
+  if constexpr (WANT == 16) {
+    constexpr int ID = z_full_id<L>();
+    const int n = a.out_planes > 0 ? 0 : kernel_prune<ID>(a.nvalid, a.center);
+    if (n == 1) {
+      hipLaunchKernelGGL((sk_zfused_fft<L, TX, 0, kernel_slots<ID>(1)>), grid, block, 0, st, b);
+      return true;
+    }
+    if (n == 2) {
+      hipLaunchKernelGGL((sk_zfused_fft<L, TX, 0, kernel_slots<ID>(2)>), grid, block, 0, st, b);
       return true;
     }
   }
@@ -1466,14 +1526,21 @@ void sk_launch_zfused_ext(const ZExtArgs& a, long ny, hipStream_t st) {
   constexpr int TX = z_fit<L, 16>();
   ZExtArgs b = a;
   b.z.ny = ny;
-  const dim3 grid((unsigned)column_tiles(a.z.nbins, TX, ny)), block(TX * threads_per_transform<L>());
-  if constexpr (PlanOf<L, false>::S == 2) {
+  const dim3 grid((unsigned)column_tiles(a.z.nbins, TX, ny)), block(TX * z_threads<L, 0>());
+  if constexpr (PlanOf<z_id<L>(), false>::S == 2) {
     if (zfused_sparse_ok<L>(a.z.nvalid)) {
-      hipLaunchKernelGGL((sk_zfused_ext<L, TX, 1>), grid, block, 0, st, b);
+      hipLaunchKernelGGL((sk_zfused_ext<L, TX, 1>), grid, dim3(TX * z_threads<L, 1>()), 0, st, b);
       return;
     }
   }
-  hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0>), grid, block, 0, st, b);
+  constexpr int ID = z_full_id<L>();
+  const int n = kernel_prune<ID>(a.z.nvalid, a.z.center);
+  if (n == 1)
+    hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0, kernel_slots<ID>(1)>), grid, block, 0, st, b);
+  else if (n == 2)
+    hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0, kernel_slots<ID>(2)>), grid, block, 0, st, b);
+  else
+    hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0>), grid, block, 0, st, b);
 }
 
 // direct kernel DFT costs kz complex MACs per output; use it while that is
@@ -1490,7 +1557,7 @@ bool sk_launch_zfused_dft(const ZArgs& a, long ny, hipStream_t st) {
   ZArgs b = a;
   b.ny = ny;
   hipLaunchKernelGGL((sk_zfused_dft<L, TX>), dim3((unsigned)column_tiles(a.nbins, TX, ny)),
-                     dim3(TX * threads_per_transform<L>()), 0, st, b);
+                     dim3(TX * z_threads<L, 0>()), 0, st, b);
   return true;
 }
 
@@ -1520,14 +1587,14 @@ template <int L>
 void sb_launch_zfused(const ZArgs* args, const int2* tasks, int ntasks, hipStream_t st) {
   constexpr int TX = fit_tile<L, 16>();
   hipLaunchKernelGGL((sb_zfused<L, TX, 0>), dim3((unsigned)ntasks),
-                     dim3(TX * threads_per_transform<L>()), 0, st, args, tasks);
+                     dim3(TX * z_threads<L, 0>()), 0, st, args, tasks);
 }
 template <int L>
 void sb_launch_zfused_sparse(const ZArgs* args, const int2* tasks, int ntasks, hipStream_t st) {
   constexpr int TX = fit_tile<L, 16>();
-  if constexpr (PlanOf<L, false>::S == 2)
+  if constexpr (PlanOf<z_id<L>(), false>::S == 2)
     hipLaunchKernelGGL((sb_zfused<L, TX, 1>), dim3((unsigned)ntasks),
-                       dim3(TX * threads_per_transform<L>()), 0, st, args, tasks);
+                       dim3(TX * z_threads<L, 1>()), 0, st, args, tasks);
 }
 
 template <int L>
@@ -1578,9 +1645,9 @@ StaticEntry make_static_entry() {
   e.batch.xinv = &sb_launch_xinv<L>;
   e.batch.col = &sb_launch_col<L>;
   e.batch.zfused = &sb_launch_zfused<L>;
-  if constexpr (PlanOf<L, false>::S == 2) {
+  if constexpr (PlanOf<z_id<L>(), false>::S == 2) {
     e.batch.zfused_sparse = &sb_launch_zfused_sparse<L>;
-    e.batch.sparse_kz = PlanOf<L, false>::R(1);
+    e.batch.sparse_kz = PlanOf<z_id<L>(), false>::R(1);
   }
   return e;
 }
