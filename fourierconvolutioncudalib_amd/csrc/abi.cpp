@@ -548,7 +548,7 @@ int fcamd_convolve3d_boundary_host(float* im, const int* imDim, const float* ker
 long long fcamd_grad_kernel_workspace_bytes(const int* imDim, const int* kernelDim) {
   long long r = -1;
   (void)guarded([&] {
-    const ConvShape s = shape_from_any(imDim, kernelDim);
+    const ConvShape s = conv_shape(imDim, kernelDim);
     r = (long long)(needs_long_path(s) ? long_workspace_bytes(s) : grad_workspace_layout(s).total());
   });
   return r;
@@ -559,8 +559,10 @@ int fcamd_conv_grad_kernel_device(float* d_dkernel, const float* d_grad_out, con
                                   long long workspace_bytes, void* stream) {
   return guarded([&] {
     FC_REQUIRE(d_dkernel && d_grad_out && d_image, kInvalidArgument, "null device pointer");
-    ConvShape s = shape_from_any(imDim, kernelDim);
+    ConvShape s = conv_shape(imDim, kernelDim);
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (d_workspace && s.extended() && workspace_bytes < (long long)grad_workspace_layout(s).total())
+      s = direct_shape(s);
     const bool lng = needs_long_path(s);
     const size_t need = lng ? long_workspace_bytes(s) : grad_workspace_layout(s).total();
     auto run = [&](void* ws) {

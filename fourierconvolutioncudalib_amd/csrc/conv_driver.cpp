@@ -977,20 +977,87 @@ void run_convolution(const ConvShape& s, float* d_out, const float* d_image,
 }
 
 GradWorkspaceLayout grad_workspace_layout(const ConvShape& s) {
-  const size_t nxp = (size_t)padded_bins(s.nx);
+  const size_t nxp = (size_t)padded_bins(s.tx());
   GradWorkspaceLayout w;
-  w.spectrum = align256(sizeof(float2) * nxp * s.ny * s.nz);
+  w.spectrum = align256(sizeof(float2) * nxp * s.ty() * s.nz);
   w.corr = align256(sizeof(float) * (size_t)s.nx * s.ny * s.kz);  // the kz support planes
   return w;
 }
 
-void enqueue_grad_kernel(const ConvShape& s, float* d_dkernel, const float* d_grad_out,
+namespace {
+
+// the kernel's taps from the kz support planes of y-columns in G (plane j
+// holding z-plane (j - cz) mod nz of the correlation): the y inverse of those
+// planes, then each support row's C2R at the support positions only (no x
+// inverse pass, no real planes)
+// (the y pass over the kz support planes takes its own tile: the tuned
+// one fits full volumes.  At 256 x 256 x 128 with 21^3 the 16-bin tile
+// leaves 170 workgroups for 256 CUs, the 8-bin tile twice as many:
+// PSF gradient 89.1 -> 86.5 us)
+void gather_from_planes(const ConvShape& s, float2* G, const FftDesc& fx, float* d_dkernel,
+                        hipStream_t st) {
+  ConvShape sub = s;
+  sub.nz = s.kz;
+  const FftDesc fy = fft_desc(s.ny, st);
+  if (s.ny > 1) {
+    ensure_kernel_attributes();
+    PassScope ps(kPassYInverse, st);
+    if (!static_ycol_fill(sub, fy, G, +1, cu_count(), st))
+      launch_gk_col(spectrum_column_args(sub, fy, G), +1, sub.nz, st);
+  }
+  launch_gather_support_c2r(s, G, padded_bins(s.nx), fx.tw, d_dkernel, st);
+}
+
+// The PSF gradient of an extended shape: the correlation u[d] = sum_i g[i]
+// im[i - d] at the lags d the kernel covers needs the image's neighbours past
+// its ends (those of the convolution) and g itself only, so both volumes run
+// at the extended lengths, g with zeros there.
+void enqueue_grad_kernel_ext(const ConvShape& s, float* d_dkernel, const float* d_grad_out,
+                             const float* d_image, float2* G, float2* I, hipStream_t st) {
+  ConvShape gs = s;
+  for (int& m : gs.mode) m = kMapZero;
+  forward_xy(gs, d_grad_out, G, nullptr, nullptr, nullptr, st);
+  forward_xy(s, d_image, I, nullptr, nullptr, nullptr, st);
+  const long nxp = padded_bins(s.px);
+  ZArgs a{};
+  a.fft = fft_desc(s.pz, st);
+  a.nbins = half_bins(s.px);
+  a.s = G;
+  a.k = I;
+  a.s_row = a.k_row = nxp;
+  a.s_plane = a.k_plane = (long)s.py * nxp;
+  a.nvalid = s.pz;
+  a.conj = 1;
+  a.scale = (float)(1.0 / ((double)s.px * s.py * s.pz));
+  a.out_planes = s.kz;
+  a.out_shift = s.cz;
+  {
+    PassScope ps(kPassZFused, st);
+    static_zcorr_ext(s, a, axis_ext(gs, 2, Op::kConvolve), axis_ext(s, 2, Op::kConvolve), st);
+  }
+  ConvShape t = direct_shape(s);
+  t.nx = s.px;
+  t.ny = s.py;
+  t.nz = s.pz;
+  gather_from_planes(t, G, fft_desc(s.px, st), d_dkernel, st);
+}
+
+}  // namespace
+
+void enqueue_grad_kernel(const ConvShape& shape, float* d_dkernel, const float* d_grad_out,
                          const float* d_image, void* ws, hipStream_t st) {
+  const ConvShape s =
+      shape.extended() && !extension_tables(shape, st) ? direct_shape(shape) : shape;
   const GradWorkspaceLayout wl = grad_workspace_layout(s);
   char* base = static_cast<char*>(ws);
   float2* G = reinterpret_cast<float2*>(base);
   float2* I = reinterpret_cast<float2*>(base + wl.spectrum);
   float* U = reinterpret_cast<float*>(base + 2 * wl.spectrum);
+  if (s.extended()) {
+    enqueue_grad_kernel_ext(s, d_dkernel, d_grad_out, d_image, G, I, st);
+    FC_HIP_CHECK(hipGetLastError());
+    return;
+  }
   // u = IFFT(FFT(g) * conj(FFT(im))) / N, the circular cross-correlation
   // u[d] = sum_i g[i] im[i - d]; dk[j] = u[(j - c) mod n].  The image goes
   // through the x and y passes as their second operand (the slot the
@@ -1007,28 +1074,14 @@ void enqueue_grad_kernel(const ConvShape& s, float* d_dkernel, const float* d_gr
   // plane j: the support is the first kz planes, inverted (y and x act
   // within a plane) as a volume of its own; U holds kz planes.
   z_pass(s, G, I, true, true, st, s.kz, s.cz);
-  ConvShape sub = s;
-  sub.nz = s.kz;
   const FftDesc fx = fft_desc(s.nx, st);
   if (fx.M == 0 && gather_support_c2r_lds(s.nx) <= 65536) {
-    // the gather reads kx of each row's nx outputs on ky of its ny rows:
-    // the y inverse of the support planes, then each support row's C2R at
-    // the support positions only (no x inverse pass, no real planes)
-    // (the y pass over the kz support planes takes its own tile: the tuned
-    // one fits full volumes.  At 256 x 256 x 128 with 21^3 the 16-bin tile
-    // leaves 170 workgroups for 256 CUs, the 8-bin tile twice as many:
-    // PSF gradient 89.1 -> 86.5 us)
-    const FftDesc fy = fft_desc(s.ny, st);
-    if (s.ny > 1) {
-      ensure_kernel_attributes();
-      PassScope ps(kPassYInverse, st);
-      if (!static_ycol_fill(sub, fy, G, +1, cu_count(), st))
-        launch_gk_col(spectrum_column_args(sub, fy, G), +1, sub.nz, st);
-    }
-    launch_gather_support_c2r(s, G, padded_bins(s.nx), fx.tw, d_dkernel, st);
+    gather_from_planes(s, G, fx, d_dkernel, st);
   } else {
     // Bluestein x (its table is not the length-nx one the direct C2R reads)
     // or a row and table past 64 KiB of LDS
+    ConvShape sub = s;
+    sub.nz = s.kz;
     inverse_yx(sub, G, U, st);
     ConvShape g = sub;
     g.cz = 0;

@@ -261,6 +261,12 @@ struct ZExtArgs {
   ZArgs z;
   AxisExt ext;
 };
+// correlation of two extended volumes (the PSF gradient): z.s, extended by
+// ext, times the conjugate of z.k, extended by kext, into z's output planes
+struct ZCorrArgs {
+  ZArgs z;
+  AxisExt ext, kext;
+};
 
 // fused multiview Richardson-Lucy passes (rl_kernels.hpp)
 constexpr int kMaxViews = 8;

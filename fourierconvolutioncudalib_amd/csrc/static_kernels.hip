@@ -338,6 +338,20 @@ void static_zfused_ext(const ConvShape& s, const ZArgs& a, const AxisExt& ext, h
   e->ext.zfused(b, (long)s.py, st);
 }
 
+void static_zcorr_ext(const ConvShape& s, const ZArgs& a, const AxisExt& ext, const AxisExt& kext,
+                      hipStream_t st) {
+  StaticEntry* e = entry_of(s.pz);
+  if (s.pz == s.nz) {
+    run_selected(e->zfused, e->selected[kSZ], a, (long)s.py, st);
+    return;
+  }
+  ZCorrArgs b{};
+  b.z = a;
+  b.ext = ext;
+  b.kext = kext;
+  e->ext.zcorr(b, (long)s.py, st);
+}
+
 void static_kernels_allow_large_lds() {}
 
 }  // namespace fcamd

@@ -37,6 +37,9 @@ void static_xinv_ext(const ConvShape& s, const FftDesc& fx, const float2* S, flo
 void static_ycol_ext(const ConvShape& s, const FftDesc& fy, float2* S, int dir,
                      const float2* krows, float2* kplanes, Op op, hipStream_t st);
 void static_zfused_ext(const ConvShape& s, const ZArgs& a, const AxisExt& ext, hipStream_t st);
+// the z pass of the PSF gradient of an extended shape (ZCorrArgs)
+void static_zcorr_ext(const ConvShape& s, const ZArgs& a, const AxisExt& ext, const AxisExt& kext,
+                      hipStream_t st);
 void static_kernels_allow_large_lds();
 
 }  // namespace fcamd

@@ -1125,9 +1125,11 @@ struct ZTile {
   // extended columns (AxisExt): planes mapped past the image's ends on the
   // way in, only the image's own planes written
   __device__ void load_ext(const ZArgs& a, const AxisExt& e, int t, float2 (&v)[MAXE]) const {
-    const long sp = a.s_plane;
-    const float2* ct = col + (long)t * sp;
-    const float2* c0 = col;
+    load_mapped(col, a.s_plane, e, t, v);
+  }
+  __device__ void load_mapped(const float2* c0, long sp, const AxisExt& e, int t,
+                              float2 (&v)[MAXE]) const {
+    const float2* ct = c0 + (long)t * sp;
     const bool okk = ok;
     sfft_for_inputs<ID, false>(t, [&](int slot, int pos) {
       float2 val = make_float2(0.f, 0.f);
@@ -1135,12 +1137,15 @@ struct ZTile {
         if (pos < e.n) {
           val = ct[(long)(pos - t) * sp];
         } else {
-          const int q = axis_ext_src(e, L, pos);
+          const int q = axis_ext_src(e, P::L, pos);
           if (q >= 0) val = c0[(long)q * sp];
         }
       }
       v[slot] = val;
     });
+  }
+  __device__ void load_operand(const ZArgs& a, const AxisExt& e, int t, float2 (&w)[MAXE]) const {
+    load_mapped(kcol, a.k_plane, e, t, w);
   }
   __device__ void store_below(const ZArgs& a, int n, int t, const float2 (&v)[MAXE]) const {
     if (!ok) return;
@@ -1328,6 +1333,27 @@ sk_zfused_ext(ZExtArgs b) {
   __shared__ float2 lds[L * TX];
   __shared__ float2 ktaps[TX * (PATH == 0 ? 1 : ktap_slots<L>())];
   zfused_body<L, TX, PATH, H, true>(b.z, &b.ext, blockIdx.x, lds, ktaps);
+}
+
+// z pass of the PSF gradient over extended volumes
+template <int L, int TX>
+__global__ void __launch_bounds__((TX * z_threads<L, 0>()))
+sk_zcorr_ext(ZCorrArgs b) {
+  constexpr int ID = z_full_id<L>();
+  using ZT = ZTile<L, TX, ID>;
+  __shared__ float2 lds[L * TX];
+  const ZArgs& a = b.z;
+  const int c = threadIdx.x % TX, t = threadIdx.x / TX;
+  const ZT tile(a, blockIdx.x, c);
+  auto addr = [&](int pos) { return pos * TX + c; };
+  float2 v[ZT::MAXE], w[ZT::MAXE];
+  tile.load_ext(a, b.ext, t, v);
+  sfft_run<ID, false, -1>(v, t, lds, addr, a.fft.stw);
+  tile.load_operand(a, b.kext, t, w);
+  sfft_run<ID, false, -1>(w, t, lds, addr, a.fft.stw);
+  zproduct<ID>(v, w, t, true, a.scale);
+  sfft_run<ID, true, +1>(v, t, lds, addr, a.fft.stw);
+  tile.template store<true>(a, t, v);
 }
 
 template <int L, int TX>
@@ -1543,6 +1569,15 @@ void sk_launch_zfused_ext(const ZExtArgs& a, long ny, hipStream_t st) {
     hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0>), grid, block, 0, st, b);
 }
 
+template <int L>
+void sk_launch_zcorr_ext(const ZCorrArgs& a, long ny, hipStream_t st) {
+  constexpr int TX = z_fit<L, 16>();
+  ZCorrArgs b = a;
+  b.z.ny = ny;
+  hipLaunchKernelGGL((sk_zcorr_ext<L, TX>), dim3((unsigned)column_tiles(a.z.nbins, TX, ny)),
+                     dim3(TX * z_threads<L, 0>()), 0, st, b);
+}
+
 // direct kernel DFT costs kz complex MACs per output; use it while that is
 // cheaper than a transform of the mostly-zero kernel column
 template <int L>
@@ -1639,6 +1674,7 @@ StaticEntry make_static_entry() {
   e.ext.xinv = &sk_launch_xinv_ext<L>;
   e.ext.col = &sk_launch_col_ext<L>;
   e.ext.zfused = &sk_launch_zfused_ext<L>;
+  e.ext.zcorr = &sk_launch_zcorr_ext<L>;
   e.batch.pairs = batch_pairs<L>();
   e.batch.tx = fit_tile<L, 16>();
   e.batch.xfwd = &sb_launch_xfwd<L>;

@@ -27,6 +27,7 @@ struct StaticExt {
   void (*xinv)(const XExtArgs&, hipStream_t) = nullptr;
   void (*col)(const ColExtArgs&, int dir, hipStream_t) = nullptr;
   void (*zfused)(const ZExtArgs&, long ny, hipStream_t) = nullptr;
+  void (*zcorr)(const ZCorrArgs&, long ny, hipStream_t) = nullptr;
 };
 
 template <class F>

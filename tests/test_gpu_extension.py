@@ -81,3 +81,20 @@ def test_unextended_workspace_is_enough(fc, oracle):
                                            ws.data_ptr(), small, None))
     torch.cuda.synchronize()
     assert oracle.rel_l2(out.cpu().numpy(), oracle.numpy_fft_conv(a, k)) < TOL
+
+
+@pytest.mark.parametrize("shape,kshape", [((64, 64, 67), (5, 5, 9)), ((61, 51, 64), (61, 8, 5)),
+                                          ((61, 67, 71), (7, 4, 10)), ((37, 33, 47), (37, 33, 47)),
+                                          ((300, 33, 41), (31, 1, 2))])
+def test_extended_gradients(fc, oracle, shape, kshape):
+    """Both gradients of extended shapes through torch autograd."""
+    import torch
+    from fourierconvolutioncudalib_amd.autograd import fft_conv3d
+    a, k = _data(shape, kshape, 4700 + sum(shape))
+    g = np.random.default_rng(4701).standard_normal(shape).astype(np.float32)
+    ta = torch.from_numpy(a).cuda().requires_grad_(True)
+    tk = torch.from_numpy(k).cuda().requires_grad_(True)
+    print("gradients", shape, kshape, flush=True)
+    fft_conv3d(ta, tk).backward(torch.from_numpy(g).cuda())
+    assert oracle.rel_l2(ta.grad.cpu().numpy(), oracle.numpy_fft_conv(g, k, conj_kernel=True)) < TOL
+    assert oracle.rel_l2(tk.grad.cpu().numpy(), oracle.fft_conv_grad_kernel(g, a, kshape)) < TOL
