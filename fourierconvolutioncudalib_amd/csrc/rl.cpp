@@ -198,13 +198,22 @@ void run_rl(const RLProblem& p, float* psi, const float* const* views, const flo
   xa.psi = psi;
   RLXArgs ua = xa;
   ua.spec[0] = Spsi;
+  // The views' spectra follow one another, so their y passes are one launch
+  // over V * nz planes where no alignment gap parts them: a launch per view
+  // ends in a partial round of workgroups each time (384 x 384 x 192 with 4
+  // views: 2316 tiles on 768 resident workgroups).
+  ConvShape all = s;
+  const bool joined =
+      l.spec == sizeof(float2) * (size_t)nxp * s.ny * s.nz && (long)s.nz * p.V < (1L << 30);
+  if (joined) all.nz = s.nz * p.V;
+  const int runs = joined ? 1 : p.V;
   for (int it = 0; it < iterations; ++it) {
     pass_x_forward(s, psi, Spsi, nullptr, nullptr, st);
     pass_y_forward(s, Spsi, nullptr, nullptr, st);
     ez->rl.zfan(za, s.ny, st);
-    for (int v = 0; v < p.V; ++v) pass_y_inverse(s, Sv[v], st);
+    for (int v = 0; v < runs; ++v) pass_y_inverse(all, Sv[v], st);
     ex->rl.xratio(xa, p.V, st);
-    for (int v = 0; v < p.V; ++v) pass_y_forward(s, Sv[v], nullptr, nullptr, st);
+    for (int v = 0; v < runs; ++v) pass_y_forward(all, Sv[v], nullptr, nullptr, st);
     ez->rl.zsum(za, s.ny, st);
     pass_y_inverse(s, Spsi, st);
     ex->rl.xupdate(ua, st);

@@ -40,23 +40,6 @@ namespace fcamd {
 #define FC_RL_BOUNDS_CAT(n, w) FC_RL_BOUNDS_##w(n)
 #define FC_RL_BOUNDS(n, w) FC_RL_BOUNDS_CAT(n, w)
 
-// loads the compact kernel column of view v (planes placed at (z - cz) mod
-// L); positions are t + (compile-time constant) after unrolling, so each
-// access is a per-thread base plus a uniform offset
-template <int L, int MAXE>
-__device__ __forceinline__ void load_kernel_column(float2 (&w)[MAXE], int t, bool ok,
-                                                   const float2* kcol, long kplane, int kz, int cz) {
-  const float2* kt = kcol + (long)(t + cz) * kplane;
-  const float2* kw = kt - (long)L * kplane;
-  sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
-    const bool wrap = pos + cz >= L;
-    const int j = wrap ? pos + cz - L : pos + cz;
-    float2 val = make_float2(0.f, 0.f);
-    if (ok && j < kz) val = (wrap ? kw : kt)[(long)(pos - t) * kplane];
-    w[slot] = val;
-  });
-}
-
 // phi / d for d = max(blur, eps) > 0.  With eps a normal number (the
 // launch-uniform case FAST) every d is one, and the hardware reciprocal (at
 // most 1 ulp) times phi replaces the IEEE division sequence: one rounding
@@ -75,7 +58,9 @@ __device__ __forceinline__ T& col_at(T* base_t, int pos, int t, long stride) {
   return base_t[(long)(pos - t) * stride];
 }
 
-template <int L, int TX>
+// H: every view's taps lie within the first and last H stage-0 slots
+// (kernel_prune; 0: anywhere)
+template <int L, int TX, int H>
 __global__ void __launch_bounds__(TX * threads_per_transform<L>())
 sk_zfan(RLZArgs a) {
   using P = PlanOf<L, false>;
@@ -97,7 +82,7 @@ sk_zfan(RLZArgs a) {
   sfft_run<L, false, -1>(X, t, lds, addr, a.fft.stw);
   for (int v = 0; v < a.nviews; ++v) {
     float2 W[P::MAXE()];
-    load_kernel_column<L>(W, t, ok, a.kplanes[v] + base, a.s_plane, a.kz[v], a.cz[v]);
+    load_kernel_taps<L, H>(W, t, ok, a.kplanes[v] + base, a.s_plane, a.kz[v], a.cz[v]);
     sfft_run<L, false, -1>(W, t, lds, addr, a.fft.stw);
     sfft_for_outputs<L, false>(t, [&](int slot, int) { W[slot] = cscale(cmul(X[slot], W[slot]), a.scale); });
     sfft_run<L, true, +1>(W, t, lds, addr, a.fft.stw);
@@ -106,7 +91,7 @@ sk_zfan(RLZArgs a) {
   }
 }
 
-template <int L, int TX>
+template <int L, int TX, int H>
 __global__ void FC_RL_BOUNDS(TX * threads_per_transform<L>(), FC_RL_ZSUM_WAVES)
 sk_zsum(RLZArgs a) {
   using P = PlanOf<L, false>;
@@ -129,7 +114,7 @@ sk_zsum(RLZArgs a) {
       if (ok) val = col_at(in_t, pos, t, a.s_plane);
       X[slot] = val;
     });
-    load_kernel_column<L>(W, t, ok, a.kplanes[v] + base, a.s_plane, a.kz[v], a.cz[v]);
+    load_kernel_taps<L, H>(W, t, ok, a.kplanes[v] + base, a.s_plane, a.kz[v], a.cz[v]);
     sfft_run<L, false, -1>(X, t, lds, addr, a.fft.stw);
     sfft_run<L, false, -1>(W, t, lds, addr, a.fft.stw);
     sfft_for_outputs<L, false>(t, [&](int slot, int) { acc[slot] = cadd(acc[slot], cmulc(X[slot], W[slot])); });
@@ -380,13 +365,32 @@ sk_xupdate_flat(RLXArgs a) {
 #define FC_RL_XFLAT 1
 #endif
 
+// calls f with the pruned tap slots that hold every view's kernel
+template <int L, class F>
+void rl_with_slots(const RLZArgs& a, F f) {
+  int n = 1;  // the widest view's; 0: some view fits neither
+  for (int v = 0; v < a.nviews; ++v) {
+    const int p = kernel_prune<L>(a.kz[v], a.cz[v]);
+    n = p == 0 || n == 0 ? 0 : p > n ? p : n;
+  }
+  if (n == 1)
+    f(std::integral_constant<int, kernel_slots<L>(1)>{});
+  else if (n == 2)
+    f(std::integral_constant<int, kernel_slots<L>(2)>{});
+  else
+    f(std::integral_constant<int, 0>{});
+}
+
 template <int L>
 void rl_launch_zfan(const RLZArgs& a, long ny, hipStream_t st) {
   constexpr int TX = fit_tile<L, 16, kTileLdsZ>();
   RLZArgs b = a;
   b.ny = ny;
-  hipLaunchKernelGGL((sk_zfan<L, TX>), dim3((unsigned)column_tiles(a.nbins, TX, ny)),
-                     dim3(TX * threads_per_transform<L>()), 0, st, b);
+  rl_with_slots<L>(a, [&](auto h) {
+    hipLaunchKernelGGL((sk_zfan<L, TX, decltype(h)::value>),
+                       dim3((unsigned)column_tiles(a.nbins, TX, ny)),
+                       dim3(TX * threads_per_transform<L>()), 0, st, b);
+  });
 }
 
 template <int L>
@@ -394,8 +398,11 @@ void rl_launch_zsum(const RLZArgs& a, long ny, hipStream_t st) {
   constexpr int TX = fit_tile<L, 16, kTileLdsZ>();
   RLZArgs b = a;
   b.ny = ny;
-  hipLaunchKernelGGL((sk_zsum<L, TX>), dim3((unsigned)column_tiles(a.nbins, TX, ny)),
-                     dim3(TX * threads_per_transform<L>()), 0, st, b);
+  rl_with_slots<L>(a, [&](auto h) {
+    hipLaunchKernelGGL((sk_zsum<L, TX, decltype(h)::value>),
+                       dim3((unsigned)column_tiles(a.nbins, TX, ny)),
+                       dim3(TX * threads_per_transform<L>()), 0, st, b);
+  });
 }
 
 // the flat forms need dense real rows; the per-pair forms take any stride

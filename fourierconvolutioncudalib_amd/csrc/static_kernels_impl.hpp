@@ -45,12 +45,15 @@ constexpr int z_threads() {
 // (L rows of the tile).  A 16-bin tile is a 128-byte line per row and takes
 // up to CAP bytes; 8-bin tiles move half lines and reach 3.0-4.1 TB/s in a
 // bare copy where 16-bin tiles reach 5.1-6.4 (384 x 384 x 192 to 512 x 512 x
-// 256).  Two workgroups per CU (80 KiB each) always pay: y passes over L x 512
-// x 64 volumes 42.8 -> 33.9 us at L = 540, 46.3 -> 43.6 at 600, the z pass at
-// 640 180 -> 126 us.  One workgroup per CU still pays in the y passes up to
-// 768 (60.6 -> 57.9 and 56.9 -> 50.2 us), not beyond (1024: 85 -> 90 us
-// forward), and never in the z pass (720: 132 -> 138 us, 960: 180 -> 201 us).
-constexpr int kTileLds = 65536, kTileLdsZ = 81920, kTileLdsCol = 98304;
+// 256).  Two workgroups per CU (80 KiB each) pay: y passes over L x 512 x 64
+// volumes 42.8 -> 33.9 us at L = 540, 46.3 -> 43.6 at 600, the z pass at 640
+// 180 -> 126 us.  One workgroup per CU still pays in the inverse y pass up to
+// 768 (56.9 -> 50.2 us), not in the z pass (720: 132 -> 138, 960: 180 -> 201
+// us), and the forward y pass takes 16 bins to 600 only: its launch may carry
+// many kernel planes, whose tiles are arithmetic alone (48 of them at 640 x
+// 640 x 48: 71 -> 77 us, at 768 x 512 x 48: 70 -> 78; without them 48 -> 47
+// and 60.6 -> 57.9).
+constexpr int kTileLds = 65536, kTileLdsFwd = 76800, kTileLdsZ = 81920, kTileLdsInv = 98304;
 template <int L, int WANT, int CAP = kTileLds, int T = threads_per_transform<L>()>
 constexpr int fit_tile() {
   int tx = WANT;
@@ -60,8 +63,10 @@ constexpr int fit_tile() {
   return tx;
 }
 // tiles of the column (y) and z passes
-template <int L, int WANT>
-constexpr int col_fit() { return fit_tile<L, WANT, WANT == 16 ? kTileLdsCol : kTileLds>(); }
+template <int L, int WANT, int DIR>
+constexpr int col_fit() {
+  return fit_tile<L, WANT, WANT != 16 ? kTileLds : DIR < 0 ? kTileLdsFwd : kTileLdsInv>();
+}
 template <int L, int WANT>
 constexpr int z_fit() {
   return fit_tile<L, WANT, WANT == 16 ? kTileLdsZ : kTileLds, z_threads<L, 0>()>();
@@ -1040,7 +1045,9 @@ inline int kernel_prune(int nvalid, int center) {
 }
 
 // w <- the kernel column's taps at the thread's stage-0 positions (ID: plan
-// identifier of length L); H as in ZTile::load_kernel
+// identifier of length L); H as in ZTile::load_kernel.  Nothing uses a value
+// here: the loads stay in flight under what follows (scaling the taps as they
+// arrive made the z pass 5-15 % slower)
 template <int ID, int H, int MAXE>
 __device__ __forceinline__ void load_kernel_taps(float2 (&w)[MAXE], int t, bool ok,
                                                  const float2* kcol, long kp, int nvalid,
@@ -1464,19 +1471,21 @@ Col2 col2_tiles(const Col2& a) {
 template <int L, int WANT, bool REV = false>
 bool sk_launch_col(const Col2& a, int dir, hipStream_t st) {
   if (REV && PlanOf<L, false>::S < 2) return false;  // one stage: same as forward order
-  constexpr int TX = col_fit<L, WANT>();
-  const Col2 b = col2_tiles<L, TX>(a);
-  const dim3 block(TX * threads_per_transform<L>());
-  if (dir < 0)
-    hipLaunchKernelGGL((sk_col<L, TX, -1, REV>), dim3((unsigned)b.ntiles), block, 0, st, b);
-  else
-    hipLaunchKernelGGL((sk_col<L, TX, +1, REV>), dim3((unsigned)b.ntiles), block, 0, st, b);
+  constexpr int TF = col_fit<L, WANT, -1>(), TI = col_fit<L, WANT, +1>();
+  constexpr int T = threads_per_transform<L>();
+  if (dir < 0) {
+    const Col2 b = col2_tiles<L, TF>(a);
+    hipLaunchKernelGGL((sk_col<L, TF, -1, REV>), dim3((unsigned)b.ntiles), dim3(TF * T), 0, st, b);
+  } else {
+    const Col2 b = col2_tiles<L, TI>(a);
+    hipLaunchKernelGGL((sk_col<L, TI, +1, REV>), dim3((unsigned)b.ntiles), dim3(TI * T), 0, st, b);
+  }
   return true;
 }
 
 template <int L, int WANT>
 bool sk_launch_col_pipe(const Col2& a, int dir, hipStream_t st) {
-  constexpr int TX = col_fit<L, WANT>();
+  constexpr int TX = col_fit<L, WANT, -1>();
   constexpr int threads = TX * threads_per_transform<L>();
   const Col2 b = col2_tiles<L, TX>(a);
   const void* fn = dir < 0 ? (const void*)sk_col_pipe<L, TX, -1> : (const void*)sk_col_pipe<L, TX, +1>;
@@ -1538,14 +1547,16 @@ void sk_launch_xinv_ext(const XExtArgs& a, hipStream_t st) {
 }
 template <int L>
 void sk_launch_col_ext(const ColExtArgs& a, int dir, hipStream_t st) {
-  constexpr int TX = col_fit<L, 16>();
+  constexpr int TF = col_fit<L, 16, -1>(), TI = col_fit<L, 16, +1>();
+  constexpr int T = threads_per_transform<L>();
   ColExtArgs b = a;
-  b.c = col2_tiles<L, TX>(a.c);
-  const dim3 grid((unsigned)b.c.ntiles), block(TX * threads_per_transform<L>());
-  if (dir < 0)
-    hipLaunchKernelGGL((sk_col_ext<L, TX, -1>), grid, block, 0, st, b);
-  else
-    hipLaunchKernelGGL((sk_col_ext<L, TX, +1>), grid, block, 0, st, b);
+  if (dir < 0) {
+    b.c = col2_tiles<L, TF>(a.c);
+    hipLaunchKernelGGL((sk_col_ext<L, TF, -1>), dim3((unsigned)b.c.ntiles), dim3(TF * T), 0, st, b);
+  } else {
+    b.c = col2_tiles<L, TI>(a.c);
+    hipLaunchKernelGGL((sk_col_ext<L, TI, +1>), dim3((unsigned)b.c.ntiles), dim3(TI * T), 0, st, b);
+  }
 }
 template <int L>
 void sk_launch_zfused_ext(const ZExtArgs& a, long ny, hipStream_t st) {
@@ -1646,13 +1657,13 @@ StaticEntry make_static_entry() {
             {"w256-ldsmirror", &sk_launch_xinv_lds<L, 256>},
             {"w256-flat", &sk_launch_xinv_flat<L, 256>},
             {"w128-flat", &sk_launch_xinv_flat<L, 128>}};
-  e.col = {{"t16", &sk_launch_col<L, 16>, col_fit<L, 16>()},
+  e.col = {{"t16", &sk_launch_col<L, 16>, col_fit<L, 16, +1>()},
            {"t16-pipe", &sk_launch_col_pipe<L, 16>},
            {"t8-pipe", &sk_launch_col_pipe<L, 8>},
            {"t16-revradix", &sk_launch_col<L, 16, true>},
-           {"t8", &sk_launch_col<L, 8>, col_fit<L, 8>()},
-           {"t32", &sk_launch_col<L, 32>, col_fit<L, 32>()},
-           {"t64", &sk_launch_col<L, 64>, col_fit<L, 64>()}};
+           {"t8", &sk_launch_col<L, 8>, col_fit<L, 8, +1>()},
+           {"t32", &sk_launch_col<L, 32>, col_fit<L, 32, +1>()},
+           {"t64", &sk_launch_col<L, 64>, col_fit<L, 64, +1>()}};
   e.zfused = {{"t16-fft", &sk_launch_zfused_fft<L, 16>},
               {"t16-dft", &sk_launch_zfused_dft<L, 16>},
               {"t8-fft", &sk_launch_zfused_fft<L, 8>},
