@@ -15,6 +15,8 @@
 // product and an inverse transform chain with no LDS exchange in between.
 #pragma once
 
+#include <type_traits>
+
 #include "fc_internal.hpp"
 #include "fft_radix.hpp"
 
@@ -287,7 +289,18 @@ __device__ __forceinline__ void sfft_compute(float2 (&v)[MAXE], int t, const flo
   }
 }
 
-// Writes stage s outputs to LDS through `addr(pos)`.
+// LDS index of position base + off (off a compile-time constant once
+// unrolled): addr(base, off) where the address form can split it, so that the
+// constant part becomes the instruction's offset, else addr(base + off)
+template <class Addr>
+__device__ __forceinline__ int lds_index(const Addr& addr, int base, int off) {
+  if constexpr (std::is_invocable_v<Addr, int, int>)
+    return addr(base, off);
+  else
+    return addr(base + off);
+}
+
+// Writes stage s outputs to LDS through `addr`.
 template <int L, bool REV, int s, int MAXE, class Addr>
 __device__ __forceinline__ void sfft_store_lds(const float2 (&v)[MAXE], int t, float2* lds, Addr addr) {
   using P = PlanOf<L, REV>;
@@ -299,7 +312,7 @@ __device__ __forceinline__ void sfft_store_lds(const float2 (&v)[MAXE], int t, f
     const int k = b % Ns;
     const int base = (b - k) * R + k;
 #pragma unroll
-    for (int r = 0; r < R; ++r) lds[addr(base + r * Ns)] = v[i * R + r];
+    for (int r = 0; r < R; ++r) lds[lds_index(addr, base, r * Ns)] = v[i * R + r];
   }
 }
 
@@ -313,7 +326,7 @@ __device__ __forceinline__ void sfft_load_lds(float2 (&v)[MAXE], int t, const fl
     const int b = t + i * P::T;
     if ((M % P::T) != 0 && b >= M) continue;
 #pragma unroll
-    for (int r = 0; r < R; ++r) v[i * R + r] = lds[addr(b + r * M)];
+    for (int r = 0; r < R; ++r) v[i * R + r] = lds[lds_index(addr, t, i * P::T + r * M)];
   }
 }
 

@@ -160,7 +160,7 @@ sk_xratio(RLXArgs a) {
     z[slot] = make_float2(A.x - B.y, A.y + B.x);
   });
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, true, +1>(z, t, row, addr, a.fft.stw);
   // real rows of the blurred estimate -> ratio rows (same positions)
   const float* fa = a.phi[v] + ra * a.rrow;
@@ -180,7 +180,7 @@ sk_xratio(RLXArgs a) {
   else
     ratio(std::false_type{});
   sfft_run<L, false, -1>(z, t, row, addr, a.fft.stw);
-  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(pos)] = z[slot]; });
+  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(t, pos - t)] = z[slot]; });
   __syncthreads();
   for (int kb = t; kb < nb; kb += T) {
     const float2 Z = row[addr(kb)];
@@ -220,7 +220,7 @@ sk_xupdate(RLXArgs a) {
     z[slot] = make_float2(A.x - B.y, A.y + B.x);
   });
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, false, +1>(z, t, row, addr, a.fft.stw);
   float* qa = a.psi + ra * a.rrow;
   float* qb = a.psi + rb * a.rrow;
@@ -239,7 +239,7 @@ template <int L, int PAIRS>
 __global__ void FC_RL_BOUNDS(PAIRS * threads_per_transform<L>(), FC_RL_XRATIO_WAVES)
 sk_xratio_flat(RLXArgs a) {
   using P = PlanOf<L, false>;
-  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL, NB = XStage<L>::NB;
+  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL;
   constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
   __shared__ float2 lds[xflat_lds_floats<L>(PAIRS) / 2];
   const long groups = ((a.nrows + 1) / 2 + PAIRS - 1) / PAIRS;
@@ -247,44 +247,29 @@ sk_xratio_flat(RLXArgs a) {
   const long r0 = 2 * (blockIdx.x - (long)v * groups) * PAIRS;
   const int nr = a.nrows - r0 < MAXR ? (int)(a.nrows - r0) : MAXR;
   float2* spec = a.spec[v];
-  xflat_load_bins<L, NT, MAXR>(spec + r0 * a.srow, a.srow, lds, nr);
+  XBins<L, PAIRS>().load(spec + r0 * a.srow, a.srow, nr, lds);
   __syncthreads();
   const int t = threadIdx.x % T, c = threadIdx.x / T;
-  const bool oka = 2 * c < nr, okb = 2 * c + 1 < nr;
-  const float2* sa = lds + 2 * c * NB;
-  const float2* sb = sa + NB;
   float2 z[P::MAXE()];
   // C2R on the reversed plan: its outputs sit where the forward plan reads
-  sfft_for_inputs<L, true>(t, [&](int slot, int pos) {
-    const bool mirror = pos >= NB;
-    const int kb = mirror ? L - pos : pos;
-    float2 A = oka ? sa[kb] : make_float2(0.f, 0.f);
-    float2 B = okb ? sb[kb] : make_float2(0.f, 0.f);
-    if (kb == 0 || 2 * kb == L) {
-      A.y = 0.f;
-      B.y = 0.f;
-    }
-    if (mirror) {
-      A.y = -A.y;
-      B.y = -B.y;
-    }
-    z[slot] = make_float2(A.x - B.y, A.y + B.x);
-  });
+  const float2* in = lds + c * LP;
+  sfft_for_inputs<L, true>(t, [&](int slot, int pos) { z[slot] = in[XRow<L>::at(t, pos - t)]; });
   __syncthreads();
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, true, +1>(z, t, row, addr, a.fft.stw);
   // phi rows through LDS; ratio at the transform's output positions
   float* st = reinterpret_cast<float*>(lds);
   xflat_load_rows<L, NT, MAXR>(a.phi[v] + r0 * L, st, nr);
   __syncthreads();
+  const float* fa = st + 2 * c * SL;
+  const float* fb = fa + (2 * c + 1 < nr ? SL : 0);  // a missing second row repeats the first
   const float eps = a.eps;
   auto ratio = [&](auto fast) {
     constexpr bool F = decltype(fast)::value;
     sfft_for_outputs<L, true>(t, [&](int slot, int pos) {
-      const float ya = oka ? rl_div<F>(st[2 * c * SL + pos], fmaxf(z[slot].x, eps)) : 0.f;
-      const float yb = okb ? rl_div<F>(st[(2 * c + 1) * SL + pos], fmaxf(z[slot].y, eps)) : 0.f;
-      z[slot] = make_float2(ya, yb);
+      z[slot] = make_float2(rl_div<F>(fa[pos], fmaxf(z[slot].x, eps)),
+                            rl_div<F>(fb[pos], fmaxf(z[slot].y, eps)));
     });
   };
   if (eps >= kMinNormal)
@@ -293,59 +278,30 @@ sk_xratio_flat(RLXArgs a) {
     ratio(std::false_type{});
   __syncthreads();
   sfft_run<L, false, -1>(z, t, row, addr, a.fft.stw);
-  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(pos)] = z[slot]; });
+  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(t, pos - t)] = z[slot]; });
   __syncthreads();
-  // Hermitian split back into the view's spectrum rows, bin-contiguous
-  constexpr int IT = (MAXR * NB + NT - 1) / NT;
-  const int n = nr * NB;
-#pragma unroll
-  for (int j = 0; j < IT; ++j) {
-    const int i = threadIdx.x + j * NT;
-    if (i < n) {
-      const int r = i / NB, kb = i - r * NB;
-      const float2* pr = lds + (r >> 1) * LP;
-      const float2 Z = pr[addr(kb)];
-      const float2 Zm = pr[addr(kb == 0 ? 0 : L - kb)];
-      spec[(r0 + r) * a.srow + kb] = (r & 1) ? make_float2(0.5f * (Z.y + Zm.y), 0.5f * (Zm.x - Z.x))
-                                            : make_float2(0.5f * (Z.x + Zm.x), 0.5f * (Z.y - Zm.y));
-    }
-  }
+  // Hermitian split back into the view's spectrum rows
+  XBins<L, PAIRS>::again().store(spec + r0 * a.srow, a.srow, nr, lds);
 }
 
 template <int L, int PAIRS>
 __global__ void __launch_bounds__(PAIRS * threads_per_transform<L>())
 sk_xupdate_flat(RLXArgs a) {
   using P = PlanOf<L, false>;
-  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL, NB = XStage<L>::NB;
+  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL;
   constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
   __shared__ float2 lds[xflat_lds_floats<L>(PAIRS) / 2];
   const long r0 = 2 * (long)blockIdx.x * PAIRS;
   const int nr = a.nrows - r0 < MAXR ? (int)(a.nrows - r0) : MAXR;
-  xflat_load_bins<L, NT, MAXR>(a.spec[0] + r0 * a.srow, a.srow, lds, nr);
+  XBins<L, PAIRS>().load(a.spec[0] + r0 * a.srow, a.srow, nr, lds);
   __syncthreads();
   const int t = threadIdx.x % T, c = threadIdx.x / T;
-  const bool oka = 2 * c < nr, okb = 2 * c + 1 < nr;
-  const float2* sa = lds + 2 * c * NB;
-  const float2* sb = sa + NB;
   float2 z[P::MAXE()];
-  sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
-    const bool mirror = pos >= NB;
-    const int kb = mirror ? L - pos : pos;
-    float2 A = oka ? sa[kb] : make_float2(0.f, 0.f);
-    float2 B = okb ? sb[kb] : make_float2(0.f, 0.f);
-    if (kb == 0 || 2 * kb == L) {
-      A.y = 0.f;
-      B.y = 0.f;
-    }
-    if (mirror) {
-      A.y = -A.y;
-      B.y = -B.y;
-    }
-    z[slot] = make_float2(A.x - B.y, A.y + B.x);
-  });
+  const float2* in = lds + c * LP;
+  sfft_for_inputs<L, false>(t, [&](int slot, int pos) { z[slot] = in[XRow<L>::at(t, pos - t)]; });
   __syncthreads();
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, false, +1>(z, t, row, addr, a.fft.stw);
   // psi rows through LDS: psi <- psi * acc / V at the output positions
   float* st = reinterpret_cast<float*>(lds);
@@ -354,8 +310,8 @@ sk_xupdate_flat(RLXArgs a) {
   __syncthreads();
   const float iv = a.inv_views;
   sfft_for_outputs<L, false>(t, [&](int slot, int pos) {
-    if (oka) st[2 * c * SL + pos] *= z[slot].x * iv;
-    if (okb) st[(2 * c + 1) * SL + pos] *= z[slot].y * iv;
+    st[2 * c * SL + pos] *= z[slot].x * iv;  // (rows past nr are not stored)
+    st[(2 * c + 1) * SL + pos] *= z[slot].y * iv;
   });
   __syncthreads();
   xflat_store_rows<L, NT, MAXR>(psi, st, nr);

@@ -95,6 +95,14 @@ template <int L>
 struct XRow {
   static constexpr int LP = L + L / 8 + 1;
   __device__ static int at(int pos) { return pos + (pos >> 3); }
+  // at(base + off): an offset of whole eights moves the index by a constant
+  __device__ static int at(int base, int off) {
+    return off % 8 == 0 ? at(base) + off + off / 8 : at(base + off);
+  }
+};
+struct XAddr {
+  __device__ int operator()(int pos) const { return XRow<0>::at(pos); }
+  __device__ int operator()(int base, int off) const { return XRow<0>::at(base, off); }
 };
 
 // ---------------------------------------------------------------------------
@@ -124,9 +132,9 @@ __device__ __forceinline__ void xfwd_body(const XPassArgs& a, long blk, float2* 
     v[slot] = make_float2(xa, xb);
   });
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, false, -1, 9>(v, t, row, addr, a.fft.stw);
-  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(pos)] = v[slot]; });
+  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(t, pos - t)] = v[slot]; });
   __syncthreads();
   float2* da = a.dst + ra * a.dst_row;
   float2* db = a.dst + rb * a.dst_row;
@@ -164,9 +172,9 @@ __device__ __forceinline__ void xfwd_vpad_body(const XPassArgs& a, long blk, flo
     v[slot] = make_float2(xa, xb);
   });
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, false, -1, 9>(v, t, row, addr, a.fft.stw);
-  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(pos)] = v[slot]; });
+  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(t, pos - t)] = v[slot]; });
   __syncthreads();
   float2* da = a.dst + ra * a.dst_row;
   float2* db = a.dst + rb * a.dst_row;
@@ -233,7 +241,7 @@ __device__ __forceinline__ void xinv_body(const XPassArgs& a, long blk, float2* 
     v[slot] = make_float2(A.x - B.y, A.y + B.x);
   });
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, false, +1>(v, t, row, addr, a.fft.stw);
   float* oa = a.rdst + ra * a.dst_row;
   float* ob = a.rdst + rb * a.dst_row;
@@ -256,7 +264,7 @@ __device__ __forceinline__ void xinv_lds_body(const XPassArgs& a, long blk, floa
   const float2* pb = a.csrc + rb * a.src_row;
   const int nb = a.nbins;
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   // Z = A' + iB' over all L positions, built from the nb bins of each row:
   // position kb takes A + iB, its mirror L - kb takes conj(A) + i conj(B)
   for (int kb = t; kb < nb; kb += T) {
@@ -273,7 +281,7 @@ __device__ __forceinline__ void xinv_lds_body(const XPassArgs& a, long blk, floa
   }
   __syncthreads();
   float2 v[P::MAXE()];
-  sfft_for_inputs<L, false>(t, [&](int slot, int pos) { v[slot] = row[addr(pos)]; });
+  sfft_for_inputs<L, false>(t, [&](int slot, int pos) { v[slot] = row[addr(t, pos - t)]; });
   __syncthreads();
   sfft_run<L, false, +1>(v, t, row, addr, a.fft.stw);
   float* oa = a.rdst + ra * a.dst_row;
@@ -315,15 +323,13 @@ struct XStage {
   static constexpr int NB = L / 2 + 1;           // half-spectrum bins per row
 };
 
-// LDS floats of a flat x-pass workgroup of `pairs` row pairs: the largest of
-// the exchange rows, the real staging rows and the spectrum staging rows
+// LDS floats of a flat x-pass workgroup of `pairs` row pairs: the larger of
+// the exchange rows and the real staging rows
 template <int L>
 constexpr int xflat_lds_floats(int pairs) {
   const int ex = 2 * pairs * XRow<L>::LP;
   const int st = 2 * pairs * XStage<L>::SL;
-  const int sc = 4 * pairs * XStage<L>::NB;
-  const int m = ex > st ? ex : st;
-  return m > sc ? m : sc;
+  return ex > st ? ex : st;
 }
 
 // row pairs of a flat x-pass workgroup: about TGT threads, within 1024
@@ -348,47 +354,59 @@ constexpr int batch_pairs() {
   return FC_BATCH_XFLAT ? flat_pairs<L, FC_BATCH_XTGT>() : fit_pairs<L, pairs_for<L, FC_BATCH_XTGT>()>();
 }
 
-// nr dense rows of L floats at g -> staging rows of stride SL
+// nr dense rows of L floats at g -> staging rows of stride SL.  A full
+// workgroup's rows move without a bounds test per piece; only the last
+// workgroup of a pass (or plane) is not full, and takes a rolled loop.
 template <int L, int NT, int MAXR>
 __device__ __forceinline__ void xflat_load_rows(const float* __restrict__ g, float* st, int nr) {
   constexpr int SL = XStage<L>::SL;
   if constexpr (XStage<L>::V4) {
     if ((reinterpret_cast<uintptr_t>(g) & 15) == 0) {
-      constexpr int Q = L / 4, IT = (MAXR * Q + NT - 1) / NT;
-      const int n = nr * Q;
+      constexpr int Q = L / 4, N = MAXR * Q, IT = (N + NT - 1) / NT;
       const float4* g4 = reinterpret_cast<const float4*>(g);
-      float4 r[IT];
+      auto put = [&](int i, float4 v) {
+        const int row = i / Q;
+        *reinterpret_cast<float4*>(st + row * SL + 4 * (i - row * Q)) = v;
+      };
+      if (nr == MAXR) {
+        float4 r[IT];
 #pragma unroll
-      for (int j = 0; j < IT; ++j) {
-        const int i = threadIdx.x + j * NT;
-        r[j] = i < n ? g4[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-#pragma unroll
-      for (int j = 0; j < IT; ++j) {
-        const int i = threadIdx.x + j * NT;
-        if (i < n) {
-          const int row = i / Q;
-          *reinterpret_cast<float4*>(st + row * SL + 4 * (i - row * Q)) = r[j];
+        for (int j = 0; j < IT; ++j) {
+          const int i = threadIdx.x + j * NT;
+          if ((j + 1) * NT <= N || i < N) r[j] = g4[i];
         }
+#pragma unroll
+        for (int j = 0; j < IT; ++j) {
+          const int i = threadIdx.x + j * NT;
+          if ((j + 1) * NT <= N || i < N) put(i, r[j]);
+        }
+      } else {
+#pragma unroll 1
+        for (int i = threadIdx.x; i < nr * Q; i += NT) put(i, g4[i]);
       }
       return;
     }
   }
-  constexpr int IT = (MAXR * L + NT - 1) / NT;
-  const int n = nr * L;
-  float r[IT];
+  constexpr int N = MAXR * L, IT = (N + NT - 1) / NT;
+  auto put = [&](int i, float v) {
+    const int row = i / L;
+    st[row * SL + (i - row * L)] = v;
+  };
+  if (nr == MAXR) {
+    float r[IT];
 #pragma unroll
-  for (int j = 0; j < IT; ++j) {
-    const int i = threadIdx.x + j * NT;
-    r[j] = i < n ? g[i] : 0.f;
-  }
-#pragma unroll
-  for (int j = 0; j < IT; ++j) {
-    const int i = threadIdx.x + j * NT;
-    if (i < n) {
-      const int row = i / L;
-      st[row * SL + (i - row * L)] = r[j];
+    for (int j = 0; j < IT; ++j) {
+      const int i = threadIdx.x + j * NT;
+      if ((j + 1) * NT <= N || i < N) r[j] = g[i];
     }
+#pragma unroll
+    for (int j = 0; j < IT; ++j) {
+      const int i = threadIdx.x + j * NT;
+      if ((j + 1) * NT <= N || i < N) put(i, r[j]);
+    }
+  } else {
+#pragma unroll 1
+    for (int i = threadIdx.x; i < nr * L; i += NT) put(i, g[i]);
   }
 }
 
@@ -398,60 +416,178 @@ __device__ __forceinline__ void xflat_store_rows(float* __restrict__ g, const fl
   constexpr int SL = XStage<L>::SL;
   if constexpr (XStage<L>::V4) {
     if ((reinterpret_cast<uintptr_t>(g) & 15) == 0) {
-      constexpr int Q = L / 4, IT = (MAXR * Q + NT - 1) / NT;
-      const int n = nr * Q;
+      constexpr int Q = L / 4, N = MAXR * Q, IT = (N + NT - 1) / NT;
       float4* g4 = reinterpret_cast<float4*>(g);
+      auto put = [&](int i) {
+        const int row = i / Q;
+        g4[i] = *reinterpret_cast<const float4*>(st + row * SL + 4 * (i - row * Q));
+      };
+      if (nr == MAXR) {
 #pragma unroll
-      for (int j = 0; j < IT; ++j) {
-        const int i = threadIdx.x + j * NT;
-        if (i < n) {
-          const int row = i / Q;
-          g4[i] = *reinterpret_cast<const float4*>(st + row * SL + 4 * (i - row * Q));
+        for (int j = 0; j < IT; ++j) {
+          const int i = threadIdx.x + j * NT;
+          if ((j + 1) * NT <= N || i < N) put(i);
         }
+      } else {
+#pragma unroll 1
+        for (int i = threadIdx.x; i < nr * Q; i += NT) put(i);
       }
       return;
     }
   }
-  constexpr int IT = (MAXR * L + NT - 1) / NT;
-  const int n = nr * L;
+  constexpr int N = MAXR * L, IT = (N + NT - 1) / NT;
+  auto put = [&](int i) {
+    const int row = i / L;
+    g[i] = st[row * SL + (i - row * L)];
+  };
+  if (nr == MAXR) {
 #pragma unroll
-  for (int j = 0; j < IT; ++j) {
-    const int i = threadIdx.x + j * NT;
-    if (i < n) {
-      const int row = i / L;
-      g[i] = st[row * SL + (i - row * L)];
+    for (int j = 0; j < IT; ++j) {
+      const int i = threadIdx.x + j * NT;
+      if ((j + 1) * NT <= N || i < N) put(i);
     }
+  } else {
+#pragma unroll 1
+    for (int i = threadIdx.x; i < nr * L; i += NT) put(i);
   }
 }
 
-// nr spectrum rows (NB bins each, row pitch `pitch`) -> dense staging rows
-template <int L, int NT, int MAXR>
-__device__ __forceinline__ void xflat_load_bins(const float2* __restrict__ g, long pitch,
-                                                float2* sc, int nr) {
-  constexpr int NB = XStage<L>::NB, IT = (MAXR * NB + NT - 1) / NT;
-  const int n = nr * NB;
-  float2 r[IT];
-#pragma unroll
-  for (int j = 0; j < IT; ++j) {
-    const int i = threadIdx.x + j * NT;
-    r[j] = make_float2(0.f, 0.f);
-    if (i < n) {
-      const int row = i / NB;
-      r[j] = g[row * pitch + (i - row * NB)];
+// Spectrum rows of a flat x-pass workgroup.  A lane keeps one bin (two or
+// more where a row is longer than the workgroup) over all row pairs, G pairs
+// at a time, so that a row or pair step moves every address by a constant;
+// walking the rows' bins as one run takes a division by the bin count and
+// 64-bit address arithmetic per bin.  The lone Nyquist bin of even L goes
+// last, one lane per pair.
+template <int L, int PAIRS>
+struct XBins {
+  static constexpr int NT = PAIRS * PlanOf<L, false>::T;
+  static constexpr int MB = (L + 1) / 2;                   // bins below Nyquist
+  static constexpr int G = NT >= MB ? NT / MB : 1;         // pairs side by side
+  static constexpr int KI = NT >= MB ? 1 : (MB + NT - 1) / NT;  // bins per lane
+  static constexpr int PI = (PAIRS + G - 1) / G;           // pair steps
+  static constexpr int LP = XRow<L>::LP;
+  int tid, g, k0;
+  __device__ explicit XBins(int t) : tid(t), g(t / MB), k0(t - g * MB) {
+    if (G == 1 && KI > 1) {
+      g = 0;
+      k0 = t;
     }
   }
-#pragma unroll
-  for (int j = 0; j < IT; ++j) {
-    const int i = threadIdx.x + j * NT;
-    if (i < n) sc[i] = r[j];
+  __device__ XBins() : XBins((int)threadIdx.x) {}
+  // for a second use far from the first: the compiler cannot tell that the
+  // lane's constants are the same and does not hold them across a transform
+  __device__ static XBins again() {
+    int t = threadIdx.x;
+    asm("" : "+v"(t));
+    return XBins(t);
   }
-}
+  // does the lane hold pair step pi of bin step ki in a full workgroup?
+  // (compile-time true but in the last steps)
+  __device__ bool has(int pi, int ki) const {
+    return ((pi + 1) * G <= PAIRS || g + pi * G < PAIRS) &&
+           ((ki + 1) * NT <= MB || k0 + ki * NT < MB);
+  }
+  __device__ bool active() const { return G * MB >= NT || g < G; }
+  // Z = A + iB of a row pair at the exchange positions of bin k, Hermitian
+  // extension included (bin 0's imaginary parts dropped, as a C2R does)
+  __device__ static void put(float2* lo, float2* hi, float2 a, float2 b, bool dc) {
+    if (dc) a.y = b.y = 0.f;
+    *lo = make_float2(a.x - b.y, a.y + b.x);
+    *hi = make_float2(a.x + b.y, b.x - a.y);
+  }
+  __device__ static void split(float2* pa, float2* pb, float2 Z, float2 Zm, bool second) {
+    *pa = make_float2(0.5f * (Z.x + Zm.x), 0.5f * (Z.y - Zm.y));
+    if (second) *pb = make_float2(0.5f * (Z.y + Zm.y), 0.5f * (Zm.x - Z.x));
+  }
+  // the exchange rows of every row pair from nr spectrum rows at g_ (row
+  // pitch `pitch`); a missing last row repeats its pair's first (its result
+  // is not stored)
+  __device__ void load(const float2* __restrict__ g_, long pitch, int nr, float2* rows) const {
+    const int npairs = (nr + 1) >> 1;
+    float2 nyq = make_float2(0.f, 0.f);
+    if (L % 2 == 0 && tid < npairs) {  // the pair whose Nyquist bin the lane moves
+      const float2* p = g_ + (long)(2 * tid) * pitch + L / 2;
+      nyq.x = p[0].x;
+      nyq.y = p[2 * tid + 1 < nr ? pitch : 0].x;
+    }
+    if (nr == 2 * PAIRS) {
+      const float2* base = g_ + (long)(2 * g) * pitch + k0;
+      float2 A[KI * PI], B[KI * PI];
+      if (active()) {
+#pragma unroll
+        for (int ki = 0; ki < KI; ++ki)
+#pragma unroll
+          for (int pi = 0; pi < PI; ++pi) {
+            if (!has(pi, ki)) continue;
+            const float2* p = base + (long)(2 * pi * G) * pitch + ki * NT;
+            A[ki * PI + pi] = p[0];
+            B[ki * PI + pi] = p[pitch];
+          }
+#pragma unroll
+        for (int ki = 0; ki < KI; ++ki) {
+          const int k = k0 + ki * NT;
+          float2* lo = rows + g * LP + XRow<L>::at(k);
+          float2* hi = rows + g * LP + XRow<L>::at(k == 0 ? 0 : L - k);
+#pragma unroll
+          for (int pi = 0; pi < PI; ++pi)
+            if (has(pi, ki))
+              put(lo + pi * G * LP, hi + pi * G * LP, A[ki * PI + pi], B[ki * PI + pi], k == 0);
+        }
+      }
+    } else {
+#pragma unroll 1
+      for (int i = tid; i < npairs * MB; i += NT) {
+        const int c = i / MB, k = i - c * MB;
+        const float2* p = g_ + (long)(2 * c) * pitch + k;
+        put(rows + c * LP + XRow<L>::at(k), rows + c * LP + XRow<L>::at(k == 0 ? 0 : L - k), p[0],
+            p[2 * c + 1 < nr ? pitch : 0], k == 0);
+      }
+    }
+    if (L % 2 == 0 && tid < npairs) rows[tid * LP + XRow<L>::at(L / 2)] = nyq;
+  }
+  // the half spectra of both rows of every pair, separated from the pair's
+  // complex transform in the exchange rows
+  __device__ void store(float2* __restrict__ g_, long pitch, int nr, const float2* rows) const {
+    const int npairs = (nr + 1) >> 1;
+    if (nr == 2 * PAIRS) {
+      float2* base = g_ + (long)(2 * g) * pitch + k0;
+      if (active()) {
+#pragma unroll
+        for (int ki = 0; ki < KI; ++ki) {
+          const int k = k0 + ki * NT;
+          const float2* lo = rows + g * LP + XRow<L>::at(k);
+          const float2* hi = rows + g * LP + XRow<L>::at(k == 0 ? 0 : L - k);
+#pragma unroll
+          for (int pi = 0; pi < PI; ++pi) {
+            if (!has(pi, ki)) continue;
+            float2* p = base + (long)(2 * pi * G) * pitch + ki * NT;
+            split(p, p + pitch, lo[pi * G * LP], hi[pi * G * LP], true);
+          }
+        }
+      }
+    } else {
+#pragma unroll 1
+      for (int i = tid; i < npairs * MB; i += NT) {
+        const int c = i / MB, k = i - c * MB;
+        float2* p = g_ + (long)(2 * c) * pitch + k;
+        split(p, p + pitch, rows[c * LP + XRow<L>::at(k)],
+              rows[c * LP + XRow<L>::at(k == 0 ? 0 : L - k)], 2 * c + 1 < nr);
+      }
+    }
+    if (L % 2 == 0 && tid < npairs) {
+      const float2 Z = rows[tid * LP + XRow<L>::at(L / 2)];
+      float2* p = g_ + (long)(2 * tid) * pitch + L / 2;
+      p[0] = make_float2(Z.x, 0.f);
+      if (2 * tid + 1 < nr) p[pitch] = make_float2(Z.y, 0.f);
+    }
+  }
+};
 
 // R2C of up to 2*PAIRS dense image rows starting at row 2*blk*PAIRS
 template <int L, int PAIRS>
 __device__ __forceinline__ void xfwd_flat_body(const XPassArgs& a, long blk, float2* lds) {
   using P = PlanOf<L, false>;
-  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL, NB = XStage<L>::NB;
+  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL;
   constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
   const long r0 = 2 * blk * PAIRS;
   if (r0 >= a.nrows) return;  // whole workgroup
@@ -460,70 +596,39 @@ __device__ __forceinline__ void xfwd_flat_body(const XPassArgs& a, long blk, flo
   xflat_load_rows<L, NT, MAXR>(a.src + r0 * L, st, nr);
   __syncthreads();
   const int t = threadIdx.x % T, c = threadIdx.x / T;
-  const bool oka = 2 * c < nr, okb = 2 * c + 1 < nr;
+  // a missing second row repeats the first (its result is not stored); pairs
+  // past the last transform what the staging area holds
+  const float* ra = st + 2 * c * SL;
+  const float* rb = ra + (2 * c + 1 < nr ? SL : 0);
   float2 v[P::MAXE()];
-  sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
-    v[slot] = make_float2(oka ? st[2 * c * SL + pos] : 0.f, okb ? st[(2 * c + 1) * SL + pos] : 0.f);
-  });
+  sfft_for_inputs<L, false>(t, [&](int slot, int pos) { v[slot] = make_float2(ra[pos], rb[pos]); });
   __syncthreads();
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, false, -1, 9>(v, t, row, addr, a.fft.stw);
-  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(pos)] = v[slot]; });
+  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(t, pos - t)] = v[slot]; });
   __syncthreads();
-  // Hermitian split, bin-contiguous over the workgroup's rows
-  float2* dst = a.dst + r0 * a.dst_row;
-  constexpr int IT = (MAXR * NB + NT - 1) / NT;
-  const int n = nr * NB;
-#pragma unroll
-  for (int j = 0; j < IT; ++j) {
-    const int i = threadIdx.x + j * NT;
-    if (i < n) {
-      const int r = i / NB, kb = i - r * NB;
-      const float2* pr = lds + (r >> 1) * LP;
-      const float2 Z = pr[addr(kb)];
-      const float2 Zm = pr[addr(kb == 0 ? 0 : L - kb)];
-      dst[r * a.dst_row + kb] = (r & 1) ? make_float2(0.5f * (Z.y + Zm.y), 0.5f * (Zm.x - Z.x))
-                                        : make_float2(0.5f * (Z.x + Zm.x), 0.5f * (Z.y - Zm.y));
-    }
-  }
+  XBins<L, PAIRS>().store(a.dst + r0 * a.dst_row, a.dst_row, nr, lds);
 }
 
 // C2R of up to 2*PAIRS spectrum rows into dense real rows
 template <int L, int PAIRS>
 __device__ __forceinline__ void xinv_flat_body(const XPassArgs& a, long blk, float2* lds) {
   using P = PlanOf<L, false>;
-  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL, NB = XStage<L>::NB;
+  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL;
   constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
   const long r0 = 2 * blk * PAIRS;
   if (r0 >= a.nrows) return;  // whole workgroup
   const int nr = a.nrows - r0 < MAXR ? (int)(a.nrows - r0) : MAXR;
-  xflat_load_bins<L, NT, MAXR>(a.csrc + r0 * a.src_row, a.src_row, lds, nr);
+  XBins<L, PAIRS>().load(a.csrc + r0 * a.src_row, a.src_row, nr, lds);
   __syncthreads();
   const int t = threadIdx.x % T, c = threadIdx.x / T;
-  const bool oka = 2 * c < nr, okb = 2 * c + 1 < nr;
-  const float2* sa = lds + 2 * c * NB;
-  const float2* sb = sa + NB;
   float2 v[P::MAXE()];
-  // Z = A' + iB' over all L positions; position L - kb takes the conjugates
-  sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
-    const bool mirror = pos >= NB;
-    const int kb = mirror ? L - pos : pos;
-    float2 A = oka ? sa[kb] : make_float2(0.f, 0.f);
-    float2 B = okb ? sb[kb] : make_float2(0.f, 0.f);
-    if (kb == 0 || 2 * kb == L) {
-      A.y = 0.f;
-      B.y = 0.f;
-    }
-    if (mirror) {
-      A.y = -A.y;
-      B.y = -B.y;
-    }
-    v[slot] = make_float2(A.x - B.y, A.y + B.x);
-  });
+  const float2* in = lds + c * LP;
+  sfft_for_inputs<L, false>(t, [&](int slot, int pos) { v[slot] = in[XRow<L>::at(t, pos - t)]; });
   __syncthreads();
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, false, +1>(v, t, row, addr, a.fft.stw);
   // sfft_run ends on a barrier after its last LDS read
   float* st = reinterpret_cast<float*>(lds);
@@ -564,37 +669,21 @@ template <int L, int PAIRS>
 __global__ void __launch_bounds__(PAIRS * threads_per_transform<L>())
 sk_xinv_crop_flat(XPassArgs a) {
   using P = PlanOf<L, false>;
-  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL, NB = XStage<L>::NB;
+  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL;
   constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
   static_assert(xflat_lds_floats<L>(PAIRS) * 4 <= 65536, "flat x pass LDS");
   __shared__ float2 lds[xflat_lds_floats<L>(PAIRS) / 2];
   const long r0 = 2 * (long)blockIdx.x * PAIRS;
   const int nr = a.nrows - r0 < MAXR ? (int)(a.nrows - r0) : MAXR;
-  xflat_load_bins<L, NT, MAXR>(a.csrc + r0 * a.src_row, a.src_row, lds, nr);
+  XBins<L, PAIRS>().load(a.csrc + r0 * a.src_row, a.src_row, nr, lds);
   __syncthreads();
   const int t = threadIdx.x % T, c = threadIdx.x / T;
-  const bool oka = 2 * c < nr, okb = 2 * c + 1 < nr;
-  const float2* sa = lds + 2 * c * NB;
-  const float2* sb = sa + NB;
   float2 v[P::MAXE()];
-  sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
-    const bool mirror = pos >= NB;
-    const int kb = mirror ? L - pos : pos;
-    float2 A = oka ? sa[kb] : make_float2(0.f, 0.f);
-    float2 B = okb ? sb[kb] : make_float2(0.f, 0.f);
-    if (kb == 0 || 2 * kb == L) {
-      A.y = 0.f;
-      B.y = 0.f;
-    }
-    if (mirror) {
-      A.y = -A.y;
-      B.y = -B.y;
-    }
-    v[slot] = make_float2(A.x - B.y, A.y + B.x);
-  });
+  const float2* in = lds + c * LP;
+  sfft_for_inputs<L, false>(t, [&](int slot, int pos) { v[slot] = in[XRow<L>::at(t, pos - t)]; });
   __syncthreads();
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, false, +1>(v, t, row, addr, a.fft.stw);
   float* st = reinterpret_cast<float*>(lds);
   sfft_for_outputs<L, false>(t, [&](int slot, int pos) {
@@ -629,7 +718,7 @@ __device__ __forceinline__ int run_row(int i, float inv_n) { return (int)(((floa
 template <int L, int PAIRS>
 __device__ __forceinline__ void xfwd_ext_body(const XExtArgs& a, long blk, float2* lds) {
   using P = PlanOf<L, false>;
-  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL, NB = XStage<L>::NB;
+  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL;
   constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
   const unsigned z = (unsigned)blk / (unsigned)a.groups;
   const int r0 = 2 * PAIRS * (int)((unsigned)blk - z * (unsigned)a.groups);
@@ -662,35 +751,21 @@ __device__ __forceinline__ void xfwd_ext_body(const XExtArgs& a, long blk, float
   }
   __syncthreads();
   const int t = threadIdx.x % T, c = threadIdx.x / T;
-  const bool oka = 2 * c < nr, okb = 2 * c + 1 < nr;
+  const float* ra = st + 2 * c * SL;  // missing rows as in xfwd_flat_body
+  const float* rb = ra + (2 * c + 1 < nr ? SL : 0);
   float2 v[P::MAXE()];
   sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
     const int q = pos < n ? pos : axis_ext_src(e, L, pos);
-    const bool in = q >= 0;
-    v[slot] = make_float2(in && oka ? st[2 * c * SL + q] : 0.f,
-                          in && okb ? st[(2 * c + 1) * SL + q] : 0.f);
+    v[slot] = q >= 0 ? make_float2(ra[q], rb[q]) : make_float2(0.f, 0.f);
   });
   __syncthreads();
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, false, -1, 9>(v, t, row, addr, a.m.fft.stw);
-  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(pos)] = v[slot]; });
+  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(t, pos - t)] = v[slot]; });
   __syncthreads();
-  float2* dst = a.m.dst + (long)z * a.spec_plane + (long)r0 * a.m.dst_row;
-  constexpr int IT = (MAXR * NB + NT - 1) / NT;
-  const int nbins = nr * NB;
-#pragma unroll
-  for (int j = 0; j < IT; ++j) {
-    const int i = threadIdx.x + j * NT;
-    if (i < nbins) {
-      const int r = i / NB, kb = i - r * NB;
-      const float2* pr = lds + (r >> 1) * LP;
-      const float2 Z = pr[addr(kb)];
-      const float2 Zm = pr[addr(kb == 0 ? 0 : L - kb)];
-      dst[r * a.m.dst_row + kb] = (r & 1) ? make_float2(0.5f * (Z.y + Zm.y), 0.5f * (Zm.x - Z.x))
-                                          : make_float2(0.5f * (Z.x + Zm.x), 0.5f * (Z.y - Zm.y));
-    }
-  }
+  XBins<L, PAIRS>().store(a.m.dst + (long)z * a.spec_plane + (long)r0 * a.m.dst_row, a.m.dst_row, nr,
+                          lds);
 }
 
 template <int L, int PAIRS>
@@ -708,40 +783,22 @@ template <int L, int PAIRS>
 __global__ void __launch_bounds__(PAIRS * threads_per_transform<L>())
 sk_xinv_ext(XExtArgs a) {
   using P = PlanOf<L, false>;
-  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL, NB = XStage<L>::NB;
+  constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL;
   constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
   static_assert(xflat_lds_floats<L>(PAIRS) * 4 <= 65536, "flat x pass LDS");
   __shared__ float2 lds[xflat_lds_floats<L>(PAIRS) / 2];
   const unsigned z = blockIdx.x / (unsigned)a.groups;
   const int r0 = 2 * PAIRS * (int)(blockIdx.x - z * (unsigned)a.groups);
   const int nr = a.ny - r0 < MAXR ? a.ny - r0 : MAXR;
-  xflat_load_bins<L, NT, MAXR>(a.m.csrc + (long)z * a.spec_plane + (long)r0 * a.m.src_row,
-                               a.m.src_row, lds, nr);
+  XBins<L, PAIRS>().load(a.m.csrc + (long)z * a.spec_plane + (long)r0 * a.m.src_row, a.m.src_row, nr, lds);
   __syncthreads();
   const int t = threadIdx.x % T, c = threadIdx.x / T;
-  const bool oka = 2 * c < nr, okb = 2 * c + 1 < nr;
-  const float2* sa = lds + 2 * c * NB;
-  const float2* sb = sa + NB;
   float2 v[P::MAXE()];
-  // Z = A' + iB' over all L positions; position L - kb takes the conjugates
-  sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
-    const bool mirror = pos >= NB;
-    const int kb = mirror ? L - pos : pos;
-    float2 A = oka ? sa[kb] : make_float2(0.f, 0.f);
-    float2 B = okb ? sb[kb] : make_float2(0.f, 0.f);
-    if (kb == 0 || 2 * kb == L) {
-      A.y = 0.f;
-      B.y = 0.f;
-    }
-    if (mirror) {
-      A.y = -A.y;
-      B.y = -B.y;
-    }
-    v[slot] = make_float2(A.x - B.y, A.y + B.x);
-  });
+  const float2* in = lds + c * LP;
+  sfft_for_inputs<L, false>(t, [&](int slot, int pos) { v[slot] = in[XRow<L>::at(t, pos - t)]; });
   __syncthreads();
   float2* row = lds + c * LP;
-  auto addr = [&](int pos) { return XRow<L>::at(pos); };
+  const XAddr addr;
   sfft_run<L, false, +1>(v, t, row, addr, a.m.fft.stw);
   // sfft_run ends on a barrier after its last LDS read
   float* st = reinterpret_cast<float*>(lds);
