@@ -365,7 +365,7 @@ void rl_launch_zsum(const RLZArgs& a, long ny, hipStream_t st) {
 template <int L>
 void rl_launch_xratio(const RLXArgs& a, int nviews, hipStream_t st) {
   if (FC_RL_XFLAT && a.rrow == L) {
-    constexpr int P = flat_pairs<L, 256>();
+    constexpr int P = flat_fill_pairs<L>();
     const long groups = ((a.nrows + 1) / 2 + P - 1) / P;
     hipLaunchKernelGGL((sk_xratio_flat<L, P>), dim3((unsigned)(groups * nviews)),
                        dim3(P * threads_per_transform<L>()), 0, st, a);
@@ -380,7 +380,7 @@ void rl_launch_xratio(const RLXArgs& a, int nviews, hipStream_t st) {
 template <int L>
 void rl_launch_xupdate(const RLXArgs& a, hipStream_t st) {
   if (FC_RL_XFLAT && a.rrow == L) {
-    constexpr int P = flat_pairs<L, 256>();
+    constexpr int P = flat_fill_pairs<L>();
     const long groups = ((a.nrows + 1) / 2 + P - 1) / P;
     hipLaunchKernelGGL((sk_xupdate_flat<L, P>), dim3((unsigned)groups),
                        dim3(P * threads_per_transform<L>()), 0, st, a);

@@ -342,6 +342,25 @@ constexpr int flat_pairs() {
   return p;
 }
 
+// Row pairs of a flat x-pass workgroup of 96 to 256 threads: the fewest whose
+// threads fill their wavefronts to within 8 % of the best (T = 45 at 540: two
+// pairs leave 30 % of the lanes idle, four 6 %: x inverse of 512 x 512 x 256
+// with a zero boundary 124 us at two pairs, 116 at five).
+template <int L>
+constexpr int flat_fill_pairs() {
+  constexpr int T = threads_per_transform<L>();
+  auto fits = [](int p) {
+    return p * T <= (T > 256 ? T : 256) && xflat_lds_floats<L>(p) * 4 <= 65536;
+  };
+  auto fill = [](int p) { return (double)(p * T) / ((p * T + 63) / 64 * 64); };
+  double best = 0;
+  for (int p = 1; fits(p); ++p)
+    if (p * T >= 96 && fill(p) > best) best = fill(p);
+  for (int p = 1; fits(p); ++p)
+    if (p * T >= 96 && fill(p) >= best - 0.08) return p;
+  return flat_pairs<L, 128>();
+}
+
 #ifndef FC_BATCH_XTGT
 #define FC_BATCH_XTGT 256
 #endif
@@ -1495,7 +1514,7 @@ bool sk_launch_xinv_lds(const XPassArgs& a, hipStream_t st) {
 template <int L, int TGT>
 bool sk_launch_xfwd_flat(const XPass2& a, hipStream_t st) {
   if (a.m.nrows > 0 && a.m.src_row != L) return false;
-  constexpr int P = flat_pairs<L, TGT>();
+  constexpr int P = TGT == 128 ? flat_fill_pairs<L>() : flat_pairs<L, TGT>();
   XPass2 b = a;
   b.m_blocks = ((a.m.nrows + 1) / 2 + P - 1) / P;
   b.k_blocks = ((a.k.nrows + 1) / 2 + P - 1) / P;
@@ -1507,7 +1526,7 @@ bool sk_launch_xfwd_flat(const XPass2& a, hipStream_t st) {
 template <int L, int TGT>
 bool sk_launch_xinv_flat(const XPassArgs& a, hipStream_t st) {
   if (a.dst_row != L) return false;
-  constexpr int P = flat_pairs<L, TGT>();
+  constexpr int P = TGT == 128 ? flat_fill_pairs<L>() : flat_pairs<L, TGT>();
   const long blocks = ((a.nrows + 1) / 2 + P - 1) / P;
   hipLaunchKernelGGL((sk_xinv_flat<L, P>), dim3((unsigned)blocks),
                      dim3(P * threads_per_transform<L>()), 0, st, a);
@@ -1587,7 +1606,7 @@ bool sk_launch_zfused_fft(const ZArgs& a, long ny, hipStream_t st) {
 // launchers over an extended image
 template <int L>
 void sk_launch_xfwd_ext(const XExtArgs& a, hipStream_t st) {
-  constexpr int P = flat_pairs<L, 256>();
+  constexpr int P = flat_fill_pairs<L>();
   XExtArgs b = a;
   b.groups = (a.ny + 2 * P - 1) / (2 * P);
   b.k_blocks = ((a.k.nrows + 1) / 2 + P - 1) / P;
@@ -1596,7 +1615,7 @@ void sk_launch_xfwd_ext(const XExtArgs& a, hipStream_t st) {
 }
 template <int L>
 void sk_launch_xinv_ext(const XExtArgs& a, hipStream_t st) {
-  constexpr int P = flat_pairs<L, 256>();
+  constexpr int P = flat_fill_pairs<L>();
   XExtArgs b = a;
   b.groups = (a.ny + 2 * P - 1) / (2 * P);
   hipLaunchKernelGGL((sk_xinv_ext<L, P>), dim3((unsigned)(b.groups * a.nplanes)),
@@ -1726,16 +1745,17 @@ StaticEntry make_static_entry() {
               {"t8-fft", &sk_launch_zfused_fft<L, 8>},
               {"t32-fft", &sk_launch_zfused_fft<L, 32>},
               {"t64-fft", &sk_launch_zfused_fft<L, 64>}};
-  // defaults (measured over (512, 1024, L) volumes): the flat x inverse at
-  // every length; the flat x forward where rows are short or not a whole
-  // number of float4s, the per-pair forward elsewhere
+  // defaults: the flat forms at about 128 threads (measured over L x 300 x 96
+  // volumes: x forward at 384 23.0 us w256, 21.2 w256-flat, 20.4 w128-flat;
+  // at 1024 53.8, 47.7, 46.4; x inverse at 384 21.3, 20.6, 19.5; at 128 to 216
+  // w64 is 0.3 to 0.7 us of 15 faster forward)
   auto index_of = [](const auto& vs, const char* name) {
     for (size_t i = 0; i < vs.size(); ++i)
       if (__builtin_strcmp(vs[i].name, name) == 0) return (int)i;
     return 0;
   };
-  e.selected[kSxInv] = index_of(e.xinv, "w256-flat");
-  if (L < 128 || L % 4 != 0) e.selected[kSxFwd] = index_of(e.xfwd, "w256-flat");
+  e.selected[kSxInv] = index_of(e.xinv, "w128-flat");
+  e.selected[kSxFwd] = index_of(e.xfwd, "w128-flat");
   e.xfwd_vpad = &sk_launch_xfwd_vpad<L, 64>;
   e.xinv_crop = &sk_launch_xinv_crop_flat<L, 256>;  // 171 vs 193 us at 600 x 600 x 288
   e.ext.xfwd = &sk_launch_xfwd_ext<L>;
