@@ -290,8 +290,7 @@ struct RLXArgs {
   FftDesc fft;  // length nx
   long nrows;
   int nbins;
-  long srow;  // spectrum row stride (nxp)
-  long rrow;  // real row stride (nx)
+  long srow;  // spectrum row stride (nxp); real rows are dense
   float eps;
   float inv_views;
   float2* spec[kMaxViews];       // per-view spectra (xratio) / summed spectrum (xupdate: [0])

@@ -188,7 +188,6 @@ void run_rl(const RLProblem& p, float* psi, const float* const* views, const flo
   xa.nrows = (long)s.ny * s.nz;
   xa.nbins = half_bins(s.nx);
   xa.srow = nxp;
-  xa.rrow = s.nx;
   xa.eps = eps;
   xa.inv_views = 1.f / (float)p.V;
   for (int v = 0; v < p.V; ++v) {

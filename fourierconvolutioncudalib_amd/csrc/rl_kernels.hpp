@@ -12,8 +12,6 @@
 //                IFFTz (correlations add in the spectral domain)
 //   sk_xupdate   x-C2R of the summed correlation with the epilogue
 //                psi <- psi * acc / V
-// (the x kernels also in flat forms, staging the workgroup's rows through
-// LDS with coalesced HBM access; used when the real rows are dense)
 #pragma once
 
 #include <type_traits>
@@ -91,7 +89,10 @@ sk_zfan(RLZArgs a) {
   }
 }
 
-template <int L, int TX, int H>
+// The taps' columns are taken whole: constant zero slots (H as in sk_zfan)
+// spread the live registers of the two transforms and cost spills, 212 us
+// against 202 for four views of 384 x 384 x 192 with 51 taps.
+template <int L, int TX>
 __global__ void FC_RL_BOUNDS(TX * threads_per_transform<L>(), FC_RL_ZSUM_WAVES)
 sk_zsum(RLZArgs a) {
   using P = PlanOf<L, false>;
@@ -114,7 +115,7 @@ sk_zsum(RLZArgs a) {
       if (ok) val = col_at(in_t, pos, t, a.s_plane);
       X[slot] = val;
     });
-    load_kernel_taps<L, H>(W, t, ok, a.kplanes[v] + base, a.s_plane, a.kz[v], a.cz[v]);
+    load_kernel_taps<L, 0>(W, t, ok, a.kplanes[v] + base, a.s_plane, a.kz[v], a.cz[v]);
     sfft_run<L, false, -1>(X, t, lds, addr, a.fft.stw);
     sfft_run<L, false, -1>(W, t, lds, addr, a.fft.stw);
     sfft_for_outputs<L, false>(t, [&](int slot, int) { acc[slot] = cadd(acc[slot], cmulc(X[slot], W[slot])); });
@@ -125,119 +126,12 @@ sk_zsum(RLZArgs a) {
   if (ok) sfft_for_outputs<L, true>(t, [&](int slot, int pos) { col_at(out_t, pos, t, a.s_plane) = acc[slot]; });
 }
 
-// x-C2R (reversed plan: its outputs sit exactly at the forward plan's
-// stage-0 input positions), ratio, x-R2C (forward plan), separation.
-template <int L, int PAIRS>
-__global__ void __launch_bounds__(PAIRS * threads_per_transform<L>())
-sk_xratio(RLXArgs a) {
-  using P = PlanOf<L, false>;
-  constexpr int T = P::T, LP = XRow<L>::LP;
-  __shared__ float2 lds[PAIRS * LP];
-  const long groups = ((a.nrows + 1) / 2 + PAIRS - 1) / PAIRS;
-  const int v = (int)(blockIdx.x / groups);
-  const long blk = blockIdx.x - (long)v * groups;
-  const int t = threadIdx.x % T, c = threadIdx.x / T;
-  const long ra = 2 * (blk * PAIRS + c), rb = ra + 1;
-  const bool oka = ra < a.nrows, okb = rb < a.nrows;
-  float2* pa = a.spec[v] + ra * a.srow;
-  float2* pb = a.spec[v] + rb * a.srow;
-  const int nb = a.nbins;
-  float2 z[P::MAXE()];
-  sfft_for_inputs<L, true>(t, [&](int slot, int pos) {
-    const bool mirror = pos >= nb;
-    const int kb = mirror ? L - pos : pos;
-    float2 A = make_float2(0.f, 0.f), B = make_float2(0.f, 0.f);
-    if (oka) A = pa[kb];
-    if (okb) B = pb[kb];
-    if (kb == 0 || 2 * kb == L) {
-      A.y = 0.f;
-      B.y = 0.f;
-    }
-    if (mirror) {
-      A.y = -A.y;
-      B.y = -B.y;
-    }
-    z[slot] = make_float2(A.x - B.y, A.y + B.x);
-  });
-  float2* row = lds + c * LP;
-  const XAddr addr;
-  sfft_run<L, true, +1>(z, t, row, addr, a.fft.stw);
-  // real rows of the blurred estimate -> ratio rows (same positions)
-  const float* fa = a.phi[v] + ra * a.rrow;
-  const float* fb = a.phi[v] + rb * a.rrow;
-  const float eps = a.eps;
-  auto ratio = [&](auto fast) {
-    sfft_for_outputs<L, true>(t, [&](int slot, int pos) {
-      float ya = 0.f, yb = 0.f;
-      constexpr bool F = decltype(fast)::value;
-      if (oka) ya = rl_div<F>(fa[pos], fmaxf(z[slot].x, eps));
-      if (okb) yb = rl_div<F>(fb[pos], fmaxf(z[slot].y, eps));
-      z[slot] = make_float2(ya, yb);
-    });
-  };
-  if (eps >= kMinNormal)
-    ratio(std::true_type{});
-  else
-    ratio(std::false_type{});
-  sfft_run<L, false, -1>(z, t, row, addr, a.fft.stw);
-  sfft_for_outputs<L, false>(t, [&](int slot, int pos) { row[addr(t, pos - t)] = z[slot]; });
-  __syncthreads();
-  for (int kb = t; kb < nb; kb += T) {
-    const float2 Z = row[addr(kb)];
-    const float2 Zm = row[addr(kb == 0 ? 0 : L - kb)];
-    if (oka) pa[kb] = make_float2(0.5f * (Z.x + Zm.x), 0.5f * (Z.y - Zm.y));
-    if (okb) pb[kb] = make_float2(0.5f * (Z.y + Zm.y), 0.5f * (Zm.x - Z.x));
-  }
-}
-
-template <int L, int PAIRS>
-__global__ void __launch_bounds__(PAIRS * threads_per_transform<L>())
-sk_xupdate(RLXArgs a) {
-  using P = PlanOf<L, false>;
-  constexpr int T = P::T, LP = XRow<L>::LP;
-  __shared__ float2 lds[PAIRS * LP];
-  const int t = threadIdx.x % T, c = threadIdx.x / T;
-  const long ra = 2 * ((long)blockIdx.x * PAIRS + c), rb = ra + 1;
-  const bool oka = ra < a.nrows, okb = rb < a.nrows;
-  const float2* pa = a.spec[0] + ra * a.srow;
-  const float2* pb = a.spec[0] + rb * a.srow;
-  const int nb = a.nbins;
-  float2 z[P::MAXE()];
-  sfft_for_inputs<L, false>(t, [&](int slot, int pos) {
-    const bool mirror = pos >= nb;
-    const int kb = mirror ? L - pos : pos;
-    float2 A = make_float2(0.f, 0.f), B = make_float2(0.f, 0.f);
-    if (oka) A = pa[kb];
-    if (okb) B = pb[kb];
-    if (kb == 0 || 2 * kb == L) {
-      A.y = 0.f;
-      B.y = 0.f;
-    }
-    if (mirror) {
-      A.y = -A.y;
-      B.y = -B.y;
-    }
-    z[slot] = make_float2(A.x - B.y, A.y + B.x);
-  });
-  float2* row = lds + c * LP;
-  const XAddr addr;
-  sfft_run<L, false, +1>(z, t, row, addr, a.fft.stw);
-  float* qa = a.psi + ra * a.rrow;
-  float* qb = a.psi + rb * a.rrow;
-  const float iv = a.inv_views;
-  sfft_for_outputs<L, false>(t, [&](int slot, int pos) {
-    if (oka) qa[pos] = qa[pos] * z[slot].x * iv;
-    if (okb) qb[pos] = qb[pos] * z[slot].y * iv;
-  });
-}
-
-// Flat forms of the two x kernels: the workgroup's spectrum rows and real
-// rows (phi, psi) move between HBM and LDS staging as coalesced runs, as in
-// the flat x passes (xflat_* in static_kernels_impl.hpp).  Real rows must be
-// dense (rrow == L).
+// The x kernels move the workgroup's spectrum rows and real rows (phi, psi)
+// between HBM and LDS staging as coalesced runs, as the flat x passes do
+// (xflat_* in static_kernels_impl.hpp).  The real rows are dense.
 template <int L, int PAIRS>
 __global__ void FC_RL_BOUNDS(PAIRS * threads_per_transform<L>(), FC_RL_XRATIO_WAVES)
-sk_xratio_flat(RLXArgs a) {
+sk_xratio(RLXArgs a) {
   using P = PlanOf<L, false>;
   constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL;
   constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
@@ -286,7 +180,7 @@ sk_xratio_flat(RLXArgs a) {
 
 template <int L, int PAIRS>
 __global__ void __launch_bounds__(PAIRS * threads_per_transform<L>())
-sk_xupdate_flat(RLXArgs a) {
+sk_xupdate(RLXArgs a) {
   using P = PlanOf<L, false>;
   constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL;
   constexpr int NT = PAIRS * T, MAXR = 2 * PAIRS;
@@ -316,10 +210,6 @@ sk_xupdate_flat(RLXArgs a) {
   __syncthreads();
   xflat_store_rows<L, NT, MAXR>(psi, st, nr);
 }
-
-#ifndef FC_RL_XFLAT
-#define FC_RL_XFLAT 1
-#endif
 
 // calls f with the pruned tap slots that hold every view's kernel
 template <int L, class F>
@@ -354,24 +244,13 @@ void rl_launch_zsum(const RLZArgs& a, long ny, hipStream_t st) {
   constexpr int TX = fit_tile<L, 16, kTileLdsZ>();
   RLZArgs b = a;
   b.ny = ny;
-  rl_with_slots<L>(a, [&](auto h) {
-    hipLaunchKernelGGL((sk_zsum<L, TX, decltype(h)::value>),
-                       dim3((unsigned)column_tiles(a.nbins, TX, ny)),
-                       dim3(TX * threads_per_transform<L>()), 0, st, b);
-  });
+  hipLaunchKernelGGL((sk_zsum<L, TX>), dim3((unsigned)column_tiles(a.nbins, TX, ny)),
+                     dim3(TX * threads_per_transform<L>()), 0, st, b);
 }
 
-// the flat forms need dense real rows; the per-pair forms take any stride
 template <int L>
 void rl_launch_xratio(const RLXArgs& a, int nviews, hipStream_t st) {
-  if (FC_RL_XFLAT && a.rrow == L) {
-    constexpr int P = flat_fill_pairs<L>();
-    const long groups = ((a.nrows + 1) / 2 + P - 1) / P;
-    hipLaunchKernelGGL((sk_xratio_flat<L, P>), dim3((unsigned)(groups * nviews)),
-                       dim3(P * threads_per_transform<L>()), 0, st, a);
-    return;
-  }
-  constexpr int P = fit_pairs<L, pairs_for<L, 256>()>();
+  constexpr int P = flat_fill_pairs<L>();
   const long groups = ((a.nrows + 1) / 2 + P - 1) / P;
   hipLaunchKernelGGL((sk_xratio<L, P>), dim3((unsigned)(groups * nviews)),
                      dim3(P * threads_per_transform<L>()), 0, st, a);
@@ -379,17 +258,10 @@ void rl_launch_xratio(const RLXArgs& a, int nviews, hipStream_t st) {
 
 template <int L>
 void rl_launch_xupdate(const RLXArgs& a, hipStream_t st) {
-  if (FC_RL_XFLAT && a.rrow == L) {
-    constexpr int P = flat_fill_pairs<L>();
-    const long groups = ((a.nrows + 1) / 2 + P - 1) / P;
-    hipLaunchKernelGGL((sk_xupdate_flat<L, P>), dim3((unsigned)groups),
-                       dim3(P * threads_per_transform<L>()), 0, st, a);
-    return;
-  }
-  constexpr int P = fit_pairs<L, pairs_for<L, 256>()>();
+  constexpr int P = flat_fill_pairs<L>();
   const long groups = ((a.nrows + 1) / 2 + P - 1) / P;
-  hipLaunchKernelGGL((sk_xupdate<L, P>), dim3((unsigned)groups), dim3(P * threads_per_transform<L>()),
-                     0, st, a);
+  hipLaunchKernelGGL((sk_xupdate<L, P>), dim3((unsigned)groups),
+                     dim3(P * threads_per_transform<L>()), 0, st, a);
 }
 
 }  // namespace fcamd
