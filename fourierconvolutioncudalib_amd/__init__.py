@@ -15,6 +15,7 @@ Volumes are C-order ``[nz, ny, nx]`` arrays.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 
 import numpy as np
@@ -145,7 +146,11 @@ def convolve(image, kernel, op=CONVOLVE, dev=0):
 
 def workspace_bytes(image_shape, kernel_shape):
     """Device workspace for one convolution of C-order shapes (z, y, x)."""
-    n = lib().fcamd_workspace_bytes(ints(tuple(image_shape)[::-1]), ints(tuple(kernel_shape)[::-1]))
+    return _checked_bytes(lib().fcamd_workspace_bytes(ints(tuple(image_shape)[::-1]),
+                                                      ints(tuple(kernel_shape)[::-1])))
+
+
+def _checked_bytes(n):
     if n < 0:
         _raise_if_failed()
     return int(n)
@@ -200,9 +205,9 @@ def _check_tensor(t, name, shape=None, device=None, contiguous=True):
         raise TypeError(f"{name} must be float32, got {t.dtype}")
     if not t.is_cuda:
         raise TypeError(f"{name} must be a CUDA tensor (there is no CPU path)")
-    if device is not None and t.device != torch.device(device):
+    if device is not None and t.device != device and t.device != torch.device(device):
         raise ValueError(f"{name} is on {t.device}, expected {device}")
-    if shape is not None and tuple(t.shape) != tuple(int(d) for d in shape):
+    if shape is not None and t.shape != shape and tuple(t.shape) != tuple(int(d) for d in shape):
         raise ValueError(f"{name} has shape {tuple(t.shape)}, expected {tuple(shape)}")
     if contiguous and not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
@@ -234,10 +239,24 @@ def _workspace(nbytes, workspace, device, stream):
     return ws.data_ptr(), int(nbytes), ws
 
 
+# A small call is bound by its host work: 64 x 64 x 64 with a 7 x 7 x 7 kernel
+# took 21.8 us of it and runs 16.5 us on the device.  Without a Stream object to
+# ask for the current stream's handle, a switch to the device that is current
+# and a second set of dims it takes 16.8 (a call on its own 38.3 -> 33).
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def _on_device(device):
+    import torch
+    if device.index == torch.cuda.current_device():
+        return _SAME_DEVICE
+    return torch.cuda.device(device)
+
+
 def _stream_handle(stream):
     if stream is None:
         import torch
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
     if isinstance(stream, int):
         return ctypes.c_void_p(stream)
     return ctypes.c_void_p(stream.cuda_stream)
@@ -264,7 +283,7 @@ class ConvolutionPlan:
         if workspace is not None:
             wptr, wbytes, _ = _workspace(workspace_bytes(self.image_shape, self.kernel_shape),
                                          workspace, self.device, stream)
-        with torch.cuda.device(self.device):
+        with _on_device(self.device):
             self._plan = lib().fcamd_conv_plan_create(
                 ints(self.image_shape[::-1]), ints(self.kernel_shape[::-1]),
                 self._kernel.data_ptr(), int(op), wptr, wbytes, _stream_handle(stream))
@@ -276,7 +295,7 @@ class ConvolutionPlan:
         _check_tensor(kernel, "kernel", self.kernel_shape, self.device, contiguous=False)
         import torch
         self._kernel = kernel.contiguous()
-        with torch.cuda.device(self.device):
+        with _on_device(self.device):
             check(lib().fcamd_conv_plan_set_kernel(self._plan, self._kernel.data_ptr(),
                                                    _stream_handle(stream)))
 
@@ -288,7 +307,7 @@ class ConvolutionPlan:
         if out is None:
             out = torch.empty_like(image)
         _check_tensor(out, "out", self.image_shape, self.device)
-        with torch.cuda.device(self.device):
+        with _on_device(self.device):
             check(lib().fcamd_conv_plan_execute(self._plan, out.data_ptr(), image.data_ptr(),
                                                 _stream_handle(stream)))
         return out
@@ -355,7 +374,7 @@ def convolve3d_boundary(image, kernel, boundary="zero", op=CONVOLVE, out=None, w
     _check_tensor(out, "out", image.shape, image.device)
     need = boundary_workspace_bytes(image.shape, kernel.shape, boundary)
     wptr, wbytes, _keep = _workspace(need, workspace, image.device, stream)
-    with torch.cuda.device(image.device):
+    with _on_device(image.device):
         check(lib().fcamd_convolve3d_boundary_device(
             out.data_ptr(), image.data_ptr(), ints(image.shape[::-1]),
             kernel.data_ptr(), ints(kernel.shape[::-1]), int(op), _boundary_code(boundary),
@@ -381,11 +400,11 @@ def convolve3d(image, kernel, op=CONVOLVE, out=None, workspace=None, stream=None
     if out is None:
         out = torch.empty_like(image)
     _check_tensor(out, "out", image.shape, image.device)
-    need = workspace_bytes(image.shape, kernel.shape)
+    dims, kdims = ints(image.shape[::-1]), ints(kernel.shape[::-1])
+    need = _checked_bytes(lib().fcamd_workspace_bytes(dims, kdims))
     wptr, wbytes, _keep = _workspace(need, workspace, image.device, stream)
-    with torch.cuda.device(image.device):
+    with _on_device(image.device):
         check(lib().fcamd_convolve3d_device(
-            out.data_ptr(), image.data_ptr(), ints(image.shape[::-1]),
-            kernel.data_ptr(), ints(kernel.shape[::-1]), int(op),
+            out.data_ptr(), image.data_ptr(), dims, kernel.data_ptr(), kdims, int(op),
             wptr, wbytes, _stream_handle(stream)))
     return out

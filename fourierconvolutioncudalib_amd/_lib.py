@@ -120,6 +120,9 @@ def check(rc: int) -> None:
         raise FCError(rc, msg.decode() if msg else "unknown error")
 
 
+_INT3 = ctypes.c_int * 3
+
+
 def ints(values):
     values = [int(v) for v in values]
-    return (ctypes.c_int * len(values))(*values)
+    return (_INT3 if len(values) == 3 else ctypes.c_int * len(values))(*values)
