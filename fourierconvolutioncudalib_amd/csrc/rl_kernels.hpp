@@ -20,23 +20,22 @@
 
 namespace fcamd {
 
-// minimum waves per SIMD asked of the two register-heaviest kernels (0: no
-// request; the compiler then sizes registers for the code alone).  4 waves
-// (the most their LDS allows) took the 10-iteration, 4-view 384 x 384 x 192
-// run from 15.34 to 15.04 ms, although the ratio kernel then spills 8
-// registers.
-#ifndef FC_RL_XRATIO_WAVES
-#define FC_RL_XRATIO_WAVES 4
-#endif
-#ifndef FC_RL_ZSUM_WAVES
-#define FC_RL_ZSUM_WAVES 4
-#endif
-#define FC_RL_BOUNDS_0(n) __launch_bounds__(n)
-#define FC_RL_BOUNDS_3(n) __launch_bounds__(n, 3)
-#define FC_RL_BOUNDS_4(n) __launch_bounds__(n, 4)
-#define FC_RL_BOUNDS_5(n) __launch_bounds__(n, 5)
-#define FC_RL_BOUNDS_CAT(n, w) FC_RL_BOUNDS_##w(n)
-#define FC_RL_BOUNDS(n, w) FC_RL_BOUNDS_CAT(n, w)
+// Waves per SIMD asked of the ratio kernel: 4, the most its LDS allows, took
+// the 10-iteration, 4-view 384 x 384 x 192 run from 15.34 to 15.04 ms.
+constexpr int kRatioWaves = 4;
+// and of the sum over views, which holds three columns of MAXE float2 (sum,
+// view, kernel) and some 30 registers more: as many as that leaves room for.
+// Four at every length spilled 130 registers at 384, 127 at 80, 200 at 112 and
+// 50 at 600; three views of 256 x 192 x z with 15 taps, us, before and after:
+// z = 80 54.7 / 37.8, 112 84.6 / 43.2, 384 255 / 175, 600 413 (8-bin tiles; 443
+// with 16-bin ones) / 244, 432 178 / 177.
+template <int L, int TX>
+constexpr int zsum_waves() {
+  constexpr int regs = 6 * PlanOf<L, false>::MAXE() + 30;
+  constexpr int wg = (TX * threads_per_transform<L>() + 63) / 64;  // its waves
+  // (of 9 to 12 waves one workgroup fits either way)
+  return regs <= 128 && (wg <= 8 || wg > 12) ? 4 : regs <= 168 ? 3 : 2;
+}
 
 // phi / d for d = max(blur, eps) > 0.  With eps a normal number (the
 // launch-uniform case FAST) every d is one, and the hardware reciprocal (at
@@ -93,7 +92,7 @@ sk_zfan(RLZArgs a) {
 // spread the live registers of the two transforms and cost spills, 212 us
 // against 202 for four views of 384 x 384 x 192 with 51 taps.
 template <int L, int TX>
-__global__ void FC_RL_BOUNDS(TX * threads_per_transform<L>(), FC_RL_ZSUM_WAVES)
+__global__ void __launch_bounds__(TX * threads_per_transform<L>(), (zsum_waves<L, TX>()))
 sk_zsum(RLZArgs a) {
   using P = PlanOf<L, false>;
   __shared__ float2 lds[L * TX];
@@ -130,7 +129,7 @@ sk_zsum(RLZArgs a) {
 // between HBM and LDS staging as coalesced runs, as the flat x passes do
 // (xflat_* in static_kernels_impl.hpp).  The real rows are dense.
 template <int L, int PAIRS>
-__global__ void FC_RL_BOUNDS(PAIRS * threads_per_transform<L>(), FC_RL_XRATIO_WAVES)
+__global__ void __launch_bounds__(PAIRS * threads_per_transform<L>(), kRatioWaves)
 sk_xratio(RLXArgs a) {
   using P = PlanOf<L, false>;
   constexpr int T = P::T, LP = XRow<L>::LP, SL = XStage<L>::SL;
