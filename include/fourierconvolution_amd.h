@@ -59,9 +59,9 @@ FCAMD_API int fcamd_convolve3d_device(float* d_out, const float* d_image, const 
  * graph capture, tight serving loops, harnesses that forbid allocation.  The
  * workspace and the twiddle tables live in one device array of the library,
  * FCAMD_NOALLOC_MAX_WORKSPACE bytes of workspace plus 1 MiB of tables, that
- * each device holds until the process ends; a call whose
- * fcamd_workspace_bytes() exceeds FCAMD_NOALLOC_MAX_WORKSPACE fails with code
- * 2 (unsupported size).  The call allocates nothing, so it may be recorded
+ * each device holds until the process ends; a call whose passes at the image's
+ * own extents need more than FCAMD_NOALLOC_MAX_WORKSPACE fails with code 2
+ * (unsupported size).  The call allocates nothing, so it may be recorded
  * into a graph, also for lengths the process has not used before.  Every
  * call on one device shares that array: calls that overlap on one device
  * (other threads, other streams) race; order them.  Same results as
