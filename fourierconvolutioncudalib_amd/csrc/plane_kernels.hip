@@ -65,8 +65,10 @@ bool planes_enabled() {
   return on;
 }
 
+// The kernels transform the image's own plane: one that is extended in x or y
+// (its spectrum has the rows and the pitch of the extended lengths) has none.
 const PlaneEntry* plane_entry(const ConvShape& s) {
-  if (!planes_enabled()) return nullptr;
+  if (!planes_enabled() || s.tx() != s.nx || s.ty() != s.ny) return nullptr;
   for (const PlaneEntry& e : kPlanes)
     if (e.nx == s.nx && e.ny == s.ny) return &e;
   return wide_plane_entry(s.nx, s.ny);
