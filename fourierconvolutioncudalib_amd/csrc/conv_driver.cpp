@@ -434,10 +434,63 @@ ConvShape direct_shape(const ConvShape& s) {
   return d;
 }
 
+namespace {
+// Whether the extended transform (lengths P) of a convolution is faster than
+// the runtime-length kernels it would replace.  What decides, over about 2000
+// shapes timed both ways (x y z here; us runtime -> extended):
+// - the largest prime of the lengths replaced.  Above 31 they run a chirp-z
+//   and the extension gains 1.5 to 15 times, until it multiplies the plane
+//   of a large problem, whose time is then its traffic: 1511 x 2 x 2000 (16
+//   times) 592 -> 655, 509 x 1 x 500 (34 times) 59 -> 75, 3001 x 1 x 2000
+//   602 -> 1257; up to 12 times, or in up to 16 MiB, it gains (509 x 3 x 500
+//   94 -> 75, 509 x 1 x 128 52 -> 33).  A row of one or two bins is padded
+//   to a tile either way, so such planes may grow as their tiles do, to y
+//   columns of 1024 (1 x 509 x 2000 514 -> 431; 1 x 1511 x 2000 1122 -> 1994).
+// - whether y is among them: its columns are what the runtime-length kernels
+//   are slowest at.
+// - the growth of a row in 16-bin column tiles: from one tile to two every y
+//   and z column costs twice, which small problems and small primes do not
+//   earn back.
+bool extension_pays(const ConvShape& s, const int (&P)[3]) {
+  const int n[3] = {s.nx, s.ny, s.nz};
+  int prime = 0;
+  for (int d = 0; d < 3; ++d)
+    if (P[d] != n[d] && n[d] > 1) prime = std::max(prime, largest_prime_factor(n[d]));
+  // (an axis of length 1 runs no transform: 64 x 64 x 1 12.8 -> 13.5)
+  if (prime == 0) return false;
+  const double area = (double)P[0] * P[1] / ((double)s.nx * s.ny);
+  const double row = (double)padded_bins(P[0]) / padded_bins(s.nx);
+  const double plane = row * P[1] / s.ny;  // growth of a plane's spectrum
+  const double mib = (double)padded_bins(P[0]) * P[1] * s.nz * sizeof(float2) / (1 << 20);
+  const bool big = mib > 16;
+  if (prime > kBluesteinPrime) return area <= 12 || !big || (plane <= 4 && P[1] <= 1024);
+  // products of 2, 3, 5 and 7: 252 x 252 x 128 with 15^3 (area x 1.3) 188 ->
+  // 86, with 101 x 101 x 128 (x 2.0) 220 -> 160, with its own size (x 4.1)
+  // 241 -> 278
+  if (prime <= 7 && area > 3) return false;
+  const bool z = P[2] != s.nz && s.nz > 1;
+  if (P[1] != s.ny) {
+    // 13 x 14 x 512 (plane x 4.6) 37 -> 40, 22 x 5 x 512 (x 13) 36 -> 39, 17
+    // x 9 x 512 (x 7.1) 37 -> 39, but 31 x 31 x 31 with its own size (x 6.2)
+    // 76 -> 21 and, the row keeping its tiles, 143 x 5 x 512 (x 6.4) 82 -> 40
+    return prime <= 7 || plane <= 4 || (plane <= 8 && s.nx > 26) ||
+           (P[0] != s.nx && row <= 1.2 && (area <= 12 || mib <= 8)) || mib <= 0.5;
+  }
+  // x or z or both.  36 x 512 x 64 (row x 1.5) 52 -> 66 and 14 x 512 x 64 (x
+  // 2) 40 -> 58, 252 x 128 x 128 with 126^3 (x 1.6) 85 -> 89; 252 x 512 x 64
+  // with 3^3 (x 1.1) 130 -> 107, 20 x 512 x 90 (x 2, but z gains) 1.5 times
+  if (prime <= 7) return row <= 1.2 || (row <= 1.4 && big) || (z && s.nz >= 90);
+  // 13 x 512 x 64 (x 2) 44 -> 58, 22 x 512 x 64 51 -> 58; 104 x 512 x 64
+  // with 52^3 (x 1.5) 108 -> 90
+  if (prime <= 13) return row <= 1.6 || big || (z && s.nz >= 52);
+  // 17 x 512 x 64 (x 2) 53 -> 58; 23 x 64 x 64 28 -> 21, 31 x 512 x 64 1.4
+  return row <= 1.9 || mib >= 16 || s.ny <= 256 || s.nx > 24 || (z && s.nz >= 27);
+}
+}  // namespace
+
 ConvShape with_extension(const ConvShape& s) {
   const int n[3] = {s.nx, s.ny, s.nz}, k[3] = {s.kx, s.ky, s.kz};
   int P[3];
-  bool any = false, smooth = true;
   for (int d = 0; d < 3; ++d) {
     P[d] = n[d];
     if (static_lookup(n[d])) continue;
@@ -446,18 +499,8 @@ ConvShape with_extension(const ConvShape& s) {
     if (n[d] > kBluesteinMaxM / 2) return s;
     P[d] = static_length_at_least(n[d] + k[d] - 1);
     if (P[d] == 0 || !static_lookup(P[d])) return s;
-    any = true;
-    smooth = smooth && smooth_at_least(n[d]) == n[d];
   }
-  if (!any) return s;
-  // The extension pays until it multiplies a plane's area about fourfold and
-  // the runtime-length kernels have only small radices to run: 252 x 252 x
-  // 128 takes 86 us extended against 188 us with a 15^3 kernel (area x 1.3),
-  // 160 against 220 us with 101 x 101 x 128 (x 2.0), but 278 against 241 us
-  // with a kernel of the whole image (x 4.1).  Lengths with larger prime
-  // factors gain there too: 158 x 158 x 218 with an image-sized kernel 257
-  // against 819 us, 444 x 333 x 200 1245 against 3107 us.
-  if (smooth && (double)P[0] * P[1] > 3.0 * s.nx * s.ny) return s;
+  if (!extension_pays(s, P)) return s;
   ConvShape e = s;
   e.px = P[0];
   e.py = P[1];

@@ -2,7 +2,9 @@
 (tests/routes/routes.cpp) linked against the static archive prints a problem's
 transform lengths, whether it takes the whole-plane kernels, and its
 workspace."""
+import math
 import os
+import random
 import subprocess
 
 import pytest
@@ -59,3 +61,46 @@ def test_extended_planes_take_no_plane_kernel(routes):
             plain += 1
     # longer in x or y: 3 kernels x 4 modes of every plane
     assert extended == 12 * len(planes) and plain == 13 * len(planes)
+
+
+# (image, kernel) x y z, and whether its axes are extended: the two sides of
+# each line of extension_pays (conv_driver.cpp)
+EXTENDED = [((509, 1, 500), (9, 1, 9), False), ((509, 1, 128), (3, 1, 5), True),
+            ((509, 3, 500), (9, 3, 9), True), ((3001, 1, 2000), (5, 1, 3), False),
+            ((3001, 2, 512), (5, 1, 3), False), ((1, 509, 2000), (1, 5, 3), True),
+            ((1, 1511, 2000), (1, 5, 3), False),
+            ((64, 64, 1), (3, 3, 1), False), ((126, 126, 1), (9, 9, 1), True),
+            ((252, 252, 128), (101, 101, 128), True), ((252, 252, 128), (252, 252, 128), False),
+            ((13, 14, 512), (3, 3, 3), False), ((22, 5, 512), (3, 1, 5), False),
+            ((31, 31, 31), (31, 31, 31), True), ((143, 5, 512), (5, 1, 3), True),
+            ((14, 512, 64), (3, 3, 3), False), ((36, 512, 64), (18, 18, 18), False),
+            ((252, 512, 64), (3, 3, 3), True), ((20, 512, 90), (3, 3, 3), True),
+            ((13, 512, 64), (3, 3, 3), False), ((104, 512, 64), (52, 52, 52), True),
+            ((17, 512, 64), (3, 3, 3), False), ((23, 64, 64), (3, 3, 3), True),
+            ((158, 158, 218), (31, 31, 91), True), ((286, 286, 346), (31, 31, 91), True)]
+
+
+def test_where_an_extension_pays(routes):
+    got = routes([(*n, *k, 0) for n, k, _ in EXTENDED])
+    for (n, k, want), g in zip(EXTENDED, got):
+        assert (g[:3] != n) == want, (n, k, g)
+
+
+def test_extended_workspace_is_bounded(routes, fc):
+    """Past 32 MiB no convolution asks for more than 13 times the workspace
+    of its own extents."""
+    rng = random.Random(7)
+    problems = []
+    while len(problems) < 3000:
+        n = [int(round(math.exp(rng.uniform(0, math.log(3413))))) for _ in range(3)]
+        if n[0] * n[1] * n[2] > 1 << 28:
+            continue
+        f = rng.choice([0.03, 0.3, 1.0])
+        problems.append((*n, *(max(1, int(f * d * rng.uniform(0.5, 1.0))) for d in n), 0))
+    fc.use_static_kernels(False)
+    try:
+        plain = [fc.workspace_bytes(p[2::-1], p[5:2:-1]) for p in problems]
+    finally:
+        fc.use_static_kernels(True)
+    for p, own, got in zip(problems, plain, routes(problems)):
+        assert got[5] <= max(32 << 20, 13 * own), (p, own, got)
