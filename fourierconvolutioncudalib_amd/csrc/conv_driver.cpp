@@ -1037,8 +1037,14 @@ namespace {
 // one fits full volumes.  At 256 x 256 x 128 with 21^3 the 16-bin tile
 // leaves 170 workgroups for 256 CUs, the 8-bin tile twice as many:
 // PSF gradient 89.1 -> 86.5 us)
+// With U, a real volume of the planes, the rows of a large kernel are inverted
+// into it instead: the direct rows cost kx * ky * nx a plane, the x pass ny *
+// nx, and they meet at kx * ky = 8 to 16 times ny (us, direct / pass: 158 x 158
+// x 218 z y x with 61^3, 15 times, 123.7 / 121.6; 127^3 with 45^3, 11 times,
+// 64.0 / 68.7; 346 x 286 x 286 with 91^3, 22 times, 362 / 346; 59 x 96 x 715
+// with 59 x 96 x 694 881 / 144).
 void gather_from_planes(const ConvShape& s, float2* G, const FftDesc& fx, float* d_dkernel,
-                        hipStream_t st) {
+                        hipStream_t st, float* U = nullptr) {
   ConvShape sub = s;
   sub.nz = s.kz;
   const FftDesc fy = fft_desc(s.ny, st);
@@ -1047,6 +1053,12 @@ void gather_from_planes(const ConvShape& s, float2* G, const FftDesc& fx, float*
     PassScope ps(kPassYInverse, st);
     if (!static_ycol_fill(sub, fy, G, +1, cu_count(), st))
       launch_gk_col(spectrum_column_args(sub, fy, G), +1, sub.nz, st);
+  }
+  if (U && (long)s.kx * s.ky > 16L * s.ny) {
+    pass_x_inverse(sub, G, U, st);
+    sub.cz = 0;
+    launch_gather_kernel_support(sub, U, d_dkernel, st);
+    return;
   }
   launch_gather_support_c2r(s, G, padded_bins(s.nx), fx.tw, d_dkernel, st);
 }
@@ -1082,7 +1094,8 @@ void enqueue_grad_kernel_ext(const ConvShape& s, float* d_dkernel, const float* 
   t.nx = s.px;
   t.ny = s.py;
   t.nz = s.pz;
-  gather_from_planes(t, G, fft_desc(s.px, st), d_dkernel, st);
+  // (the image's spectrum is done with, and larger than those planes)
+  gather_from_planes(t, G, fft_desc(s.px, st), d_dkernel, st, reinterpret_cast<float*>(I));
 }
 
 }  // namespace
