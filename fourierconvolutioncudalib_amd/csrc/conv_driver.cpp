@@ -476,10 +476,16 @@ bool extension_pays(const ConvShape& s, const int (&P)[3]) {
     return prime <= 7 || plane <= 4 || (plane <= 8 && s.nx > 26) ||
            (P[0] != s.nx && row <= 1.2 && (area <= 12 || mib <= 8)) || mib <= 0.5;
   }
-  // x or z or both.  36 x 512 x 64 (row x 1.5) 52 -> 66 and 14 x 512 x 64 (x
-  // 2) 40 -> 58, 252 x 128 x 128 with 126^3 (x 1.6) 85 -> 89; 252 x 512 x 64
-  // with 3^3 (x 1.1) 130 -> 107, 20 x 512 x 90 (x 2, but z gains) 1.5 times
-  if (prime <= 7) return row <= 1.2 || (row <= 1.4 && big) || (z && s.nz >= 90);
+  // x or z or both; where z is one of two, or alone, and y short, it gains
+  // (128 x 128 x 21 26 -> 21, 117 x 144 x 25 with its own size 58 -> 30)
+  if (z && s.ny <= 256) return true;
+  // 36 x 512 x 64 (row x 1.5) 52 -> 66 and 14 x 512 x 64 (x 2) 40 -> 58, 252
+  // x 128 x 128 with 126^3 (x 1.6) 85 -> 89; 252 x 512 x 64 with 3^3 (x 1.1)
+  // 130 -> 107, 50 x 64 x 64 (x 1.5) 29 -> 23, 126 x 448 x 70 (x 1.3, z too)
+  // 117 -> 83, 20 x 512 x 90 (x 2, z too) 1.5 times
+  if (prime <= 7)
+    return row <= 1.2 || (row <= 1.4 && big) || (row <= 1.6 && s.ny <= 128) ||
+           (z && s.nz >= (row <= 1.6 ? 45 : 90));
   // 13 x 512 x 64 (x 2) 44 -> 58, 22 x 512 x 64 51 -> 58; 104 x 512 x 64
   // with 52^3 (x 1.5) 108 -> 90
   if (prime <= 13) return row <= 1.6 || big || (z && s.nz >= 52);

@@ -75,6 +75,8 @@ EXTENDED = [((509, 1, 500), (9, 1, 9), False), ((509, 1, 128), (3, 1, 5), True),
             ((31, 31, 31), (31, 31, 31), True), ((143, 5, 512), (5, 1, 3), True),
             ((14, 512, 64), (3, 3, 3), False), ((36, 512, 64), (18, 18, 18), False),
             ((252, 512, 64), (3, 3, 3), True), ((20, 512, 90), (3, 3, 3), True),
+            ((50, 64, 64), (15, 11, 39), True), ((126, 448, 70), (31, 31, 33), True),
+            ((128, 128, 21), (3, 3, 10), True),
             ((13, 512, 64), (3, 3, 3), False), ((104, 512, 64), (52, 52, 52), True),
             ((17, 512, 64), (3, 3, 3), False), ((23, 64, 64), (3, 3, 3), True),
             ((158, 158, 218), (31, 31, 91), True), ((286, 286, 346), (31, 31, 91), True)]
