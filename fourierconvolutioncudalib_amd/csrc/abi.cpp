@@ -85,9 +85,9 @@ ConvShape shape_from_any(const int* imDim, const int* kernelDim) {
 
 // shape_from_any as the convolution entry points run it: extended to
 // compile-time transform lengths where that is faster
-ConvShape conv_shape(const int* imDim, const int* kernelDim) {
+ConvShape conv_shape(const int* imDim, const int* kernelDim, bool gradient = false) {
   const ConvShape s = shape_from_any(imDim, kernelDim);
-  return needs_long_path(s) ? s : with_extension(s);
+  return needs_long_path(s) ? s : with_extension(s, gradient);
 }
 
 // device workspace of one device-resident convolution of `s`
@@ -548,7 +548,7 @@ int fcamd_convolve3d_boundary_host(float* im, const int* imDim, const float* ker
 long long fcamd_grad_kernel_workspace_bytes(const int* imDim, const int* kernelDim) {
   long long r = -1;
   (void)guarded([&] {
-    const ConvShape s = conv_shape(imDim, kernelDim);
+    const ConvShape s = conv_shape(imDim, kernelDim, true);
     r = (long long)(needs_long_path(s) ? long_workspace_bytes(s) : grad_workspace_layout(s).total());
   });
   return r;
@@ -559,7 +559,7 @@ int fcamd_conv_grad_kernel_device(float* d_dkernel, const float* d_grad_out, con
                                   long long workspace_bytes, void* stream) {
   return guarded([&] {
     FC_REQUIRE(d_dkernel && d_grad_out && d_image, kInvalidArgument, "null device pointer");
-    ConvShape s = conv_shape(imDim, kernelDim);
+    ConvShape s = conv_shape(imDim, kernelDim, true);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (d_workspace && s.extended() && workspace_bytes < (long long)grad_workspace_layout(s).total())
       s = direct_shape(s);

@@ -435,9 +435,10 @@ ConvShape direct_shape(const ConvShape& s) {
 }
 
 namespace {
-// Whether the extended transform (lengths P) of a convolution is faster than
-// the runtime-length kernels it would replace.  What decides, over about 2000
-// shapes timed both ways (x y z here; us runtime -> extended):
+// Whether the extended transform (lengths P) of a convolution, or of a PSF
+// gradient, is faster than the runtime-length kernels it would replace.  What
+// decides, over about 2000 shapes timed both ways (x y z here; us runtime ->
+// extended):
 // - the largest prime of the lengths replaced.  Above 31 they run a chirp-z
 //   and the extension gains 1.5 to 15 times, until it multiplies the plane
 //   of a large problem, whose time is then its traffic: 1511 x 2 x 2000 (16
@@ -451,7 +452,10 @@ namespace {
 // - the growth of a row in 16-bin column tiles: from one tile to two every y
 //   and z column costs twice, which small problems and small primes do not
 //   earn back.
-bool extension_pays(const ConvShape& s, const int (&P)[3]) {
+// A gradient gains less: its two volumes run their x and y passes in two
+// launches each where the runtime-length kernels pair them, and its z pass
+// transforms both columns whole.
+bool extension_pays(const ConvShape& s, const int (&P)[3], bool gradient) {
   const int n[3] = {s.nx, s.ny, s.nz};
   int prime = 0;
   for (int d = 0; d < 3; ++d)
@@ -468,33 +472,64 @@ bool extension_pays(const ConvShape& s, const int (&P)[3]) {
   // 86, with 101 x 101 x 128 (x 2.0) 220 -> 160, with its own size (x 4.1)
   // 241 -> 278
   if (prime <= 7 && area > 3) return false;
-  const bool z = P[2] != s.nz && s.nz > 1;
+  const bool x = P[0] != s.nx, z = P[2] != s.nz && s.nz > 1;
+  // x among them, and its row keeps its tiles
+  const bool x_keeps = x && row <= 1.2 && (area <= 12 || mib <= 8);
+  if (gradient) {
+    if (P[1] != s.ny) {
+      // products of 2, 3, 5 and 7: 128 x 28 x 128 (plane x 1.7) 37 -> 45, 20 x
+      // 28 x 512 (x 2.3) 42 -> 53; 256 x 63 x 256 (x 1.3) gains, and 75 x 54 x
+      // 48 (x 1.6, x too) 47 -> 32, 126 x 126 x 126 (all three) 2 times
+      if (prime <= 7)
+        return plane <= 1.3 || (plane <= 2.6 && big) || (x && plane <= (z ? 2.6 : 1.8));
+      // 14 x 22 x 512 (x 2.9) 45 -> 53, 14 x 26 x 512 (x 2.5) 48 -> 53; 26 x
+      // 29 x 133 (x 3.3, all three) 114 -> 40
+      if (prime <= 13)
+        return plane <= 2.1 || (plane <= 2.4 && row <= 1.2) || (big && area <= 12) || x_keeps ||
+               (x && z && plane <= 8);
+      // 17 x 20 x 512 (x 3.2) 42 -> 52, 17 x 14 x 512 (x 4.6) 40 -> 53; 23 x
+      // 248 x 130 (x 5.4, all three) 302 -> 96
+      return plane <= 3.1 || (area <= 12 && (big || mib < 1)) || x_keeps || (z && plane <= 8);
+    }
+    // 36 x 512 x 64 (row x 1.5) 52 -> 77; z alone: 64 x 64 x 14 23 -> 28, 64
+    // x 512 x 45 61 -> 72, but 256 x 256 x 168 1.9 times
+    if (prime <= 7) return row <= 1.2 && (!z || big);
+    // 55 x 512 x 14 (x 1.5, z too) 42 -> 58; z alone: 64 x 64 x 13 25 -> 27;
+    // 88 x 100 x 195 (x 1.7, z too) 123 -> 61
+    if (prime <= 13)
+      return big || (!z ? row <= 1.4
+                        : x ? row <= 1.2 || (row <= 1.9 && s.nz >= 39) : s.nz >= 26);
+    // 23 x 64 x 64 (x 2) 27 -> 29, 17 x 512 x 64 53 -> 64
+    return row <= 1.9 || mib >= 16;
+  }
   if (P[1] != s.ny) {
     // 13 x 14 x 512 (plane x 4.6) 37 -> 40, 22 x 5 x 512 (x 13) 36 -> 39, 17
     // x 9 x 512 (x 7.1) 37 -> 39, but 31 x 31 x 31 with its own size (x 6.2)
     // 76 -> 21 and, the row keeping its tiles, 143 x 5 x 512 (x 6.4) 82 -> 40
     return prime <= 7 || plane <= 4 || (plane <= 8 && s.nx > 26) ||
-           (P[0] != s.nx && row <= 1.2 && (area <= 12 || mib <= 8)) || mib <= 0.5;
+           x_keeps || mib <= 0.5;
   }
   // x or z or both; where z is one of two, or alone, and y short, it gains
   // (128 x 128 x 21 26 -> 21, 117 x 144 x 25 with its own size 58 -> 30)
   if (z && s.ny <= 256) return true;
   // 36 x 512 x 64 (row x 1.5) 52 -> 66 and 14 x 512 x 64 (x 2) 40 -> 58, 252
   // x 128 x 128 with 126^3 (x 1.6) 85 -> 89; 252 x 512 x 64 with 3^3 (x 1.1)
-  // 130 -> 107, 50 x 64 x 64 (x 1.5) 29 -> 23, 126 x 448 x 70 (x 1.3, z too)
-  // 117 -> 83, 20 x 512 x 90 (x 2, z too) 1.5 times
+  // 130 -> 107, 126 x 240 x 48 (x 1.3) 54 -> 43, 50 x 64 x 64 (x 1.5) 29 ->
+  // 23, 126 x 448 x 70 (x 1.3, z too) 117 -> 83, 20 x 512 x 90 (x 2, z too)
+  // 1.5 times
   if (prime <= 7)
-    return row <= 1.2 || (row <= 1.4 && big) || (row <= 1.6 && s.ny <= 128) ||
+    return row <= 1.2 || (row <= 1.4 && (big || s.ny <= 256)) || (row <= 1.6 && s.ny <= 128) ||
            (z && s.nz >= (row <= 1.6 ? 45 : 90));
   // 13 x 512 x 64 (x 2) 44 -> 58, 22 x 512 x 64 51 -> 58; 104 x 512 x 64
   // with 52^3 (x 1.5) 108 -> 90
   if (prime <= 13) return row <= 1.6 || big || (z && s.nz >= 52);
-  // 17 x 512 x 64 (x 2) 53 -> 58; 23 x 64 x 64 28 -> 21, 31 x 512 x 64 1.4
-  return row <= 1.9 || mib >= 16 || s.ny <= 256 || s.nx > 24 || (z && s.nz >= 27);
+  // 17 x 512 x 64 (x 2) 53 -> 58, 19 x 384 x 35 (z too) 45 -> 48; 23 x 64 x
+  // 64 28 -> 21, 31 x 512 x 64 1.4
+  return row <= 1.9 || mib >= 16 || s.ny <= 256 || s.nx > 24 || (z && s.nz >= 40);
 }
 }  // namespace
 
-ConvShape with_extension(const ConvShape& s) {
+ConvShape with_extension(const ConvShape& s, bool gradient) {
   const int n[3] = {s.nx, s.ny, s.nz}, k[3] = {s.kx, s.ky, s.kz};
   int P[3];
   for (int d = 0; d < 3; ++d) {
@@ -506,7 +541,7 @@ ConvShape with_extension(const ConvShape& s) {
     P[d] = static_length_at_least(n[d] + k[d] - 1);
     if (P[d] == 0 || !static_lookup(P[d])) return s;
   }
-  if (!extension_pays(s, P)) return s;
+  if (!extension_pays(s, P, gradient)) return s;
   ConvShape e = s;
   e.px = P[0];
   e.py = P[1];

@@ -33,8 +33,9 @@ struct ConvShape {
 // length that has (AxisExt in kernels.hpp): a circular convolution by a
 // compact kernel only needs its k - 1 neighbours past the ends, so any
 // length >= n + k - 1 gives the same result.  Returned unchanged where no
-// such length is worth it (the runtime-length kernels then run).
-ConvShape with_extension(const ConvShape& s);
+// such length is worth it (the runtime-length kernels then run).  `gradient`:
+// for the PSF gradient of that convolution.
+ConvShape with_extension(const ConvShape& s, bool gradient = false);
 // the same problem without the extension
 ConvShape direct_shape(const ConvShape& s);
 

@@ -1,5 +1,6 @@
 // Prints how the library would run convolutions, without a device.  Input:
-// one problem a line, "nx ny nz kx ky kz boundary"; output: its transform
+// one problem a line, "nx ny nz kx ky kz boundary" (boundary 5: the PSF
+// gradient of the periodic convolution); output: its transform
 // lengths, whether its forward and its inverse take a whole-plane kernel
 // (each 0 or 1) and its workspace bytes.
 #include <cstdio>
@@ -18,8 +19,8 @@ int main() {
       s.cy = s.ky / 2;
       s.cz = s.kz / 2;
       ConvShape e = s;
-      if (boundary == kMapPeriodic) {
-        e = with_extension(s);
+      if (boundary == kMapPeriodic || boundary == 5) {
+        e = with_extension(s, boundary == 5);
       } else {
         const PaddedProblem p = padded_problem(s, boundary);
         // (a padded problem never takes the plane kernels)

@@ -76,7 +76,8 @@ EXTENDED = [((509, 1, 500), (9, 1, 9), False), ((509, 1, 128), (3, 1, 5), True),
             ((14, 512, 64), (3, 3, 3), False), ((36, 512, 64), (18, 18, 18), False),
             ((252, 512, 64), (3, 3, 3), True), ((20, 512, 90), (3, 3, 3), True),
             ((50, 64, 64), (15, 11, 39), True), ((126, 448, 70), (31, 31, 33), True),
-            ((128, 128, 21), (3, 3, 10), True),
+            ((128, 128, 21), (3, 3, 10), True), ((126, 240, 48), (13, 39, 31), True),
+            ((19, 384, 35), (1, 32, 3), False),
             ((13, 512, 64), (3, 3, 3), False), ((104, 512, 64), (52, 52, 52), True),
             ((17, 512, 64), (3, 3, 3), False), ((23, 64, 64), (3, 3, 3), True),
             ((158, 158, 218), (31, 31, 91), True), ((286, 286, 346), (31, 31, 91), True)]
@@ -85,6 +86,25 @@ EXTENDED = [((509, 1, 500), (9, 1, 9), False), ((509, 1, 128), (3, 1, 5), True),
 def test_where_an_extension_pays(routes):
     got = routes([(*n, *k, 0) for n, k, _ in EXTENDED])
     for (n, k, want), g in zip(EXTENDED, got):
+        assert (g[:3] != n) == want, (n, k, g)
+
+
+EXTENDED_GRADIENTS = [((128, 28, 128), (14, 14, 14), False), ((256, 63, 256), (3, 3, 3), True),
+                      ((126, 126, 126), (6, 6, 6), True), ((14, 22, 512), (3, 3, 3), False),
+                      ((256, 26, 256), (3, 3, 3), True), ((17, 20, 512), (3, 3, 3), False),
+                      ((64, 23, 64), (3, 3, 3), True), ((36, 512, 64), (18, 18, 18), False),
+                      ((64, 64, 14), (3, 3, 3), False), ((256, 256, 168), (3, 3, 3), True),
+                      ((55, 512, 14), (27, 27, 14), False), ((64, 64, 13), (3, 3, 3), False),
+                      ((77, 512, 64), (3, 3, 3), True), ((17, 512, 64), (3, 3, 3), False),
+                      ((23, 64, 64), (3, 3, 3), False), ((58, 512, 64), (3, 3, 3), True),
+                      ((75, 54, 48), (25, 11, 19), True), ((23, 248, 130), (23, 189, 94), True),
+                      ((26, 29, 133), (9, 11, 49), True), ((88, 100, 195), (35, 17, 7), True),
+                      ((158, 158, 218), (31, 31, 91), True), ((509, 1, 500), (9, 1, 9), False)]
+
+
+def test_where_an_extended_gradient_pays(routes):
+    got = routes([(*n, *k, 5) for n, k, _ in EXTENDED_GRADIENTS])
+    for (n, k, want), g in zip(EXTENDED_GRADIENTS, got):
         assert (g[:3] != n) == want, (n, k, g)
 
 
