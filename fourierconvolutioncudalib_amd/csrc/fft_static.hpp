@@ -203,6 +203,16 @@ constexpr int z_full_id() {
   return p.n > 0 && !(p.r[0] == 18 && p.r[1] == 15) ? (L | kZPlan) : L;
 }
 
+// And for whole second columns (the PSF gradient's, kernels past half the
+// column): the lopsided plans 25 * 10 and 20 * 10 lose there.  The gradient's z
+// pass, two stages against three, us: 128 x 512 x 250 69 / 43, x 200 44 / 35,
+// 320 x 64 x 250 26 / 26, x 200 20 / 22.
+template <int L>
+constexpr int z_whole_id() {
+  constexpr StaticPlanData p = z_plan(L);
+  return p.n > 0 && p.r[0] >= 2 * p.r[1] ? L : z_full_id<L>();
+}
+
 // Per-stage twiddle tables of a static plan, stored for the forward stage
 // order and then for the reversed order (then the same for the z plan): stage s holds Ns(s) rows of
 // even(R) float2, row k = exp(-2 pi i r k / (Ns R)) for r = 0..R-1, so a

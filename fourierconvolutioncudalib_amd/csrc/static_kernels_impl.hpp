@@ -31,14 +31,15 @@ constexpr int threads_per_transform() {
 }
 
 // plan identifier and threads per column of the fused z kernels (PATH 1: the
-// tap path)
-template <int L, int PATH>
+// tap path; 0: a second column transformed like the image's, H = 0: a whole
+// one, else cut to H slots)
+template <int L, int PATH, int H = 0>
 constexpr int zk_id() {
-  return PATH == 1 ? z_id<L>() : z_full_id<L>();
+  return PATH == 1 ? z_id<L>() : H == 0 ? z_whole_id<L>() : z_full_id<L>();
 }
-template <int L, int PATH>
+template <int L, int PATH, int H = 0>
 constexpr int z_threads() {
-  return PlanOf<zk_id<L, PATH>(), false>::T;
+  return PlanOf<zk_id<L, PATH, H>(), false>::T;
 }
 
 // Largest tile <= want that keeps a workgroup within 1024 threads and its LDS
@@ -69,7 +70,8 @@ constexpr int col_fit() {
 }
 template <int L, int WANT>
 constexpr int z_fit() {
-  return fit_tile<L, WANT, WANT == 16 ? kTileLdsZ : kTileLds, z_threads<L, 0>()>();
+  constexpr int whole = z_threads<L, 0, 0>(), cut = z_threads<L, 0, 1>();
+  return fit_tile<L, WANT, WANT == 16 ? kTileLdsZ : kTileLds, (whole > cut ? whole : cut)>();
 }
 
 // row pairs per x-pass workgroup for about TGT threads (T threads per row
@@ -1359,7 +1361,7 @@ __host__ __device__ constexpr bool zfused_sparse_ok(int nvalid) {
 template <int L, int TX, int PATH, int H = 0, bool EXT = false>
 __device__ __forceinline__ void zfused_body(const ZArgs& a, const AxisExt* ext, long tile_index,
                                             float2* lds, float2* ktaps) {
-  constexpr int ID = zk_id<L, PATH>();
+  constexpr int ID = zk_id<L, PATH, H>();
   using ZT = ZTile<L, TX, ID>;
   const int c = threadIdx.x % TX, t = threadIdx.x / TX;
   const ZT tile(a, tile_index, c);
@@ -1393,7 +1395,7 @@ __device__ __forceinline__ void zfused_body(const ZArgs& a, const AxisExt* ext, 
 }
 
 template <int L, int TX, int PATH, int H = 0>
-__global__ void __launch_bounds__((TX * z_threads<L, PATH>()))
+__global__ void __launch_bounds__((TX * z_threads<L, PATH, H>()))
 sk_zfused_fft(ZArgs a) {
   __shared__ float2 lds[L * TX];
   __shared__ float2 ktaps[TX * (PATH == 0 ? 1 : ktap_slots<L>())];
@@ -1411,7 +1413,7 @@ sb_zfused(const ZArgs* __restrict__ args, const int2* __restrict__ tasks) {
 
 // the fused z pass of an extended image; PATH 0 and 1 as above
 template <int L, int TX, int PATH, int H = 0>
-__global__ void __launch_bounds__((TX * z_threads<L, PATH>()))
+__global__ void __launch_bounds__((TX * z_threads<L, PATH, H>()))
 sk_zfused_ext(ZExtArgs b) {
   __shared__ float2 lds[L * TX];
   __shared__ float2 ktaps[TX * (PATH == 0 ? 1 : ktap_slots<L>())];
@@ -1422,7 +1424,7 @@ sk_zfused_ext(ZExtArgs b) {
 template <int L, int TX>
 __global__ void __launch_bounds__((TX * z_threads<L, 0>()))
 sk_zcorr_ext(ZCorrArgs b) {
-  constexpr int ID = z_full_id<L>();
+  constexpr int ID = zk_id<L, 0>();
   using ZT = ZTile<L, TX, ID>;
   __shared__ float2 lds[L * TX];
   const ZArgs& a = b.z;
@@ -1440,7 +1442,7 @@ sk_zcorr_ext(ZCorrArgs b) {
 }
 
 template <int L, int TX>
-__global__ void __launch_bounds__((TX * z_threads<L, 0>()))
+__global__ void __launch_bounds__((TX * z_threads<L, 0, 1>()))
 sk_zfused_dft(ZArgs a) {
   using ZT = ZTile<L, TX, z_full_id<L>()>;
   __shared__ float2 lds[L * TX];
@@ -1581,6 +1583,7 @@ bool sk_launch_zfused_fft(const ZArgs& a, long ny, hipStream_t st) {
   ZArgs b = a;
   b.ny = ny;
   const dim3 grid((unsigned)column_tiles(a.nbins, TX, ny)), block(TX * z_threads<L, 0>());
+  const dim3 cut(TX * z_threads<L, 0, 1>());
   if constexpr (PlanOf<z_id<L>(), false>::S == 2) {
     if (zfused_sparse_ok<L>(a.nvalid)) {
       hipLaunchKernelGGL((sk_zfused_fft<L, TX, 1>), grid, dim3(TX * z_threads<L, 1>()), 0, st, b);
@@ -1591,11 +1594,11 @@ bool sk_launch_zfused_fft(const ZArgs& a, long ny, hipStream_t st) {
     constexpr int ID = z_full_id<L>();
     const int n = a.out_planes > 0 ? 0 : kernel_prune<ID>(a.nvalid, a.center);
     if (n == 1) {
-      hipLaunchKernelGGL((sk_zfused_fft<L, TX, 0, kernel_slots<ID>(1)>), grid, block, 0, st, b);
+      hipLaunchKernelGGL((sk_zfused_fft<L, TX, 0, kernel_slots<ID>(1)>), grid, cut, 0, st, b);
       return true;
     }
     if (n == 2) {
-      hipLaunchKernelGGL((sk_zfused_fft<L, TX, 0, kernel_slots<ID>(2)>), grid, block, 0, st, b);
+      hipLaunchKernelGGL((sk_zfused_fft<L, TX, 0, kernel_slots<ID>(2)>), grid, cut, 0, st, b);
       return true;
     }
   }
@@ -1640,6 +1643,7 @@ void sk_launch_zfused_ext(const ZExtArgs& a, long ny, hipStream_t st) {
   ZExtArgs b = a;
   b.z.ny = ny;
   const dim3 grid((unsigned)column_tiles(a.z.nbins, TX, ny)), block(TX * z_threads<L, 0>());
+  const dim3 cut(TX * z_threads<L, 0, 1>());
   if constexpr (PlanOf<z_id<L>(), false>::S == 2) {
     if (zfused_sparse_ok<L>(a.z.nvalid)) {
       hipLaunchKernelGGL((sk_zfused_ext<L, TX, 1>), grid, dim3(TX * z_threads<L, 1>()), 0, st, b);
@@ -1649,9 +1653,9 @@ void sk_launch_zfused_ext(const ZExtArgs& a, long ny, hipStream_t st) {
   constexpr int ID = z_full_id<L>();
   const int n = kernel_prune<ID>(a.z.nvalid, a.z.center);
   if (n == 1)
-    hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0, kernel_slots<ID>(1)>), grid, block, 0, st, b);
+    hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0, kernel_slots<ID>(1)>), grid, cut, 0, st, b);
   else if (n == 2)
-    hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0, kernel_slots<ID>(2)>), grid, block, 0, st, b);
+    hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0, kernel_slots<ID>(2)>), grid, cut, 0, st, b);
   else
     hipLaunchKernelGGL((sk_zfused_ext<L, TX, 0>), grid, block, 0, st, b);
 }
@@ -1679,7 +1683,7 @@ bool sk_launch_zfused_dft(const ZArgs& a, long ny, hipStream_t st) {
   ZArgs b = a;
   b.ny = ny;
   hipLaunchKernelGGL((sk_zfused_dft<L, TX>), dim3((unsigned)column_tiles(a.nbins, TX, ny)),
-                     dim3(TX * z_threads<L, 0>()), 0, st, b);
+                     dim3(TX * z_threads<L, 0, 1>()), 0, st, b);
   return true;
 }
 

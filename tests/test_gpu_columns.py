@@ -44,3 +44,25 @@ def test_x_workgroups(fc, oracle, rows):
         ref = oracle.numpy_fft_conv(a, k)
         got = fc.convolve3d(torch.from_numpy(a).cuda(), torch.from_numpy(k).cuda())
         assert oracle.rel_l2(got.cpu().numpy(), ref) < TOL, nx
+
+
+@pytest.mark.parametrize("nz", [200, 216, 250, 270, 400])
+def test_whole_second_columns(fc, oracle, nz):
+    """PSF gradients and kernels past half the column, on lengths whose whole
+    columns and cut ones run different plans (200, 250) and the same."""
+    import numpy as np
+    import torch
+    from fourierconvolutioncudalib_amd import synth
+    from fourierconvolutioncudalib_amd.autograd import grad_kernel
+    shape = (nz, 33, 64)
+    a = synth.uniform(shape, 5500 + nz)
+    g = np.random.default_rng(5501).standard_normal(shape).astype(np.float32)
+    ta, tg = torch.from_numpy(a).cuda(), torch.from_numpy(g).cuda()
+    for kz in (1, 9, nz // 2 + 1, nz):
+        kshape = (kz, 3, 5)
+        print("whole columns", nz, kz, flush=True)
+        got = grad_kernel(tg, ta, kshape).cpu().numpy()
+        assert oracle.rel_l2(got, oracle.fft_conv_grad_kernel(g, a, kshape)) < TOL, kz
+        k = synth.random_psf(kshape, 5600 + kz)
+        got = fc.convolve3d(ta, torch.from_numpy(k).cuda()).cpu().numpy()
+        assert oracle.rel_l2(got, oracle.numpy_fft_conv(a, k)) < TOL, kz
