@@ -89,6 +89,12 @@ struct RLLayout {
   }
 };
 
+// the same problem with no view extended
+RLProblem unextended(RLProblem p) {
+  for (ConvShape& s : p.views) s = direct_shape(s);
+  return p;
+}
+
 RLLayout rl_layout(const RLProblem& p) {
   RLLayout l{};
   const size_t nxp = padded_bins(p.img.nx);
@@ -103,6 +109,10 @@ RLLayout rl_layout(const RLProblem& p) {
   }
   l.vol = a256(sizeof(float) * (size_t)p.img.voxels());
   return l;
+}
+
+size_t rl_workspace(const RLProblem& p, bool fused) {
+  return rl_layout(p).total(p, fused) + a256(sizeof(float*) * kMaxViews);
 }
 
 void run_rl(const RLProblem& p, float* psi, const float* const* views, const float* const* kernels,
@@ -250,7 +260,7 @@ long long fcamd_rl_workspace_bytes(int nviews, const int* imDim, const int* kern
   (void)rl_guarded([&] {
     RLProblem p = make_problem(nviews, imDim, kernelDims);
     const bool f = fused != 0 && fused_available(p);
-    r = (long long)(rl_layout(p).total(p, f) + a256(sizeof(float*) * kMaxViews));
+    r = (long long)rl_workspace(p, f);
   });
   return r;
 }
@@ -274,17 +284,19 @@ int fcamd_rl_multiview_device(float* d_psi, const float* const* d_views, int nvi
     for (int v = 0; v < nviews; ++v)
       FC_REQUIRE(d_views[v] && d_kernels[v], kInvalidArgument, "null view or kernel");
     const bool f = fused != 0 && fused_available(p);
-    const size_t need = rl_layout(p).total(p, f) + a256(sizeof(float*) * kMaxViews);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (d_workspace) {
-      FC_REQUIRE(workspace_bytes >= (long long)need, kInvalidArgument, "workspace too small");
+      // a workspace that holds the unextended transforms is enough for them
+      if (workspace_bytes < (long long)rl_workspace(p, f)) p = unextended(p);
+      FC_REQUIRE(workspace_bytes >= (long long)rl_workspace(p, f), kInvalidArgument,
+                 "workspace too small");
       run_rl(p, d_psi, d_views, d_kernels, iterations, eps, init_psi != 0, f, d_workspace, st);
     } else {
       int dev = 0;
       FC_HIP_CHECK(hipGetDevice(&dev));
       DevicePool& pool = device_pool(dev);
       std::lock_guard<std::mutex> lk(pool.mu);
-      void* ws = pool_reserve(&pool.ws, &pool.ws_bytes, need);
+      void* ws = pool_reserve(&pool.ws, &pool.ws_bytes, rl_workspace(p, f));
       run_rl(p, d_psi, d_views, d_kernels, iterations, eps, init_psi != 0, f, ws, st);
       FC_HIP_CHECK(hipStreamSynchronize(st));
     }
