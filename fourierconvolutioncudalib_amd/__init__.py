@@ -34,6 +34,7 @@ __all__ = [
 
 CONVOLVE = 0
 CORRELATE = 1
+_INVALID_ARGUMENT = 1  # status code of the library
 
 _fp = ctypes.POINTER(ctypes.c_float)
 
@@ -216,7 +217,8 @@ def _check_tensor(t, name, shape=None, device=None, contiguous=True):
 
 def _workspace(nbytes, workspace, device, stream):
     """(pointer, bytes, keep-alive tensor) of the workspace for one call:
-    the caller's, else a new one from torch's caching allocator (no
+    the caller's (whether it is large enough is the library's to say, see
+    _check_call), else a new one from torch's caching allocator (no
     synchronisation, usable under graph capture).  A new workspace used on a
     stream other than torch's current one is recorded on that stream so the
     allocator does not hand it out again before the call's kernels ran."""
@@ -227,8 +229,8 @@ def _workspace(nbytes, workspace, device, stream):
         if workspace.device != device or not workspace.is_contiguous():
             raise ValueError("workspace must be a contiguous tensor on the image's device")
         have = workspace.numel() * workspace.element_size()
-        if have < nbytes:
-            raise ValueError(f"workspace holds {have} bytes, {nbytes} needed")
+        if have == 0 and nbytes > 0:  # no pointer: the library would take its own
+            raise ValueError(f"workspace holds 0 bytes, {nbytes} needed")
         return workspace.data_ptr(), have, workspace
     ws = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
     if stream is not None:
@@ -237,6 +239,14 @@ def _workspace(nbytes, workspace, device, stream):
         if stream.cuda_stream != torch.cuda.current_stream(device).cuda_stream:
             ws.record_stream(stream)
     return ws.data_ptr(), int(nbytes), ws
+
+
+def _check_call(rc, have, need):
+    """check() for a call given a workspace of ``have`` bytes.  One below
+    ``need`` may be enough (the library then runs the unextended transform)."""
+    if rc == _INVALID_ARGUMENT and have < need:
+        raise ValueError(f"workspace holds {have} bytes, {need} needed")
+    check(rc)
 
 
 # A small call is bound by its host work: 64 x 64 x 64 with a 7 x 7 x 7 kernel
@@ -279,16 +289,16 @@ class ConvolutionPlan:
         self.device = kernel.device
         self._kernel = kernel.contiguous()
         self._workspace = workspace
-        wptr, wbytes = None, 0
+        wptr, wbytes, need = None, 0, 0
         if workspace is not None:
-            wptr, wbytes, _ = _workspace(workspace_bytes(self.image_shape, self.kernel_shape),
-                                         workspace, self.device, stream)
+            need = workspace_bytes(self.image_shape, self.kernel_shape)
+            wptr, wbytes, _ = _workspace(need, workspace, self.device, stream)
         with _on_device(self.device):
             self._plan = lib().fcamd_conv_plan_create(
                 ints(self.image_shape[::-1]), ints(self.kernel_shape[::-1]),
                 self._kernel.data_ptr(), int(op), wptr, wbytes, _stream_handle(stream))
         if not self._plan:
-            check(lib().fcamd_last_error())
+            _check_call(lib().fcamd_last_error(), wbytes, need)
 
     def set_kernel(self, kernel, stream=None):
         """Replace the kernel (same dims); transformed on ``stream``."""
@@ -375,10 +385,10 @@ def convolve3d_boundary(image, kernel, boundary="zero", op=CONVOLVE, out=None, w
     need = boundary_workspace_bytes(image.shape, kernel.shape, boundary)
     wptr, wbytes, _keep = _workspace(need, workspace, image.device, stream)
     with _on_device(image.device):
-        check(lib().fcamd_convolve3d_boundary_device(
+        _check_call(lib().fcamd_convolve3d_boundary_device(
             out.data_ptr(), image.data_ptr(), ints(image.shape[::-1]),
             kernel.data_ptr(), ints(kernel.shape[::-1]), int(op), _boundary_code(boundary),
-            wptr, wbytes, _stream_handle(stream)))
+            wptr, wbytes, _stream_handle(stream)), wbytes, need)
     return out
 
 
@@ -404,7 +414,7 @@ def convolve3d(image, kernel, op=CONVOLVE, out=None, workspace=None, stream=None
     need = _checked_bytes(lib().fcamd_workspace_bytes(dims, kdims))
     wptr, wbytes, _keep = _workspace(need, workspace, image.device, stream)
     with _on_device(image.device):
-        check(lib().fcamd_convolve3d_device(
+        _check_call(lib().fcamd_convolve3d_device(
             out.data_ptr(), image.data_ptr(), dims, kernel.data_ptr(), kdims, int(op),
-            wptr, wbytes, _stream_handle(stream)))
+            wptr, wbytes, _stream_handle(stream)), wbytes, need)
     return out

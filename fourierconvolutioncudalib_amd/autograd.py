@@ -20,7 +20,7 @@ from ._lib import check, ints, lib
 def grad_kernel(grad_out, image, kernel_shape, workspace=None, stream=None):
     """dk[j] = sum_i g[i] * image[(i - (j - k//2)) mod n] on a kernel of
     C-order shape ``kernel_shape`` (torch CUDA float32)."""
-    from . import _check_tensor, _on_device, _stream_handle, _workspace
+    from . import _check_call, _check_tensor, _on_device, _stream_handle, _workspace
     _check_tensor(image, "image", contiguous=False)
     _check_tensor(grad_out, "grad_out", image.shape, image.device, contiguous=False)
     if image.dim() != 3 or len(kernel_shape) != 3:
@@ -31,9 +31,9 @@ def grad_kernel(grad_out, image, kernel_shape, workspace=None, stream=None):
     need = grad_kernel_workspace_bytes(image.shape, kernel_shape)
     wptr, wbytes, _keep = _workspace(need, workspace, image.device, stream)
     with _on_device(image.device):
-        check(lib().fcamd_conv_grad_kernel_device(
+        _check_call(lib().fcamd_conv_grad_kernel_device(
             dk.data_ptr(), grad_out.data_ptr(), image.data_ptr(), ints(image.shape[::-1]),
-            ints(tuple(kernel_shape)[::-1]), wptr, wbytes, _stream_handle(stream)))
+            ints(tuple(kernel_shape)[::-1]), wptr, wbytes, _stream_handle(stream)), wbytes, need)
     return dk
 
 
