@@ -232,7 +232,10 @@ def _workspace(nbytes, workspace, device, stream):
         if have == 0 and nbytes > 0:  # no pointer: the library would take its own
             raise ValueError(f"workspace holds 0 bytes, {nbytes} needed")
         return workspace.data_ptr(), have, workspace
-    ws = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
+    try:
+        ws = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None, 0, None  # the library's own, of the unextended size if need be
     if stream is not None:
         if isinstance(stream, int):
             stream = torch.cuda.ExternalStream(stream, device=device)

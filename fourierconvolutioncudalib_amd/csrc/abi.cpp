@@ -271,14 +271,14 @@ void host_convolution_padded(const ConvShape& raw, const PaddedProblem& p, int b
   const ConvShape& s = p.padded;
   const size_t nimg = sizeof(float) * (size_t)p.vp.n[0] * p.vp.n[1] * p.vp.n[2];
   const size_t nker = sizeof(float) * (size_t)s.kx * s.ky * s.kz;
-  const size_t nws = boundary_workspace(raw, p, boundary);
   void* dimg = pool_reserve(reinterpret_cast<void**>(&pool.img), &pool.img_bytes, nimg);
   void* dker = pool_reserve(reinterpret_cast<void**>(&pool.ker), &pool.ker_bytes, nker);
-  void* ws = pool_reserve(&pool.ws, &pool.ws_bytes, nws);
+  const size_t nws = pool_reserve_workspace(pool, boundary_workspace(raw, p, boundary),
+                                            workspace_layout(p.padded).total());
   staged_upload(dev, dimg, im, nimg, pool.stream);
   staged_upload(dev, dker, kernel, nker, pool.stream);
   enqueue_boundary(raw, p, boundary, static_cast<float*>(dimg), static_cast<float*>(dimg),
-                   static_cast<float*>(dker), op, ws, nws, pool.stream);
+                   static_cast<float*>(dker), op, pool.ws, nws, pool.stream);
   staged_download(dev, out, dimg, nimg, pool.stream);
 }
 
@@ -480,8 +480,9 @@ int fcamd_convolve3d_device(float* d_out, const float* d_image, const int* imDim
       FC_HIP_CHECK(hipGetDevice(&dev));
       DevicePool& pool = device_pool(dev);
       std::lock_guard<std::mutex> lk(pool.mu);
-      void* ws = pool_reserve(&pool.ws, &pool.ws_bytes, need);
-      enqueue_any(s, d_out, d_image, d_kernel, o, ws, st);
+      if (pool_reserve_workspace(pool, need, conv_workspace_bytes(direct_shape(s))) < need)
+        s = direct_shape(s);
+      enqueue_any(s, d_out, d_image, d_kernel, o, pool.ws, st);
       // the pooled workspace is reused by the next call: finish before unlocking
       FC_HIP_CHECK(hipStreamSynchronize(st));
     }
@@ -527,9 +528,9 @@ int fcamd_convolve3d_boundary_device(float* d_out, const float* d_image, const i
       FC_HIP_CHECK(hipGetDevice(&dev));
       DevicePool& pool = device_pool(dev);
       std::lock_guard<std::mutex> lk(pool.mu);
-      const size_t need = boundary_workspace(raw, p, boundary);
-      void* ws = pool_reserve(&pool.ws, &pool.ws_bytes, need);
-      enqueue_boundary(raw, p, boundary, d_out, d_image, d_kernel, o, ws, need, st);
+      const size_t got = pool_reserve_workspace(pool, boundary_workspace(raw, p, boundary),
+                                                workspace_layout(p.padded).total());
+      enqueue_boundary(raw, p, boundary, d_out, d_image, d_kernel, o, pool.ws, got, st);
       // the pooled workspace is reused by the next call: finish before unlocking
       FC_HIP_CHECK(hipStreamSynchronize(st));
     }
@@ -565,7 +566,7 @@ int fcamd_conv_grad_kernel_device(float* d_dkernel, const float* d_grad_out, con
       s = direct_shape(s);
     const bool lng = needs_long_path(s);
     const size_t need = lng ? long_workspace_bytes(s) : grad_workspace_layout(s).total();
-    auto run = [&](void* ws) {
+    auto run = [&](const ConvShape& s, void* ws) {
       if (lng)
         enqueue_grad_kernel_long(s, d_dkernel, d_grad_out, d_image, ws, st);
       else
@@ -573,14 +574,16 @@ int fcamd_conv_grad_kernel_device(float* d_dkernel, const float* d_grad_out, con
     };
     if (d_workspace) {
       FC_REQUIRE(workspace_bytes >= (long long)need, kInvalidArgument, "workspace too small");
-      run(d_workspace);
+      run(s, d_workspace);
     } else {
       int dev = 0;
       FC_HIP_CHECK(hipGetDevice(&dev));
       DevicePool& pool = device_pool(dev);
       std::lock_guard<std::mutex> lk(pool.mu);
-      void* ws = pool_reserve(&pool.ws, &pool.ws_bytes, need);
-      run(ws);
+      const ConvShape d = direct_shape(s);
+      const size_t got =
+          pool_reserve_workspace(pool, need, lng ? need : grad_workspace_layout(d).total());
+      run(got < need ? d : s, pool.ws);
       FC_HIP_CHECK(hipStreamSynchronize(st));
     }
   });

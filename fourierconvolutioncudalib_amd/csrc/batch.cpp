@@ -278,8 +278,19 @@ BatchPlan::BatchPlan(int n, const int* imDims, const int* kernelDims, float* con
       }
     };
     plan_lanes();
-    if (ws && ws_bytes < ws_need_) {  // room for the unextended blocks only
-      for (Block& bl : blocks_) bl.s = direct_shape(bl.s);
+    // the blocks unextended where the caller's workspace, or the device, has
+    // no room for more
+    const size_t want = ws_need_;
+    const std::vector<Block> extended = blocks_;
+    for (Block& bl : blocks_) bl.s = direct_shape(bl.s);
+    plan_lanes();
+    size_t have = ws_bytes;
+    if (!ws) {
+      have = alloc_workspace(&ws_, want, ws_need_);
+      own_ws_ = true;
+    }
+    if (have >= want) {
+      blocks_ = extended;
       plan_lanes();
     }
   } else {
@@ -288,7 +299,7 @@ BatchPlan::BatchPlan(int n, const int* imDims, const int* kernelDims, float* con
   if (ws) {
     FC_REQUIRE(ws_bytes >= ws_need_, kInvalidArgument, "batch workspace too small");
     ws_ = ws;
-  } else {
+  } else if (!own_ws_) {
     FC_HIP_CHECK(hipMalloc(&ws_, ws_need_));
     own_ws_ = true;
   }

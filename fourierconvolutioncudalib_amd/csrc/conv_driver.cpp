@@ -1213,6 +1213,30 @@ void* pool_reserve(void** p, size_t* cap, size_t bytes) {
   return *p;
 }
 
+size_t alloc_workspace(void** p, size_t want, size_t enough) {
+  const hipError_t rc = hipMalloc(p, want);
+  if (rc == hipErrorOutOfMemory && enough < want) {
+    (void)hipGetLastError();  // the failed allocation's
+    FC_HIP_CHECK(hipMalloc(p, enough));
+    return enough;
+  }
+  FC_HIP_CHECK(rc);
+  return want;
+}
+
+size_t pool_reserve_workspace(DevicePool& pool, size_t want, size_t enough) {
+  if (pool.ws && pool.ws_bytes >= want) return want;
+  if (pool.ws) {
+    FC_HIP_CHECK(hipDeviceSynchronize());
+    FC_HIP_CHECK(hipFree(pool.ws));
+    pool.ws = nullptr;
+    pool.ws_bytes = 0;
+  }
+  const size_t got = alloc_workspace(&pool.ws, want, enough);
+  pool.ws_bytes = got;
+  return got;
+}
+
 DeviceGuard::DeviceGuard(int dev) {
   int n = 0;
   if (hipGetDeviceCount(&n) != hipSuccess || n <= 0)

@@ -276,6 +276,10 @@ struct DevicePool {
 
 DevicePool& device_pool(int dev);
 void* pool_reserve(void** p, size_t* cap, size_t bytes);
+// Workspaces of extended shapes: `want` bytes, or `enough` (the unextended
+// shape's) where the device has no memory for those.  Both return which.
+size_t alloc_workspace(void** p, size_t want, size_t enough);
+size_t pool_reserve_workspace(DevicePool& pool, size_t want, size_t enough);
 
 // RAII: makes `dev` current and restores the caller's device on exit.
 class DeviceGuard {

@@ -90,8 +90,10 @@ void* fcamd_conv_plan_create(const int* imDim, const int* kernelDim, const float
         FC_REQUIRE(workspace_bytes >= (long long)need, kInvalidArgument, "workspace too small");
         p->ws = d_workspace;
       } else {
-        FC_HIP_CHECK(hipMalloc(&p->ws, need));
+        const size_t got =
+            alloc_workspace(&p->ws, need, lng ? need : workspace_layout(direct_shape(s)).total());
         p->own = true;
+        if (got < need) p->s = s = direct_shape(s);
       }
       if (!lng) {
         const WorkspaceLayout wl = workspace_layout(s);

@@ -296,8 +296,10 @@ int fcamd_rl_multiview_device(float* d_psi, const float* const* d_views, int nvi
       FC_HIP_CHECK(hipGetDevice(&dev));
       DevicePool& pool = device_pool(dev);
       std::lock_guard<std::mutex> lk(pool.mu);
-      void* ws = pool_reserve(&pool.ws, &pool.ws_bytes, rl_workspace(p, f));
-      run_rl(p, d_psi, d_views, d_kernels, iterations, eps, init_psi != 0, f, ws, st);
+      const size_t need = rl_workspace(p, f);
+      if (pool_reserve_workspace(pool, need, rl_workspace(unextended(p), f)) < need)
+        p = unextended(p);
+      run_rl(p, d_psi, d_views, d_kernels, iterations, eps, init_psi != 0, f, pool.ws, st);
       FC_HIP_CHECK(hipStreamSynchronize(st));
     }
   });

@@ -15,18 +15,22 @@ ROOT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..")
 MODES = {"periodic": 0, "zero": 1, "nearest": 2, "reflect": 3, "mirror": 4}
 
 
+def _build(fc, directory, name, *link):
+    prog = str(directory / name)
+    archive = os.path.join(os.path.dirname(fc._lib.LIB_PATH),
+                           "libFourierConvolutionCUDALib_static.a")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", fc._lib.CSRC,
+                    "-I/opt/rocm/include", os.path.join(ROOT, "tests", "routes", name + ".cpp"),
+                    archive, "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib",
+                    "-lpthread", *link, "-o", prog], check=True)
+    return prog
+
+
 @pytest.fixture(scope="session")
 def routes(fc, tmp_path_factory):
     """routes([(nx, ny, nz, kx, ky, kz, boundary), ...]) -> [(px, py, pz,
     plane forward, plane inverse, workspace bytes), ...]"""
-    prog = str(tmp_path_factory.mktemp("routes") / "routes")
-    csrc = fc._lib.CSRC
-    archive = os.path.join(os.path.dirname(fc._lib.LIB_PATH),
-                           "libFourierConvolutionCUDALib_static.a")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-D__HIP_PLATFORM_AMD__", "-I", csrc,
-                    "-I/opt/rocm/include", os.path.join(ROOT, "tests", "routes", "routes.cpp"),
-                    archive, "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib",
-                    "-lpthread", "-o", prog], check=True)
+    prog = _build(fc, tmp_path_factory.mktemp("routes"), "routes")
 
     def ask(problems):
         # every split form on, so that no rule asks a device for its CU count
@@ -126,3 +130,31 @@ def test_extended_workspace_is_bounded(routes, fc):
         fc.use_static_kernels(True)
     for p, own, got in zip(problems, plain, routes(problems)):
         assert got[5] <= max(32 << 20, 13 * own), (p, own, got)
+
+
+def test_workspace_where_memory_ends(fc, tmp_path):
+    """The pool's workspace for an extended transform, or for the unextended
+    one where the device has no memory for that; an error where it has for
+    neither."""
+    prog = _build(fc, tmp_path, "reserve", "-Wl,--wrap=hipMalloc,--wrap=hipFree,"
+                  "--wrap=hipDeviceSynchronize")
+    # memory, already held, wanted, enough -> returned, held afterwards, last request
+    cases = {(1000, 0, 800, 300): "800 800 800", (1000, 900, 800, 300): "800 900 0",
+             (500, 0, 800, 300): "300 300 300", (500, 400, 800, 300): "300 300 300",
+             (200, 0, 800, 300): "error 3 0", (500, 0, 800, 800): "error 3 0"}
+    r = subprocess.run([prog], input="\n".join(" ".join(map(str, c)) for c in cases),
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    assert r.stdout.splitlines() == list(cases.values())
+
+
+def test_tensor_workspace_where_memory_ends(fc, monkeypatch):
+    """Without memory for a call's workspace the wrapper leaves it to the
+    library."""
+    import torch
+
+    def empty(*a, **k):
+        raise torch.OutOfMemoryError("no memory")
+
+    monkeypatch.setattr(torch, "empty", empty)
+    assert fc._workspace(1 << 20, None, torch.device("cpu"), None) == (None, 0, None)
