@@ -311,6 +311,7 @@ BatchPlan::BatchPlan(int n, const int* imDims, const int* kernelDims, float* con
       long_prepare_tables(bl.s, nullptr);
       continue;
     }
+    if (bl.s.extended()) (void)extension_tables(bl.s, nullptr);
     int lens[5];
     for (int i = 0, n = table_lengths(bl.s, lens); i < n; ++i) (void)fft_desc(lens[i]);
   }

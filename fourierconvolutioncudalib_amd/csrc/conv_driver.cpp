@@ -1012,32 +1012,26 @@ void enqueue_inverse(const ConvShape& s, float2* S, float* d_out, hipStream_t st
     inverse_yx(s, S, d_out, st);
 }
 
-namespace {
-// Whether the tables of an extended shape exist or may be made now.  A
-// stream that is capturing records neither the allocation nor the copy: such
-// a call runs the shape unextended, whose tables depend on the image's
-// extents only (any kernel size used before has made them, below).
 bool extension_tables(const ConvShape& s, hipStream_t st) {
-  int lens[5];
-  const int n = table_lengths(s, lens);
-  bool have = true;
+  const ConvShape d = direct_shape(s);
+  int lens[5], own[5];
+  const int n = table_lengths(s, lens), m = table_lengths(d, own);
+  bool have = true, all = true;
   {
     const int dev = current_device();
     std::lock_guard<std::mutex> lk(g_tw_mu);
     for (int i = 0; i < n; ++i) have = have && g_desc.count(std::make_pair(dev, lens[i])) != 0;
+    for (int i = 0; i < m; ++i) all = all && g_desc.count(std::make_pair(dev, own[i])) != 0;
   }
-  if (have) return true;
+  if (have && all) return true;
   if (st != nullptr) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     FC_HIP_CHECK(hipStreamIsCapturing(st, &cs));
-    if (cs != hipStreamCaptureStatusNone) return false;
+    if (cs != hipStreamCaptureStatusNone) return have;
   }
-  const ConvShape d = direct_shape(s);
-  const int m = table_lengths(d, lens);
-  for (int i = 0; i < m; ++i) (void)fft_desc(lens[i]);
+  for (int i = 0; i < m; ++i) (void)fft_desc(own[i]);
   return true;
 }
-}  // namespace
 
 void enqueue_convolution(const ConvShape& shape, float* d_out, const float* d_image,
                          const float* d_kernel, Op op, void* ws, hipStream_t st) {

@@ -116,7 +116,14 @@ void pass_timing_collect(double* ms, int* count);
 void enqueue_convolution(const ConvShape& s, float* d_out, const float* d_image,
                          const float* d_kernel, Op op, void* ws, hipStream_t stream);
 
-// the same for a shape that is known to have (or may make) its tables
+// Whether the tables of an extended shape `s` exist or may be made now.  A
+// stream that is capturing records neither the allocation nor the copy: such
+// a call runs the shape unextended, whose tables depend on the image's
+// extents only.  So that any earlier call of those extents is enough for that,
+// whatever its kernel, a call outside a capture makes them here.
+bool extension_tables(const ConvShape& s, hipStream_t stream);
+
+// enqueue_convolution for a shape that is known to have (or may make) its tables
 void run_convolution(const ConvShape& s, float* d_out, const float* d_image,
                      const float* d_kernel, Op op, void* ws, hipStream_t stream);
 // its three parts: image (and kernel) to S (and Kxy), the product with the

@@ -79,6 +79,8 @@ void* fcamd_conv_plan_create(const int* imDim, const int* kernelDim, const float
       if (!d_workspace || workspace_bytes >= (long long)workspace_layout(e).total()) s = e;
     }
     driver_init();
+    if (s.extended() && !extension_tables(s, static_cast<hipStream_t>(stream)))
+      s = direct_shape(s);
     auto* p = new ConvPlan();
     p->s = s;
     p->lng = lng;

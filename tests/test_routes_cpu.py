@@ -158,3 +158,57 @@ def test_tensor_workspace_where_memory_ends(fc, monkeypatch):
 
     monkeypatch.setattr(torch, "empty", empty)
     assert fc._workspace(1 << 20, None, torch.device("cpu"), None) == (None, 0, None)
+
+
+_DEVICE_CALLS = ("hipMalloc", "hipFree", "hipMemcpy", "hipGetDevice", "hipGetLastError",
+                 "hipStreamIsCapturing", "__hipPushCallConfiguration",
+                 "__hipPopCallConfiguration", "hipLaunchKernel", "hipFuncSetAttribute",
+                 "hipDeviceGetAttribute", "hipOccupancyMaxActiveBlocksPerMultiprocessor",
+                 "hipStreamCreateWithFlags", "hipStreamDestroy", "hipEventCreateWithFlags",
+                 "hipEventDestroy")
+
+
+@pytest.fixture(scope="session")
+def steps(fc, tmp_path_factory):
+    """steps([(what, capturing, image, kernel), ...]) -> per step (launches,
+    allocations), or the status code of a refusal (tests/routes/capture.cpp);
+    every call starts from a process without tables"""
+    prog = _build(fc, tmp_path_factory.mktemp("capture"), "capture",
+                  "-Wl," + ",".join("--wrap=" + c for c in _DEVICE_CALLS))
+    env = {k: v for k, v in os.environ.items() if not k.startswith("FCAMD_")}
+
+    def run(what):
+        r = subprocess.run([prog], input="\n".join(" ".join(map(str, (w, c, *n, *k)))
+                                                   for w, c, n, k in what),
+                           env=env, capture_output=True, text=True)
+        assert r.returncode == 0, r.stderr
+        out = [line.split() for line in r.stdout.splitlines()]
+        assert len(out) == len(what)
+        return [int(o[1]) if o[0] == "error" else tuple(map(int, o)) for o in out]
+
+    return run
+
+
+CONV, GRADIENT, PLAN, BATCH = range(4)
+
+
+@pytest.mark.parametrize("first", [CONV, GRADIENT, PLAN, BATCH])
+@pytest.mark.parametrize("then", [CONV, GRADIENT, PLAN])
+def test_capture_after_any_kernel_size(steps, first, then):
+    """One eager call of an image's extents is enough to capture calls of any
+    kernel size on it, also where the first call's extended lengths were
+    there already and the second's are not."""
+    n = (126, 126, 126)  # extends to 128 with 3 taps, to 144 with 13
+    got = steps([(CONV, 0, (128, 128, 128), (3, 3, 3)), (first, 0, n, (3, 3, 3)),
+                 (then, 1, n, (13, 13, 13)), (then, 0, n, (13, 13, 13)),
+                 (then, 1, n, (13, 13, 13))])
+    assert got[1][1] > 0, "no table of the image's own extents"
+    assert got[2][0] > 0 and got[2][1] == 0, "captured"
+    assert got[3][0] > 0 and got[4][0] > 0 and got[4][1] == 0
+
+
+def test_capture_without_any_call_is_refused(steps):
+    n, k = (126, 126, 126), (3, 3, 3)
+    assert steps([(CONV, 1, n, k), (GRADIENT, 1, n, k)]) == [1, 1]
+    # and what is captured with its tables there allocates nothing
+    assert steps([(CONV, 0, n, k), (CONV, 1, n, k)])[1][1] == 0
