@@ -212,3 +212,17 @@ def test_capture_without_any_call_is_refused(steps):
     assert steps([(CONV, 1, n, k), (GRADIENT, 1, n, k)]) == [1, 1]
     # and what is captured with its tables there allocates nothing
     assert steps([(CONV, 0, n, k), (CONV, 1, n, k)])[1][1] == 0
+
+
+def test_current_stream_without_the_raw_handle(fc, monkeypatch):
+    """The current stream's handle from torch's public interface where the
+    direct one is not there."""
+    import torch
+
+    class Stream:
+        cuda_stream = 4096
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: Stream())
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    assert fc._stream_handle(None).value == 4096
