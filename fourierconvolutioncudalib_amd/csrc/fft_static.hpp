@@ -214,9 +214,10 @@ constexpr int z_whole_id() {
 }
 
 // Per-stage twiddle tables of a static plan, stored for the forward stage
-// order and then for the reversed order (then the same for the z plan): stage s holds Ns(s) rows of
-// even(R) float2, row k = exp(-2 pi i r k / (Ns R)) for r = 0..R-1, so a
-// thread fetches its butterfly's twiddles with R/2 aligned 16-byte loads.
+// order and then for the reversed order (then the same for the z plan): stage
+// s holds Ns(s) rows of even(R) float2, row k = exp(-2 pi i r k / (Ns R)) for
+// r = 0..R-1, so a thread fetches its butterfly's twiddles with R/2 aligned
+// 16-byte loads.
 constexpr int even_up(int r) { return (r + 1) / 2 * 2; }
 
 constexpr int static_tw_size(const StaticPlanData& p, bool rev) {
@@ -376,17 +377,29 @@ __device__ __forceinline__ void sfft_for_outputs(int t, F f) {
 #ifndef FC_TW_COMPACT_MIN
 #define FC_TW_COMPACT_MIN 8
 #endif
+// The z plan 18 * 16 loads whole rows: a product of two roots rounds twice
+// more, and there it showed (error against FP64 over 48 x 80 x 288 columns of
+// zero mean: the three-stage plan 3.18e-7, bases 3.26e-7, rows 3.17e-7).  The
+// registers are there, and the z pass takes the same time (128 x 512 x 288
+// with 61 taps 46 us).  At 216 the rows cost a wave per SIMD (34 -> 39 us), at
+// 336 and above as well (52 -> 65), and bases round no more than before.
+template <int ID>
+constexpr int tw_compact_min() {
+  constexpr StaticPlanData p = z_plan(ID & (kZPlan - 1));
+  return (ID & kZPlan) != 0 && p.r[0] == 18 && p.r[1] == 16 ? 32 : FC_TW_COMPACT_MIN;
+}
 // Stage s twiddle rows of the thread's butterflies, loaded ahead of use.
 // Stages of radix 8 and above keep bases instead of the row's R - 1
 // entries: W^k, W^2k, W^3k (q[0].xy, q[0].zw, q[1].xy), W^4k (q[1].zw) and,
 // from radix 9, W^8k, W^12k (q[2]), from radix 17 W^16k, W^20k (q[3]) and
-// from radix 25 W^24k (q[4]); entry r = r1 + 4*r2 is W^(r1 k) * W^(4 r2 k).  That is one product more for the entries with
-// r1, r2 > 0, but fewer loads and registers (12 instead of 32 at radix 16):
+// from radix 25 W^24k (q[4]); entry r = r1 + 4*r2 is W^(r1 k) * W^(4 r2 k).
+// That is one product more for the entries with r1, r2 > 0, but fewer loads
+// and registers (12 instead of 32 at radix 16):
 // one stage's twiddles are live beside the image's and the kernel column's
 // values at the fused z pass's register peak, and their loads sit between
 // the two barriers of every exchange.  Measured at 512 x 512 x 256: the z
 // pass 124 -> 115 us.
-template <int L, bool REV, int s, int CM = FC_TW_COMPACT_MIN>
+template <int L, bool REV, int s, int CM = tw_compact_min<L>()>
 struct StageTw {
   using P = PlanOf<L, REV>;
   static constexpr int R = P::R(s), Ns = P::Ns(s), NB = P::NB(s), RP = even_up(R);
@@ -539,7 +552,7 @@ __device__ __forceinline__ void sfft_rest(float2 (&v)[MAXE], int t, float2* lds,
 // smallest radix whose stages keep compact twiddles (StageTw); the x-R2C
 // passes measured faster with full rows at radix 8 (512 x 512 x 256: 105
 // against 110 us) and with compact ones at radix 16 (256 x 256 x 128).
-template <int L, bool REV, int DIR, int CM = FC_TW_COMPACT_MIN, int MAXE, class Addr>
+template <int L, bool REV, int DIR, int CM = tw_compact_min<L>(), int MAXE, class Addr>
 __device__ __forceinline__ void sfft_run(float2 (&v)[MAXE], int t, float2* lds, Addr addr,
                                          const float2* __restrict__ tw) {
   sfft_compute<L, REV, DIR, 0>(v, t, tw);
