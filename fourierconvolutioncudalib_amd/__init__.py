@@ -247,9 +247,10 @@ def _workspace(nbytes, workspace, device, stream):
 def _check_call(rc, have, need):
     """check() for a call given a workspace of ``have`` bytes.  One below
     ``need`` may be enough (the library then runs the unextended transform)."""
-    if rc == _INVALID_ARGUMENT and have < need:
-        raise ValueError(f"workspace holds {have} bytes, {need} needed")
-    check(rc)
+    if rc:
+        if rc == _INVALID_ARGUMENT and have < need:
+            raise ValueError(f"workspace holds {have} bytes, {need} needed")
+        check(rc)
 
 
 # A small call is bound by its host work: 64 x 64 x 64 with a 7 x 7 x 7 kernel
@@ -269,11 +270,10 @@ def _on_device(device):
 def _stream_handle(stream):
     if stream is None:
         import torch
-        # (not part of torch's public interface, so it may go away)
-        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-        if raw is None:
+        try:
+            return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+        except AttributeError:  # (it is not part of torch's public interface)
             return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-        return ctypes.c_void_p(raw(torch.cuda.current_device()))
     if isinstance(stream, int):
         return ctypes.c_void_p(stream)
     return ctypes.c_void_p(stream.cuda_stream)

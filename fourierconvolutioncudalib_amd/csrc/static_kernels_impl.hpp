@@ -322,7 +322,6 @@ template <int L>
 struct XStage {
   static constexpr bool V4 = (L % 4) == 0;       // real rows split into float4s
   static constexpr int SL = V4 ? L + 4 : L + 1;  // staging row stride (floats)
-  static constexpr int NB = L / 2 + 1;           // half-spectrum bins per row
 };
 
 // LDS floats of a flat x-pass workgroup of `pairs` row pairs: the larger of
