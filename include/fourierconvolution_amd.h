@@ -48,7 +48,10 @@ FCAMD_API long long fcamd_host_device_bytes(const int* imDim, const int* kernelD
  * the current device; d_out may alias d_image; `stream` is a hipStream_t
  * (NULL = the null stream).  d_workspace may be NULL (a per-device pooled
  * buffer is used; calls on one device are then serialised) or must hold
- * fcamd_workspace_bytes() bytes.  Asynchronous with respect to the host. */
+ * fcamd_workspace_bytes() bytes.  For extents without compile-time kernels
+ * that size is often the one of a faster transform at longer extents; a
+ * workspace that only holds the transform at the image's own extents is taken
+ * as well, and runs that.  Asynchronous with respect to the host. */
 FCAMD_API long long fcamd_workspace_bytes(const int* imDim, const int* kernelDim);
 FCAMD_API int fcamd_convolve3d_device(float* d_out, const float* d_image, const int* imDim,
                                       const float* d_kernel, const int* kernelDim, int op,
@@ -65,7 +68,8 @@ FCAMD_API int fcamd_convolve3d_device(float* d_out, const float* d_image, const 
  * into a graph, also for lengths the process has not used before.  Every
  * call on one device shares that array: calls that overlap on one device
  * (other threads, other streams) race; order them.  Same results as
- * fcamd_convolve3d_device; d_out may alias d_image. */
+ * fcamd_convolve3d_device, to rounding where that runs extents without
+ * compile-time kernels at longer ones; d_out may alias d_image. */
 #define FCAMD_NOALLOC_MAX_WORKSPACE (128LL << 20)
 FCAMD_API int fcamd_convolve3d_device_noalloc(float* d_out, const float* d_image,
                                               const int* imDim, const float* d_kernel,
